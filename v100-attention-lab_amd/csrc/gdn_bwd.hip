@@ -26,12 +26,12 @@
 // Only S (forward) and dS (backward) carry from chunk to chunk, and each
 // needs a few products per chunk; everything else is independent per chunk.
 // So the backward is three launches, on the fp32 matrix cores
-// (v_mfma_f32_16x16x4_f32) except the 16-bit recurrences:
+// (v_mfma_f32_16x16x4_f32) or, for 16-bit q, k, v and dO, on the fp16 ones
+// with fp32 values as hi + lo pairs:
 //   1. prep_kernel, one workgroup per (chunk, head): gates, K K^T, P, T and
-//      (fp32 only) W, written once to a per-chunk record (the
-//      state-independent half of the chunk's forward, shared by every
-//      V-slice below), and for 16-bit inputs T diag(beta) and P as fp16
-//      pairs as well;
+//      W, written once to a per-chunk record (the state-independent half of
+//      the chunk's forward, shared by every V-slice below), or prep16_kernel:
+//      the gates, T and P, the last two as fp16 pairs;
 //   2. recur_kernel (fp32) or recur16_kernel (16-bit q, k, v, dO: fp16 MFMA
 //      on hi + lo pairs), one workgroup per (sequence, head, 16-column V
 //      slice) and direction, both directions in one launch: the forward
@@ -39,88 +39,25 @@
 //      stores each chunk's dS' and du and finally dh0.  The 16-bit walks
 //      store S and dS' in fp16 (half the bytes of the largest arrays of
 //      the backward), in their range-shifted units with one scale per
-//      walk;
+//      walk, and T^T du in place of du;
 //   3. grad_kernel, one workgroup per (chunk, head) over all of V: every
 //      gradient of the chunk from the stored S, dS', u, du and the record,
 //      written directly in the output dtypes (V is walked in 32-column steps,
 //      16 when V is an odd multiple of 16, with the C x K products held in
-//      MFMA accumulators).
+//      MFMA accumulators), or after the 16-bit walks grad16_kernel
+//      (gdn_bwd_grad16.h).
 // Packed sequences (cu_seqlens): sequence i owns chunk slots floor(t0 / C) +
 // i onwards, one per chunk; the ranges are disjoint, so every launch handles
 // packed sequences like a batch.
 
-#include "gdn_fwd_pipe.h"
-#include "gdn_tiles_f16.h"
+#include "gdn_bwd_args.h"
+#include "gdn_bwd_grad16.h"
 
 namespace gdn {
 namespace bwd {
 
-using namespace tiles;
-
-constexpr int C = 32;
-constexpr int BV = 16;    // state columns per workgroup of the recurrences
 constexpr int NTP = 256;  // threads: prep_kernel and recur_kernel (4 waves)
 constexpr int NTG = 512;  // threads: grad_kernel (8 waves)
-
-struct BArgs {
-  const void* q;
-  const void* k;
-  const void* v;
-  const void* g;
-  const void* beta;
-  const float* h0;
-  const void* d_o;
-  const float* dfs;
-  void* dq;
-  void* dk;
-  void* dv;
-  void* dg;
-  void* dbeta;
-  float* dh0;
-  float* rec;  // per (slot, head): the prep kernel's record
-  // per (slot, head): S at the chunk start and dS', the gradient of the
-  // state after the chunk: fp32 [K][V], or from the 16-bit walks fp16 [V][K]
-  // (rows = state columns, in each walk's range-shifted units: scl below
-  // scales them back)
-  float* ckS;
-  float* ckD;
-  float* uu;   // per (slot, head): u, [C][V]
-  float* du;   // per (slot, head): du, [C][V]
-  f16* r16;    // per (slot, head): T diag(beta) and P as fp16 pairs (16-bit walks)
-  float* scl;  // per walk unit (sequence, head, V-slice): the power of two that
-               // takes the fp16 ckS (units first) and ckD (then) back to true units
-  int w16;     // the recurrences run on fp16 pairs (16-bit q, k, v and dO)
-  int64_t sq[3], sk[3], sv[3], sg[3], sb[3], sdo[3], sdq[3], sdk[3], sdv[3], sdg[3], sdb[3];
-  int64_t sh0[4], sdfs[4], sdh0[4];
-  int B, T, H, V, nv, nchmax, units;
-  float scale;
-  int g_dtype, beta_dtype, do_dtype;
-  const int64_t* cu;
-  int xcd_remap;
-};
-
-// Per-(slot, head) record, in floats: T, P = M o Q K^T and K K^T as [C][C],
-// W as [C][K], then b, gam, D as [C] each and gam_C (first of a [C] row).
-template <int K>
-struct Rec {
-  static constexpr int T = 0, PM = C * C, KK = 2 * C * C, W = 3 * C * C;
-  static constexpr int G = W + C * K;
-  static constexpr int SIZE = G + 4 * C;
-};
-inline int64_t rec_size(int K) { return 3 * C * C + (int64_t)C * K + 4 * C; }
-// The 16-bit walks' per-(slot, head) record, in floats: T as [C][C], then
-// the gates as in Rec (their products take P, K K^T and W from elsewhere).
-struct RecT {
-  static constexpr int T = 0, G = C * C;
-  static constexpr int SIZE = G + 4 * C;
-};
-// The same chunk's operands of the 16-bit recurrences, in halves: T diag(beta)
-// and P as [C][C], each an fp16 pair hi + lo.
-struct Rec16 {
-  static constexpr int TBH = 0, TBL = C * C, PH = 2 * C * C, PL = 3 * C * C;
-  static constexpr int SIZE = 4 * C * C;
-};
-inline int64_t rec16_size(int) { return 4 * C * C; }
 
 // ---------------------------------------------------------------------------
 // 1. prep: the state-independent half of a chunk's forward
@@ -146,7 +83,6 @@ __global__ __launch_bounds__(NTP) void prep_kernel(const BArgs p) {
   if (!slot_chunk<C>(p, slot, rs, c)) return;
   const int t0 = c * C, nval = min(C, rs.T - t0);
   float* const rec = p.rec + (slot * p.H + hi) * (int64_t)R::SIZE;
-  f16* const rh = p.r16 + (slot * p.H + hi) * (int64_t)Rec16::SIZE;
 
   {
     RowLoad<TIn, C, K, NTP> lq, lk;
@@ -212,7 +148,6 @@ __global__ __launch_bounds__(NTP) void prep_kernel(const BArgs p) {
     s.a[t][j] = j < t ? s.bt[t] * mv * s.kk[t][j] : 0.f;
     rec[R::PM + e] = mv * s.qk[t][j];
     rec[R::KK + e] = s.kk[t][j];
-    if (p.w16) tiles16::split_f16(mv * s.qk[t][j], rh[Rec16::PH + e], rh[Rec16::PL + e]);
   }
   if (tid < C) {
     rec[R::G + tid] = s.b[tid];
@@ -239,22 +174,10 @@ __global__ __launch_bounds__(NTP) void prep_kernel(const BArgs p) {
     }
   }
   __syncthreads();
-  // the 16-bit recurrences' operand T diag(beta) as fp16 pairs, 4 entries
-  // per lane
-  if (p.w16) {
-    static_assert(C * C == 4 * NTP, "4 entries of T per lane");
-    const int t = tid / (C / 4), j0 = 4 * (tid % (C / 4));
-    f16 h[4], l[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) tiles16::split_f16(s.t[t][j0 + i] * s.bt[j0 + i], h[i], l[i]);
-    *reinterpret_cast<f16x4*>(rh + Rec16::TBH + t * C + j0) = f16x4{h[0], h[1], h[2], h[3]};
-    *reinterpret_cast<f16x4*>(rh + Rec16::TBL + t * C + j0) = f16x4{l[0], l[1], l[2], l[3]};
-  }
-  // W = T diag(beta gam) K, read by the fp32 recurrences only
-  if (!p.w16)
-    mmx<NTP, C, K>(tid, [&](int m, int n, float x) { rec[R::W + m * K + n] = x; },
-                   seg<C>([&](int m, int kk) { return s.t[m][kk]; },
-                          [&](int kk, int n) { return s.bt[kk] * s.gam[kk] * s.k[kk][n]; }));
+  // W = T diag(beta gam) K
+  mmx<NTP, C, K>(tid, [&](int m, int n, float x) { rec[R::W + m * K + n] = x; },
+                 seg<C>([&](int m, int kk) { return s.t[m][kk]; },
+                        [&](int kk, int n) { return s.bt[kk] * s.gam[kk] * s.k[kk][n]; }));
 }
 
 // 16-bit q or k rows as MFMA operands: 8 elements (16 bytes) per lane, in
@@ -269,32 +192,15 @@ __device__ __forceinline__ f32x4 mma16(const u32x4& a, const u32x4& b, const f32
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), acc,
                                                    0, 0, 0);
 }
-// 8 consecutive fp32 values that hold 16-bit inputs, back in their own type
-// (exact).
-template <typename TIn>
-__device__ __forceinline__ u32x4 pack16(const float* x) {
-  u32x4 r;
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    if constexpr (std::is_same<TIn, f16>::value) {
-      const f16 lo = (f16)x[2 * e], hi = (f16)x[2 * e + 1];
-      r[e] = (uint32_t)__builtin_bit_cast(uint16_t, lo) | ((uint32_t)__builtin_bit_cast(uint16_t, hi) << 16);
-    } else {
-      r[e] = (__float_as_uint(x[2 * e]) >> 16) | (__float_as_uint(x[2 * e + 1]) & 0xffff0000u);
-    }
-  }
-  return r;
-}
-
 // The prep of the 16-bit recurrences: one wave per two (chunk, head)
 // records, with no workgroup barrier.  Per record: the gates (a prefix sum
 // across lanes), K K^T and Q K^T on the 16-bit matrix cores (exact
 // products, fp32 sums), A = beta_t e^{b_t - b_j} K K^T (t > j) staged as
 // A^T in the wave's LDS, then T = (I + A)^-1 by substitution with one lane
-// per row of T (lanes 0-31: record 0, lanes 32-63: record 1).  It writes T
-// and the gates to the fp32 record, and T diag(beta) and P = M o Q K^T as
-// fp16 pairs; the gradient kernel forms P and K K^T in fp32 itself (from
-// the q and k rows it loads anyway), so they are not written here.  Rows
+// per row of T (lanes 0-31: record 0, lanes 32-63: record 1).  It writes the
+// gates to the fp32 record, and T and P = M o Q K^T as fp16 pairs; the
+// gradient kernel forms Q K^T and K K^T in fp32 itself (from the q and k rows
+// it loads anyway), so they are not written here.  Rows
 // past a chunk's end read the last row again: their beta and gate are
 // zero, which zeroes their rows of A and T (and their rows of P are
 // zeroed), so the record equals that of zero rows.
@@ -372,7 +278,7 @@ __global__ __launch_bounds__(256) void prep16_kernel(const BArgs p, int64_t nrec
     rec_h[R::G + c] = b;
     rec_h[R::G + C + c] = expf(b);
     rec_h[R::G + 2 * C + c] = expf(bC - b);
-    rec_h[R::G + 3 * C + c] = c == 0 ? expf(bC) : 0.f;
+    rec_h[R::G + 3 * C + c] = bv;
   }
   __builtin_amdgcn_wave_barrier();
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -447,28 +353,20 @@ __global__ __launch_bounds__(256) void prep16_kernel(const BArgs p, int64_t nrec
   pipe::solve_rows1<3, 6>(at, c, xc);
   pipe::solve_rows1<0, 3>(at, c, xc);
   if ((half ? nval[1] : nval[0]) > 0) {
-    float* const tr = rec_h + R::T + c * C;
-#pragma unroll
-    for (int i = 0; i < C; i += 4) *reinterpret_cast<f32x4*>(tr + i) = f32x4{xc[i], xc[i + 1], xc[i + 2], xc[i + 3]};
-    // row c of T diag(beta) as fp16 pairs
+    // row c of T as fp16 pairs
     f16* const rh = p.r16 + (half ? ri[1] : ri[0]) * (int64_t)Rec16::SIZE + c * C;
-    const float* const be = s_beta[wave][half];
 #pragma unroll
     for (int j = 0; j < C; j += 8) {
-      const f32x4 b0 = *reinterpret_cast<const f32x4*>(be + j), b1 = *reinterpret_cast<const f32x4*>(be + j + 4);
       f16x8 h, l;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
+      for (int i = 0; i < 8; ++i) {
         f16 hh, ll;
-        tiles16::split_f16(xc[j + i] * b0[i], hh, ll);
+        tiles16::split_f16(xc[j + i], hh, ll);
         h[i] = hh;
         l[i] = ll;
-        tiles16::split_f16(xc[j + 4 + i] * b1[i], hh, ll);
-        h[4 + i] = hh;
-        l[4 + i] = ll;
       }
-      *reinterpret_cast<f16x8*>(rh + Rec16::TBH + j) = h;
-      *reinterpret_cast<f16x8*>(rh + Rec16::TBL + j) = l;
+      *reinterpret_cast<f16x8*>(rh + Rec16::TH + j) = h;
+      *reinterpret_cast<f16x8*>(rh + Rec16::TL + j) = l;
     }
   }
 }
@@ -805,14 +703,6 @@ __global__ __launch_bounds__(NTP) void recur_kernel(const BArgs p) {
 
 namespace w16 {
 
-using tiles16::HP;
-using tiles16::frag8;
-using tiles16::frag4_t;
-using tiles16::store_pair4;
-
-typedef short s16x4 __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
-
 // A chunk's inputs reach LDS by LDS-DMA: global_load_lds_dwordx4 (_dword)
 // copies 16 (4) bytes a lane from global memory to LDS at M0 + 16 (4) lane,
 // complete once the issuing wave's vmcnt has drained.  The walks' barriers
@@ -822,62 +712,6 @@ typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
 // compiler then sees no LDS write in flight and adds no vmcnt wait before
 // the transposing LDS reads (which it cannot tell apart from the copies'
 // targets).  M0 is written here and nowhere else in these kernels.
-// LDS address of a generic pointer into LDS: its low 32 bits (the LDS
-// aperture sits in the high half)
-__device__ __forceinline__ uint32_t lds_addr(const void* p) {
-  return __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)p);
-}
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
-__device__ __forceinline__ void dma16(const void* src, void* lds_base) {
-  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(lds_addr(lds_base))
-               : "memory", "m0");
-}
-__device__ __forceinline__ void dma4(const void* src, void* lds_base) {
-  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dword %0, off" ::"v"(src), "s"(lds_addr(lds_base))
-               : "memory", "m0");
-}
-#pragma clang diagnostic pop
-__device__ __forceinline__ void bar() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-__device__ __forceinline__ void wait_dma() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
-
-__device__ __forceinline__ f16x4 read_tr4(const f16* a) {
-  return __builtin_bit_cast(f16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)a));
-}
-
-// Rows of W halves (W = 32, 64, 128) unpadded in LDS, each row's 16-byte
-// pieces permuted: piece s of row t sits at s ^ swz<W>(t).  The 16 rows that
-// a row read (frag8, 16-lane passes) takes at one piece, and the 8 rows x 2
-// pieces of a pass of a transposing read (frag8_ts, 32-lane passes), then
-// use every bank once.
-template <int W>
-__device__ __forceinline__ int swz(int t) {
-  if constexpr (W == 128) return (((t >> 3) & 1) << 3) | ((t & 3) << 1) | ((t >> 2) & 1);
-  else if constexpr (W == 64) return (((t >> 3) & 1) << 2) | (((t >> 1) & 1) << 1) | ((t >> 2) & 1);
-  else {
-    static_assert(W == 32, "rows of 32, 64 or 128 halves");
-    return (((t >> 3) & 1) << 1) | ((t >> 2) & 1);
-  }
-}
-// offset in halves of element (t, col)
-template <int W>
-__device__ __forceinline__ int soff(int t, int col) {
-  return t * W + ((((col >> 3) ^ swz<W>(t))) << 3) + (col & 7);
-}
-// halves col .. col + 7 of row t
-template <int W>
-__device__ __forceinline__ f16x8 frag8_s(const f16* x, int t, int col) {
-  return frag8(x + soff<W>(t, col));
-}
-// Row m0 + r of X^T, contraction indices t0 + 8 kq .. + 7, by two
-// ds_read_b64_tr_b16 (lane layout as tiles16::frag8_t)
-template <int W>
-__device__ __forceinline__ f16x8 frag8_ts(const f16* x, int t0, int m0, int r, int kq) {
-  const int t = t0 + 8 * kq + (r >> 2), col = m0 + 4 * (r & 3);
-  const f16x4 lo = read_tr4(x + soff<W>(t, col)), hi = read_tr4(x + soff<W>(t + 4, col));
-  return f16x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-}
-
 // dO rows of a slice (BV halves) in LDS: row t at row dperm(t), bits 2 and
 // 3 of t swapped, so that the rows of a 32-lane pass of a transposing read
 // (t = 0..3 and 8..11, + 4 h) fill 256 contiguous bytes.
@@ -978,9 +812,9 @@ __device__ __forceinline__ void fix_v(f16* dst, int nval, float sc, int lane) {
 template <int K>
 struct alignas(16) FIn {
   f16 k[C * K];               // K rows, swz<K>
-  f16 th[C * C], tl[C * C];   // T diag(beta) as fp16 pairs, swz<C>
+  f16 th[C * C], tl[C * C];   // T as fp16 pairs, swz<C>
   f16 v[C * BV];              // V rows of the slice
-  float gv[4][C];             // b, gam, D, {gam_C, 0 ..}
+  float gv[4][C];             // b, gam, D, beta
 };
 
 // The forward walk's inputs are triple-buffered (chunk c in in[c % 3]): a
@@ -988,7 +822,7 @@ struct alignas(16) FIn {
 template <int K>
 struct alignas(16) FMem {
   f16 sh[BV][K + HP], sl[BV][K + HP];  // S^T
-  f16 yh[BV][C + HP], yl[BV][C + HP];  // (V - diag(gam) K S)^T
+  f16 yh[BV][C + HP], yl[BV][C + HP];  // (diag(beta) (V - diag(gam) K S))^T
   f16 dh[BV][C + HP], dl[BV][C + HP];  // (diag(D) u)^T
   float uf[C][BV];                     // u rows, on their way to uu
   FIn<K> in[3];
@@ -998,7 +832,7 @@ struct alignas(16) FMem {
 template <int K>
 struct alignas(16) RIn {
   f16 q[C * K], k[C * K];     // Q, K rows, swz<K>
-  f16 th[C * C], tl[C * C];   // T diag(beta), swz<C>
+  f16 th[C * C], tl[C * C];   // T, swz<C>
   f16 ph[C * C], pl[C * C];   // P, swz<C>
   f16 dot[C * BV];            // dO rows of the slice, row t at dperm(t)
   float gv[4][C];
@@ -1009,8 +843,8 @@ struct alignas(16) RMem {
   f16 sh[BV][K + HP], sl[BV][K + HP];  // dS'^T
   f16 gh[BV][C + HP], gl[BV][C + HP];  // (diag(gam) dO)^T
   f16 uh[BV][C + HP], ul[BV][C + HP];  // du^T
-  f16 zh[BV][C + HP], zl[BV][C + HP];  // (diag(gam) (T diag(beta))^T du)^T
-  float duf[C][BV];                    // du rows, on their way to du
+  f16 zh[BV][C + HP], zl[BV][C + HP];  // (diag(beta gam) T^T du)^T
+  float duf[C][BV];                    // T^T du rows, on their way to du
   RIn<K> in[2];
 };
 
@@ -1096,8 +930,8 @@ __device__ __forceinline__ void walk_forward16(const BArgs& p, FMem<K>& s, const
     const int nval = min(C, rs.T - cn * C);
     const uint16_t* const rh = reinterpret_cast<const uint16_t*>(p.r16 + ri * (int64_t)Rec16::SIZE);
     dma_rows<K, 1>(reinterpret_cast<const uint16_t*>(kg) + (int64_t)cn * C * p.sk[1], p.sk[1], nval, d.k, 0, lane);
-    dma_rows<C, 1>(rh + Rec16::TBH, C, C, d.th, 0, lane);
-    dma_rows<C, 1>(rh + Rec16::TBL, C, C, d.tl, 0, lane);
+    dma_rows<C, 1>(rh + Rec16::TH, C, C, d.th, 0, lane);
+    dma_rows<C, 1>(rh + Rec16::TL, C, C, d.tl, 0, lane);
     dma_v(reinterpret_cast<const uint16_t*>(vg) + (int64_t)cn * C * p.sv[1], p.sv[1], nval, d.v, lane);
     if (lane < C) dma16(p.rec + ri * (int64_t)RecT::SIZE + RecT::G + 4 * lane, &d.gv[0][0]);
   };
@@ -1124,7 +958,8 @@ __device__ __forceinline__ void walk_forward16(const BArgs& p, FMem<K>& s, const
     const int b1 = b == 2 ? 0 : b + 1, b2 = b1 == 2 ? 0 : b1 + 1;
     const bool issuer = loader && lw == (c & 1);
     if (!loader) {
-      // Y = V - diag(gam) K S for rows 16 w .. (k exact in fp16), as Y^T pairs
+      // Y = diag(beta) (V - diag(gam) K S), rows 16 w .. (k exact in fp16), as
+      // Y^T pairs
       const int um0 = 16 * wave;
       f32x4 ak = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -1135,15 +970,16 @@ __device__ __forceinline__ void walk_forward16(const BArgs& p, FMem<K>& s, const
       }
       const int t = um0 + 4 * kq;
       const f16x4 vv = frag4_t(reinterpret_cast<const f16 (*)[BV]>(in.v), um0, 0, r, kq);
-      const float y[4] = {(float)vv[0] - in.gv[1][t] * ak[0], (float)vv[1] - in.gv[1][t + 1] * ak[1],
-                          (float)vv[2] - in.gv[1][t + 2] * ak[2], (float)vv[3] - in.gv[1][t + 3] * ak[3]};
+      float y[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) y[i] = in.gv[3][t + i] * ((float)vv[i] - in.gv[1][t + i] * ak[i]);
       store_pair4(&s.yh[r][t], &s.yl[r][t], y);
     } else if (issuer && c + 2 < nch) {
       fetch(c + 2, b2);
     }
     bar();
     if (!loader) {
-      // u = T diag(beta) Y, rows 16 w .. (W S = T diag(beta) diag(gam) K S)
+      // u = T Y, rows 16 w ..
       const int um0 = 16 * wave;
       f32x4 au = {0.f, 0.f, 0.f, 0.f};
       const f16x8 th = frag8_s<C>(in.th, um0 + r, 8 * kq), yh = frag8(&s.yh[r][8 * kq]);
@@ -1172,7 +1008,7 @@ __device__ __forceinline__ void walk_forward16(const BArgs& p, FMem<K>& s, const
         a = __builtin_amdgcn_mfma_f32_16x16x32_f16(kt, frag8(&s.dh[r][8 * kq]), a, 0, 0, 0);
         a = __builtin_amdgcn_mfma_f32_16x16x32_f16(kt, frag8(&s.dl[r][8 * kq]), a, 0, 0, 0);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) S.st[j][i] = in.gv[3][0] * S.st[j][i] + a[i];
+        for (int i = 0; i < 4; ++i) S.st[j][i] = in.gv[1][C - 1] * S.st[j][i] + a[i];
       }
     }
     S.put(s.sh, s.sl, wave, r, kq);
@@ -1193,9 +1029,10 @@ __device__ __forceinline__ void walk_forward16(const BArgs& p, FMem<K>& s, const
   wait_dma();
 }
 
-// Backward walk: dS' of each chunk -> ckD (fp16), du -> du, at the end dh0.
+// Backward walk: dS' of each chunk -> ckD (fp16), T^T du -> du, at the end
+// dh0.
 // For bf16 inputs the walk runs on dO and d_final_state shifted into fp16's
-// range (every output of the walk is linear in them) and shifts du and dh0
+// range (every output of the walk is linear in them) and shifts T^T du and dh0
 // back: small gradients keep their hi / lo precision.  ckD stays in the
 // shifted units; the factor that takes it back goes to scl[units + unit].
 // Waves 2 and 3 (the loaders) copy the previous chunk's inputs but its q
@@ -1232,8 +1069,8 @@ __device__ __forceinline__ void walk_backward16(const BArgs& p, RMem<K>& s, cons
     const int64_t ri = (slot0 + cn) * p.H + hi;
     const uint16_t* const rh = reinterpret_cast<const uint16_t*>(p.r16 + ri * (int64_t)Rec16::SIZE);
     dma_rows<K, 2>(reinterpret_cast<const uint16_t*>(kg) + (int64_t)cn * C * p.sk[1], p.sk[1], nval, d.k, lw, lane);
-    dma_rows<C, 2>(rh + Rec16::TBH, C, C, d.th, lw, lane);
-    dma_rows<C, 2>(rh + Rec16::TBL, C, C, d.tl, lw, lane);
+    dma_rows<C, 2>(rh + Rec16::TH, C, C, d.th, lw, lane);
+    dma_rows<C, 2>(rh + Rec16::TL, C, C, d.tl, lw, lane);
     dma_rows<C, 2>(rh + Rec16::PH, C, C, d.ph, lw, lane);
     dma_rows<C, 2>(rh + Rec16::PL, C, C, d.pl, lw, lane);
     dma_dot(reinterpret_cast<const uint16_t*>(dg) + (int64_t)cn * C * p.sdo[1], p.sdo[1], nval, d.dot, lw, lane);
@@ -1252,6 +1089,13 @@ __device__ __forceinline__ void walk_backward16(const BArgs& p, RMem<K>& s, cons
         fix_dot<TIn>(d.dot, nval, rsd.v, lw, lane);
       }
     }
+  };
+  // a loader: chunk cn's rows of T^T du (still in duf) -> du, 16 bytes a lane
+  auto store_duf = [&](int cn) __attribute__((always_inline)) {
+    static_assert(C * BV == 4 * 128, "four entries per loader lane");
+    const int row = ll / (BV / 4), c4 = 4 * (ll % (BV / 4));
+    *reinterpret_cast<f32x4*>(p.du + (((slot0 + cn) * p.H + hi) * C + row) * (int64_t)p.V + v0 + c4) =
+        *reinterpret_cast<const f32x4*>(&s.duf[row][c4]);
   };
   State<K> S;
   S.load(p.dfs, p.sdfs, bi, hi, v0, wave, r, kq, rsd.v);
@@ -1282,7 +1126,6 @@ __device__ __forceinline__ void walk_backward16(const BArgs& p, RMem<K>& s, cons
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         du[i] = scale * a1[i] + in.gv[2][t + i] * a2[i];
-        s.duf[t + i][r] = du[i] * rsd.fs;
       }
       store_pair4(&s.uh[r][t], &s.ul[r][t], du);
       if (c >= 1) fetch(c - 1);
@@ -1297,11 +1140,14 @@ __device__ __forceinline__ void walk_backward16(const BArgs& p, RMem<K>& s, cons
                           in.gv[1][t4 + 2] * (float)dv[2], in.gv[1][t4 + 3] * (float)dv[3]};
       store_pair4(&s.gh[r][t4], &s.gl[r][t4], x);
       copy_state_rows<K, 128>(s.sh, reinterpret_cast<f16*>(p.ckD) + (ri * p.V + v0) * (int64_t)K, ll);
+      // chunk c + 1's rows of T^T du: a chunk late, so that the drain at its
+      // end did not wait for their stores
+      if (c + 1 < nch) store_duf(c + 1);
     }
     bar();
-    // W^T du = K^T diag(beta gam) T^T du = K^T (diag(gam) (T diag(beta))^T du):
-    // z on waves 0-1 (rows 16 w .. of z, T diag(beta) transposed by the
-    // reads) while waves 2-3 form their Q^T diag(gam) dO term
+    // W^T du = K^T diag(beta gam) T^T du = K^T z: T^T du and z on waves 0-1
+    // (rows 16 w .., T transposed by the reads) while waves 2-3 form their
+    // Q^T diag(gam) dO term
     f32x4 aq[State<K>::NST];
     auto q_term = [&]() __attribute__((always_inline)) {
 #pragma unroll
@@ -1324,16 +1170,15 @@ __device__ __forceinline__ void walk_backward16(const BArgs& p, RMem<K>& s, cons
       az = __builtin_amdgcn_mfma_f32_16x16x32_f16(tth, frag8(&s.ul[r][8 * kq]), az, 0, 0, 0);
       az = __builtin_amdgcn_mfma_f32_16x16x32_f16(ttl, uh, az, 0, 0, 0);
       const int t = um0 + 4 * kq;
-      const float z[4] = {in.gv[1][t] * az[0], in.gv[1][t + 1] * az[1], in.gv[1][t + 2] * az[2],
-                          in.gv[1][t + 3] * az[3]};
+      float z[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        z[i] = in.gv[1][t + i] * in.gv[3][t + i] * az[i];
+        s.duf[t + i][r] = az[i] * rsd.fs;
+      }
       store_pair4(&s.zh[r][t], &s.zl[r][t], z);
     } else {
       q_term();
-      // du rows -> du: 16 bytes a loader lane
-      static_assert(C * BV == 4 * 128, "four du entries per loader lane");
-      const int row = ll / (BV / 4), c4 = 4 * (ll % (BV / 4));
-      *reinterpret_cast<f32x4*>(p.du + (ri * C + row) * (int64_t)p.V + v0 + c4) =
-          *reinterpret_cast<const f32x4*>(&s.duf[row][c4]);
     }
     bar();
     if (!loader) q_term();
@@ -1347,13 +1192,14 @@ __device__ __forceinline__ void walk_backward16(const BArgs& p, RMem<K>& s, cons
         b = __builtin_amdgcn_mfma_f32_16x16x32_f16(kt, frag8(&s.zh[r][8 * kq]), b, 0, 0, 0);
         b = __builtin_amdgcn_mfma_f32_16x16x32_f16(kt, frag8(&s.zl[r][8 * kq]), b, 0, 0, 0);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) S.st[j][i] = scale * aq[j][i] + in.gv[3][0] * S.st[j][i] - b[i];
+        for (int i = 0; i < 4; ++i) S.st[j][i] = scale * aq[j][i] + in.gv[1][C - 1] * S.st[j][i] - b[i];
       }
     }
     S.put(s.sh, s.sl, wave, r, kq);
     if (c >= 1) settle(c - 1);
     bar();
   }
+  if (loader && nch > 0) store_duf(0);
   wait_dma();
   if (p.dh0 != nullptr) {
 #pragma unroll
@@ -1409,64 +1255,28 @@ struct alignas(16) GSmem {
   float yp[C][CD];   // dQK o Q K^T = scale (dO u^T) o P
   float dt[C][CD];   // dT, then dA
   float z[C][CD];    // T^T dT, then dKK
-  // The V step's tiles: fp32 (w), or for fp16 inputs with fp16 states
-  // MFMA operand rows in fp16 (h: v, dO and the states exact, u and du as
-  // hi + lo pairs; HD = VS + 16 halves, 16-byte aligned rows).
-  static constexpr int HD = VS + 16;
-  union {
-    struct {
-      float v[C][SD], dO[C][SD], u[C][SD], du[C][SD];
-      union {
-        struct {
-          float S[K][SD], dS[K][SD];  // fp32 states
-        } f;
-        struct {
-          // fp16 states of the 16-bit walks, as stored; K + 16 halves (8
-          // words past a multiple of 64) puts the 8-byte transposed reads
-          // of 32 lanes (rows 4 kq + r / 4, columns 4 (r % 4)) in 64
-          // different banks
-          f16 ST[VS][K + 16], dST[VS][K + 16];
-        } h;
-      } st;
-    } w;
-    struct {
-      f16 v[C][HD], dO[C][HD], uh[C][HD], ul[C][HD], dh[C][HD], dl[C][HD];
-      f16 ST[VS][K + 8], dST[VS][K + 8];  // S^T, dS'^T rows (as stored)
-    } h;
-    // after the walk (fp16 inputs): operands of the dq / dk products, q and
-    // k exact in fp16, dQK and dKK + dKK^T as hi + lo pairs, all row-major
-    // (transposed operands are read with ds_read_b64_tr_b16)
-    struct {
-      f16 q[C][K + 8], k[C][K + 8];
-      f16 dwh[C][K + 8], dwl[C][K + 8];  // dW
-      f16 yh[C][C + 8], yl[C][C + 8];    // dQK
-      f16 zh[C][C + 8], zl[C][C + 8];    // Z = T^T dT, later dKK + dKK^T
-      f16 th[C][C + 8], tl[C][C + 8];    // T
-      f16 dth[C][C + 8], dtl[C][C + 8];  // dT
-    } x;
-  };
+  // the V step's tiles
+  struct {
+    float v[C][SD], dO[C][SD], u[C][SD], du[C][SD];
+    float S[K][SD], dS[K][SD];
+  } w;
   float b[C], gam[C], D[C], bt[C];
   float rq[K / 16][C], rk[K / 16][C], rw[K / 16][C];  // row partials, one row per 16-column tile
   float vu[VS / 16][C];  // v.dU~ row partials, one row per 16-column tile
   float kw[C], dgam[C], dD[C], db[C], dbt[C];
-  float scs[VS], scd[VS];  // the V step's state scales per state column (16-bit walks)
   float red[NTG / 64];
   float gC, dgC;
 };
 
 // VS: V columns per step of the V walk (32, or 16 when V is an odd
-// multiple of 16).  ST16: ckS and ckD hold fp16 in the walks' shifted units
-// (the 16-bit walks), scaled back per 16-column slice by scl when staged.
+// multiple of 16).
 // NVS: the number of V steps when fixed at compile time (V = 128 or 64;
 // 0: V / VS at run time), so that the walk unrolls into straight-line code
 // whose waits cover exactly the step being staged.
-template <typename TIn, int K, int VS, bool ST16, int NVS>
+template <typename TIn, int K, int VS, int NVS>
 __global__ __launch_bounds__(NTG) void grad_kernel(const BArgs p) {
-  using R = typename std::conditional<ST16, RecT, Rec<K>>::type;
+  using R = Rec<K>;
   constexpr int RL = NTG / C;
-  // fp16 inputs with fp16 states (no range shift): the V walk's products on
-  // v_mfma_f32_16x16x32_f16, one 32-column step per product
-  constexpr bool F16W = ST16 && std::is_same<TIn, f16>::value && VS == 32;
   __shared__ GSmem<K, VS> s;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1474,18 +1284,14 @@ __global__ __launch_bounds__(NTG) void grad_kernel(const BArgs p) {
   const int64_t slot = blockIdx.x / p.H;
   const int hi = blockIdx.x % p.H;
   RowSpan rs;
-  int c, seq;
-  if (!slot_chunk<C>(p, slot, rs, c, seq)) return;
+  int c;
+  if (!slot_chunk<C>(p, slot, rs, c)) return;
   const int t0 = c * C, nval = min(C, rs.T - t0);
   const float scale = p.scale;
   const int64_t ri = slot * p.H + hi;
   const float* const rec = p.rec + ri * R::SIZE;
-  using TS = typename std::conditional<ST16, f16, float>::type;
-  const TS* const cks = reinterpret_cast<const TS*>(p.ckS) + ri * (int64_t)K * p.V;
-  const TS* const ckd = reinterpret_cast<const TS*>(p.ckD) + ri * (int64_t)K * p.V;
-  // the state scales of this head's 16-column walk slices
-  const float* const sclS = ST16 ? p.scl + ((int64_t)seq * p.H + hi) * p.nv : nullptr;
-  const float* const sclD = ST16 ? sclS + p.units : nullptr;
+  const float* const cks = p.ckS + ri * (int64_t)K * p.V;
+  const float* const ckd = p.ckD + ri * (int64_t)K * p.V;
   const float* const uu = p.uu + ri * (int64_t)C * p.V;
   const float* const dug = p.du + ri * (int64_t)C * p.V;
   const int64_t qb = head_base(rs, hi, p.sq) + (int64_t)t0 * p.sq[1];
@@ -1503,10 +1309,8 @@ __global__ __launch_bounds__(NTG) void grad_kernel(const BArgs p) {
   lq.load(tid, static_cast<const TIn*>(p.q) + qb, p.sq[1], nval);
   lk.load(tid, static_cast<const TIn*>(p.k) + kb, p.sk[1], nval);
   lt.load(tid, rec + R::T, C, C);
-  if constexpr (!ST16) {
-    lp.load(tid, rec + R::PM, C, C);
-    lkk.load(tid, rec + R::KK, C, C);
-  }
+  lp.load(tid, rec + R::PM, C, C);
+  lkk.load(tid, rec + R::KK, C, C);
   const float gate = tid < 4 * C ? rec[R::G + tid] : 0.f;
   const uint32_t bvb =
       tid < nval ? load_bits(p.beta, head_base(rs, hi, p.sb) + (int64_t)(t0 + tid) * p.sb[1], p.beta_dtype) : 0u;
@@ -1548,17 +1352,11 @@ __global__ __launch_bounds__(NTG) void grad_kernel(const BArgs p) {
   // products to arrive).
   // Every load of a step is unconditional (rows past the chunk's end read
   // its last row again and are zeroed when stored), so that staging one
-  // step waits only for that step's loads.  With the 16-bit walks dO has
-  // q's dtype and 4-byte aligned rows: one element pair per thread.
-  constexpr int NDP = C * VS / 2;  // dO element pairs of a step (VS = 16: waves 0-3 only)
-  static_assert(!ST16 || NDP == NTG || NDP == NTG / 2, "at most one dO pair per thread");
-  // states: fp32 [K][V] rows, or fp16 [V][K] rows from the 16-bit walks
-  using SLoad = typename std::conditional<ST16, RowLoad<f16, VS, K, NTG>, RowLoad<float, K, VS, NTG>>::type;
+  // step waits only for that step's loads.
   struct StepRows {
     RowLoad<TIn, C, VS, NTG> lv;
     RowLoad<float, C, VS, NTG> lu, ldu;
-    SLoad lS, ldS;
-    float scS[2], scD[2];
+    RowLoad<float, K, VS, NTG> lS, ldS;
     uint32_t rdo[NDO];
   };
   auto load_step = [&](StepRows& x, int vsi) __attribute__((always_inline)) {
@@ -1566,77 +1364,24 @@ __global__ __launch_bounds__(NTG) void grad_kernel(const BArgs p) {
     x.lv.load_clamped(tid, static_cast<const TIn*>(p.v) + vb + v0, p.sv[1], nval);
     x.lu.load_clamped(tid, uu + v0, p.V, C);
     x.ldu.load_clamped(tid, dug + v0, p.V, C);
-    if constexpr (ST16) {
-      x.lS.load_clamped(tid, cks + (int64_t)v0 * K, K, VS);
-      x.ldS.load_clamped(tid, ckd + (int64_t)v0 * K, K, VS);
-    } else {
-      x.lS.load_clamped(tid, cks + v0, p.V, K);
-      x.ldS.load_clamped(tid, ckd + v0, p.V, K);
-    }
-    x.scS[0] = x.scS[1] = x.scD[0] = x.scD[1] = 1.f;
-    if constexpr (ST16) {
+    x.lS.load_clamped(tid, cks + v0, p.V, K);
+    x.ldS.load_clamped(tid, ckd + v0, p.V, K);
 #pragma unroll
-      for (int j = 0; j < VS / 16; ++j) {
-        x.scS[j] = sclS[v0 / 16 + j];
-        x.scD[j] = sclD[v0 / 16 + j];
-      }
-      const int t = tid / (VS / 2), c2 = 2 * (tid % (VS / 2));
-      if (NDP == NTG || tid < NDP)
-        x.rdo[0] = *reinterpret_cast<const uint32_t*>(static_cast<const TIn*>(p.d_o) + dob +
-                                                      (int64_t)min(t, nval - 1) * p.sdo[1] + v0 + c2);
-    } else {
-#pragma unroll
-      for (int i = 0; i < NDO; ++i) {
-        const int e = tid + i * NTG, t = e / VS, c2 = e % VS;
-        x.rdo[i] = t < nval ? load_bits(p.d_o, dob + (int64_t)t * p.sdo[1] + v0 + c2, p.do_dtype) : 0u;
-      }
+    for (int i = 0; i < NDO; ++i) {
+      const int e = tid + i * NTG, t = e / VS, c2 = e % VS;
+      x.rdo[i] = t < nval ? load_bits(p.d_o, dob + (int64_t)t * p.sdo[1] + v0 + c2, p.do_dtype) : 0u;
     }
   };
   auto store_step = [&](const StepRows& x) __attribute__((always_inline)) {
-    if constexpr (F16W) {
-      x.lv.store_raw(tid, s.h.v, nval);
-      x.lu.store_pairs(tid, s.h.uh, s.h.ul);
-      x.ldu.store_pairs(tid, s.h.dh, s.h.dl);
-      x.lS.store_raw(tid, s.h.ST);
-      x.ldS.store_raw(tid, s.h.dST);
-      const int t = tid / (VS / 2), c2 = 2 * (tid % (VS / 2));
-      if (NDP == NTG || tid < NDP) *reinterpret_cast<uint32_t*>(&s.h.dO[t][c2]) = t < nval ? x.rdo[0] : 0u;
-      return;
-    }
     x.lv.store_masked(tid, s.w.v, nval);
     x.lu.store(tid, s.w.u);
     x.ldu.store(tid, s.w.du);
-    if constexpr (ST16) {
-      // [V][K] fp16 rows as they are; the products read them transposed and
-      // scale them back per 16-column slice
-      x.lS.store_raw(tid, s.w.st.h.ST);
-      x.ldS.store_raw(tid, s.w.st.h.dST);
-      {
-        // every thread writes its column's scales (the same value as the
-        // other threads of the column): the scale loads are consumed on
-        // every lane, so they stay where they were issued, a step ahead
-        // (constant indices into the register arrays: a variable index
-        // would put the step's rows in scratch memory)
-        const int v = (tid / (K / 8)) % VS;
-        s.scs[v] = v < 16 ? x.scS[0] : x.scS[VS / 16 - 1];
-        s.scd[v] = v < 16 ? x.scD[0] : x.scD[VS / 16 - 1];
-      }
-      const int t = tid / (VS / 2), c2 = 2 * (tid % (VS / 2));
-      if (NDP == NTG || tid < NDP) {
-        // dO has q's dtype here: a compile-time conversion
-        constexpr int dt = std::is_same<TIn, f16>::value ? GDN_DTYPE_F16 : GDN_DTYPE_BF16;
-        const bool ok = t < nval;
-        s.w.dO[t][c2] = ok ? bits_to_float(x.rdo[0] & 0xffffu, dt) : 0.f;
-        s.w.dO[t][c2 + 1] = ok ? bits_to_float(x.rdo[0] >> 16, dt) : 0.f;
-      }
-    } else {
-      x.lS.store(tid, s.w.st.f.S);
-      x.ldS.store(tid, s.w.st.f.dS);
+    x.lS.store(tid, s.w.S);
+    x.ldS.store(tid, s.w.dS);
 #pragma unroll
-      for (int i = 0; i < NDO; ++i) {
-        const int e = tid + i * NTG;
-        s.w.dO[e / VS][e % VS] = bits_to_float(x.rdo[i], p.do_dtype);
-      }
+    for (int i = 0; i < NDO; ++i) {
+      const int e = tid + i * NTG;
+      s.w.dO[e / VS][e % VS] = bits_to_float(x.rdo[i], p.do_dtype);
     }
   };
   StepRows ra, rb;
@@ -1644,10 +1389,8 @@ __global__ __launch_bounds__(NTG) void grad_kernel(const BArgs p) {
   lq.store(tid, s.q);
   lk.store(tid, s.k);
   lt.store(tid, s.t);
-  if constexpr (!ST16) {
-    lp.store(tid, s.pm);
-    lkk.store(tid, s.kk);
-  }
+  lp.store(tid, s.pm);
+  lkk.store(tid, s.kk);
   if (tid < C) {
     s.b[tid] = gate;
     s.bt[tid] = bits_to_float(bvb, p.beta_dtype);
@@ -1665,62 +1408,22 @@ __global__ __launch_bounds__(NTG) void grad_kernel(const BArgs p) {
     const int t = e / C, j = e % C;
     s.m[t][j] = j <= t ? expf(s.b[t] - s.b[j]) : 0.f;
   }
-  if constexpr (ST16 && !F16W) {
-    // K K^T (waves 0-3) and P = M o Q K^T (waves 4-7) from the 16-bit q
-    // and k rows (the 16-bit prep does not store them): one 16 x 16 tile
-    // per wave, the products exact and the sums in fp32 as in the prep
-    // (fp16 inputs form them after the V walk instead)
-    const int mt = (wave >> 1) & 1, nt = wave & 1;
-    constexpr int KD = GSmem<K, VS>::KD;
-    const float* const arow = (wave < 4 ? &s.k[0][0] : &s.q[0][0]) + (16 * mt + r) * KD + 8 * kq;
-    const float* const brow = &s.k[0][0] + (16 * nt + r) * KD + 8 * kq;
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int kb = 0; kb < K; kb += 32) acc = mma16<TIn>(pack16<TIn>(arow + kb), pack16<TIn>(brow + kb), acc);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int t = 16 * mt + 4 * kq + i, j = 16 * nt + r;
-      if (wave < 4) s.kk[t][j] = acc[i];
-      else s.pm[t][j] = j <= t ? expf(s.b[t] - s.b[j]) * acc[i] : 0.f;
-    }
-  }
   // step vsi: `cur` holds step vsi + 1's rows (loaded a step ago), `nxt`
   // receives step vsi + 2's
-  // this thread's part of <S, dS'> over the step's fp16 state rows ([V][K]
-  // as stored): 8 consecutive keys of state column tid / (K / 8), times the
-  // column's two scales
-  auto state_dot = [&](const auto& st, const auto& dst, float fs, float fd) __attribute__((always_inline)) {
-    static_assert(VS * K / 8 <= NTG, "one 8-key piece per thread at most");
-    float x = 0.f;
-    const int v = tid / (K / 8), k0 = 8 * (tid % (K / 8));
-    if (VS * K / 8 == NTG || tid < VS * K / 8) {
-      const f16x8 a = *reinterpret_cast<const f16x8*>(&st[v][k0]);
-      const f16x8 b = *reinterpret_cast<const f16x8*>(&dst[v][k0]);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) x = __builtin_fmaf((float)a[j], (float)b[j], x);
-    }
-    return x * (fs * fd);
-  };
   auto step = [&](int vsi, StepRows& cur, StepRows& nxt) __attribute__((always_inline)) {
     const int v0 = vsi * VS;
     // dU~ of the step and dv first: its stores go out before the next
     // step's loads, so that waiting for those loads does not wait for them
     if (du_wave) {
       f32x4 a[1] = {f32x4{0.f, 0.f, 0.f, 0.f}};
-      if constexpr (F16W)
-        seg_mfma<1>(a, um0, un0, 1, r, kq,
-                    seg<C>([&](int m, int kk) { return s.t[kk][m]; },
-                           [&](int kk, int n) { return (float)s.h.dh[kk][n] + (float)s.h.dl[kk][n]; }));
-      else
-        seg_mfma<1>(a, um0, un0, 1, r, kq,
+      seg_mfma<1>(a, um0, un0, 1, r, kq,
                     seg<C>([&](int m, int kk) { return s.t[kk][m]; }, [&](int kk, int n) { return s.w.du[kk][n]; }));
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int row = um0[0] + 4 * kq + i;
         const int col = un0[0] + r;
         if (row < nval) stx<TIn>(p.dv, dvb + (int64_t)row * p.sdv[1] + v0 + col, s.bt[row] * a[0][i]);
-        const float vv = F16W ? (float)s.h.v[row][col] : s.w.v[row][col];
-        vu_acc[i] = __builtin_fmaf(vv, a[0][i], vu_acc[i]);
+        vu_acc[i] = __builtin_fmaf(s.w.v[row][col], a[0][i], vu_acc[i]);
       }
     }
     if (vsi + 2 < nvs) load_step(nxt, vsi + 2);
@@ -1728,78 +1431,32 @@ __global__ __launch_bounds__(NTG) void grad_kernel(const BArgs p) {
     // X[m][v] Y[n][v]: the contraction runs in 16-column groups in which
     // lane (r, kq) covers columns 4 kq .. 4 kq + 3 over four MFMA steps, so
     // each operand is one 16-byte read per four steps.
-    if constexpr (F16W) {
-      // lane (r, kq) supplies 8 consecutive columns 8 kq .. of its row; the
-      // accumulators keep the layout of the fp32 products below
-      const int c8 = 8 * kq;
+#pragma unroll
+    for (int c0 = 0; c0 < VS; c0 += 16) {
+      const int cc = c0 + 4 * kq;
 #pragma unroll
       for (int g = 0; g < NPW; ++g) {
         if (g < ana) {
-          // S[an0 + r][8 kq + j] = S^T[8 kq + j][an0 + r]: transposed reads
-          const f16x8 sb = tiles16::frag8_t(s.h.ST, 0, an0[g], r, kq), db = tiles16::frag8_t(s.h.dST, 0, an0[g], r, kq);
-          const f16x8 xo = tiles16::frag8(&s.h.dO[am0[g] + r][c8]);
-          accW[g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(tiles16::frag8(&s.h.dh[am0[g] + r][c8]), sb, accW[g], 0, 0, 0);
-          accW[g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(tiles16::frag8(&s.h.dl[am0[g] + r][c8]), sb, accW[g], 0, 0, 0);
-          accQ[g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xo, sb, accQ[g], 0, 0, 0);
-          accK[g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(tiles16::frag8(&s.h.uh[am0[g] + r][c8]), db, accK[g], 0, 0, 0);
-          accK[g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(tiles16::frag8(&s.h.ul[am0[g] + r][c8]), db, accK[g], 0, 0, 0);
-        }
-      }
-      // dO u^T (waves 0-3) or du V^T (waves 4-7; diag(beta) applied when stored)
-      const f16x8 xh = tiles16::frag8(wave < 4 ? &s.h.dO[cm0[0] + r][c8] : &s.h.dh[cm0[0] + r][c8]);
-      const f16x8 xl = tiles16::frag8(&s.h.dl[cm0[0] + r][c8]);
-      const f16x8 yh = tiles16::frag8(wave < 4 ? &s.h.uh[cn0[0] + r][c8] : &s.h.v[cn0[0] + r][c8]);
-      const f16x8 yl = tiles16::frag8(&s.h.ul[cn0[0] + r][c8]);
-      accC[0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh, yh, accC[0], 0, 0, 0);
-      accC[0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wave < 4 ? xh : xl, wave < 4 ? yl : yh, accC[0], 0, 0, 0);
-      dgc_acc += state_dot(s.h.ST, s.h.dST, 1.f, 1.f);
-    } else {
+          const f32x4 sb = ld4(s.w.S, an0[g] + r, cc), db = ld4(s.w.dS, an0[g] + r, cc);
+          const f32x4 xa = ld4(s.w.du, am0[g] + r, cc), xo = ld4(s.w.dO, am0[g] + r, cc);
+          const f32x4 xu = ld4(s.w.u, am0[g] + r, cc);
 #pragma unroll
-      for (int c0 = 0; c0 < VS; c0 += 16) {
-        const int cc = c0 + 4 * kq;
-#pragma unroll
-        for (int g = 0; g < NPW; ++g) {
-          if (g < ana) {
-            f32x4 sb, db;
-            if constexpr (ST16) {
-              // S[an0 + r][cc + j] = S^T[cc + j][an0 + r]: transposed reads
-              const f16x4 hs = tiles16::frag4_t(s.w.st.h.ST, c0, an0[g], r, kq);
-              const f16x4 hd = tiles16::frag4_t(s.w.st.h.dST, c0, an0[g], r, kq);
-              const float fs = s.scs[c0], fd = s.scd[c0];
-#pragma unroll
-              for (int j = 0; j < 4; ++j) {
-                sb[j] = (float)hs[j] * fs;
-                db[j] = (float)hd[j] * fd;
-              }
-            } else {
-              sb = ld4(s.w.st.f.S, an0[g] + r, cc);
-              db = ld4(s.w.st.f.dS, an0[g] + r, cc);
-            }
-            const f32x4 xa = ld4(s.w.du, am0[g] + r, cc), xo = ld4(s.w.dO, am0[g] + r, cc);
-            const f32x4 xu = ld4(s.w.u, am0[g] + r, cc);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-              accW[g] = __builtin_amdgcn_mfma_f32_16x16x4f32(xa[j], sb[j], accW[g], 0, 0, 0);
-              accQ[g] = __builtin_amdgcn_mfma_f32_16x16x4f32(xo[j], sb[j], accQ[g], 0, 0, 0);
-              accK[g] = __builtin_amdgcn_mfma_f32_16x16x4f32(xu[j], db[j], accK[g], 0, 0, 0);
-            }
+          for (int j = 0; j < 4; ++j) {
+            accW[g] = __builtin_amdgcn_mfma_f32_16x16x4f32(xa[j], sb[j], accW[g], 0, 0, 0);
+            accQ[g] = __builtin_amdgcn_mfma_f32_16x16x4f32(xo[j], sb[j], accQ[g], 0, 0, 0);
+            accK[g] = __builtin_amdgcn_mfma_f32_16x16x4f32(xu[j], db[j], accK[g], 0, 0, 0);
           }
         }
-        // dO u^T (waves 0-3) or du (diag(beta) V)^T (waves 4-7)
-        const f32x4 xc = wave < 4 ? ld4(s.w.dO, cm0[0] + r, cc) : ld4(s.w.du, cm0[0] + r, cc);
-        f32x4 yc = wave < 4 ? ld4(s.w.u, cn0[0] + r, cc) : ld4(s.w.v, cn0[0] + r, cc);
-        if (wave >= 4) yc *= s.bt[cn0[0] + r];
+      }
+      // dO u^T (waves 0-3) or du (diag(beta) V)^T (waves 4-7)
+      const f32x4 xc = wave < 4 ? ld4(s.w.dO, cm0[0] + r, cc) : ld4(s.w.du, cm0[0] + r, cc);
+      f32x4 yc = wave < 4 ? ld4(s.w.u, cn0[0] + r, cc) : ld4(s.w.v, cn0[0] + r, cc);
+      if (wave >= 4) yc *= s.bt[cn0[0] + r];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) accC[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(xc[j], yc[j], accC[0], 0, 0, 0);
-      }
-      if constexpr (ST16) {
-        const int v = (tid / (K / 8)) % VS;
-        dgc_acc += state_dot(s.w.st.h.ST, s.w.st.h.dST, s.scs[v], s.scd[v]);
-      } else {
-        for (int e = tid; e < K * VS; e += NTG)
-          dgc_acc = __builtin_fmaf(s.w.st.f.S[e / VS][e % VS], s.w.st.f.dS[e / VS][e % VS], dgc_acc);
-      }
+      for (int j = 0; j < 4; ++j) accC[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(xc[j], yc[j], accC[0], 0, 0, 0);
     }
+    for (int e = tid; e < K * VS; e += NTG)
+      dgc_acc = __builtin_fmaf(s.w.S[e / VS][e % VS], s.w.dS[e / VS][e % VS], dgc_acc);
     __syncthreads();
     if (vsi + 1 < nvs) {
       store_step(cur);
@@ -1828,11 +1485,6 @@ __global__ __launch_bounds__(NTG) void grad_kernel(const BArgs p) {
       for (int e = 0; e < 4; ++e) {
         const int row = am0[i] + 4 * kq + e, col = an0[i] + r;
         s.dw[row][col] = -accW[i][e];
-        if constexpr (F16W) {
-          const float w = pin(-accW[i][e]);
-          s.x.dwh[row][col] = (f16)w;
-          s.x.dwl[row][col] = (f16)(w - (float)(f16)w);
-        }
         pq[e] = sum16(s.q[row][col] * accQ[i][e]);
         pk[e] = sum16(s.k[row][col] * accK[i][e]);
       }
@@ -1845,30 +1497,14 @@ __global__ __launch_bounds__(NTG) void grad_kernel(const BArgs p) {
       }
     }
   }
-  if constexpr (F16W) {
-    for (int e = tid; e < C * C; e += NTG) {
-      const float x = pin(s.t[e / C][e % C]);
-      s.x.th[e / C][e % C] = (f16)x;
-      s.x.tl[e / C][e % C] = (f16)(x - (float)(f16)x);
-    }
-    // q and k rows in fp16: the raw rows loaded at the start (kept in
-    // registers through the walk; rows past the chunk end are zero)
-    lq.store_raw(tid, s.x.q);
-    lk.store_raw(tid, s.x.k);
-  }
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
     const int row = cm0[0] + 4 * kq + e, col = cn0[0] + r;
     if (wave < 4) {
-      const float y = pin(scale * s.m[row][col] * accC[0][e]);
-      s.y[row][col] = y;
-      if constexpr (!F16W) s.yp[row][col] = scale * accC[0][e] * s.pm[row][col];
-      if constexpr (F16W) {
-        s.x.yh[row][col] = (f16)y;
-        s.x.yl[row][col] = (f16)(y - (float)(f16)y);
-      }
+      s.y[row][col] = scale * s.m[row][col] * accC[0][e];
+      s.yp[row][col] = scale * accC[0][e] * s.pm[row][col];
     } else {
-      s.dt[row][col] = F16W ? s.bt[col] * accC[0][e] : accC[0][e];
+      s.dt[row][col] = accC[0][e];
     }
   }
   if (du_wave) {
@@ -1886,72 +1522,12 @@ __global__ __launch_bounds__(NTG) void grad_kernel(const BArgs p) {
   }
   __syncthreads();
   // dT = du (beta V)^T + dW (beta gam K)^T;  dW~ = T^T dW
-  f32x4 aw[NPW];  // fp16 inputs: dW~ in the tiles of accW
-  if constexpr (F16W) {
-    // fp16 MFMA on hi + lo pairs; transposed operands (T^T, dW columns) by
-    // ds_read_b64_tr_b16.  dT: waves 0-3, one 16 x 16 tile each.
-    if (wave < 4) {
-      const int dm = (wave >> 1) * 16, dn = (wave & 1) * 16;
-      f32x4 a = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int kb = 0; kb < K; kb += 32) {
-        const f16x8 kf = tiles16::frag8(&s.x.k[dn + r][kb + 8 * kq]);
-        a = __builtin_amdgcn_mfma_f32_16x16x32_f16(tiles16::frag8(&s.x.dwh[dm + r][kb + 8 * kq]), kf, a, 0, 0, 0);
-        a = __builtin_amdgcn_mfma_f32_16x16x32_f16(tiles16::frag8(&s.x.dwl[dm + r][kb + 8 * kq]), kf, a, 0, 0, 0);
-      }
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int row = dm + 4 * kq + e, col = dn + r;
-        const float x = pin(s.dt[row][col] + s.bt[col] * s.gam[col] * a[e]);
-        s.dt[row][col] = x;
-        s.x.dth[row][col] = (f16)x;
-        s.x.dtl[row][col] = (f16)(x - (float)(f16)x);
-      }
-    } else {
-      // K K^T and Q K^T (the 16-bit prep does not store them; exact
-      // products of the fp16 rows), one 16 x 16 tile of each per wave:
-      // K K^T -> kk, dQK o Q K^T = y o Q K^T -> yp
-      const int pm0 = ((wave - 4) >> 1) * 16, pn0 = (wave & 1) * 16;
-      f32x4 akk = {0.f, 0.f, 0.f, 0.f}, aqk = akk;
-#pragma unroll
-      for (int kb = 0; kb < K; kb += 32) {
-        const f16x8 kf = tiles16::frag8(&s.x.k[pn0 + r][kb + 8 * kq]);
-        akk = __builtin_amdgcn_mfma_f32_16x16x32_f16(tiles16::frag8(&s.x.k[pm0 + r][kb + 8 * kq]), kf, akk, 0, 0, 0);
-        aqk = __builtin_amdgcn_mfma_f32_16x16x32_f16(tiles16::frag8(&s.x.q[pm0 + r][kb + 8 * kq]), kf, aqk, 0, 0, 0);
-      }
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int row = pm0 + 4 * kq + e, col = pn0 + r;
-        s.kk[row][col] = akk[e];
-        s.yp[row][col] = s.y[row][col] * aqk[e];
-      }
-    }
-#pragma unroll
-    for (int g = 0; g < NPW; ++g) {
-      aw[g] = f32x4{0.f, 0.f, 0.f, 0.f};
-      if (g < ana) {
-        const f16x8 th = tiles16::frag8_t(s.x.th, 0, am0[g], r, kq), tl = tiles16::frag8_t(s.x.tl, 0, am0[g], r, kq);
-        const f16x8 wh = tiles16::frag8_t(s.x.dwh, 0, an0[g], r, kq);
-        aw[g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(th, wh, aw[g], 0, 0, 0);
-        aw[g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(th, tiles16::frag8_t(s.x.dwl, 0, an0[g], r, kq), aw[g], 0,
-                                                       0, 0);
-        aw[g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(tl, wh, aw[g], 0, 0, 0);
-        float pw[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) pw[e] = sum16(s.k[am0[g] + 4 * kq + e][an0[g] + r] * aw[g][e]);
-        if (r == 0) {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) s.rw[an0[g] / 16][am0[g] + 4 * kq + e] = pw[e];
-        }
-      }
-    }
-  } else {
-    mmx<NTG, C, C>(tid, [&](int m, int n, float x) { s.dt[m][n] += x; },
-                   seg<K>([&](int m, int kk) { return s.dw[m][kk]; },
-                          [&](int kk, int n) { return s.bt[n] * s.gam[n] * s.k[n][kk]; }));
-    mmx<NTG, C, K>(tid, [&](int m, int n, float x) { s.dwt[m][n] = x; },
-                   seg<C>([&](int m, int kk) { return s.t[kk][m]; }, [&](int kk, int n) { return s.dw[kk][n]; }));
-  }
+  mmx<NTG, C, C>(tid, [&](int m, int n, float x) { s.dt[m][n] += x; },
+                 seg<K>([&](int m, int kk) { return s.dw[m][kk]; },
+                        [&](int kk, int n) { return s.bt[n] * s.gam[n] * s.k[n][kk]; }));
+  mmx<NTG, C, K>(tid, [&](int m, int n, float x) { s.dwt[m][n] = x; },
+                 seg<C>([&](int m, int kk) { return s.t[kk][m]; }, [&](int kk, int n) { return s.dw[kk][n]; }));
+
   if (tid < C) {
     float a = 0.f, b = 0.f;
     for (int j = 0; j < NCT; ++j) {
@@ -1968,53 +1544,16 @@ __global__ __launch_bounds__(NTG) void grad_kernel(const BArgs p) {
   }
   __syncthreads();
   // Z = T^T dT;  k_t.dW~_t
-  if constexpr (F16W) {
-    if (wave < 4) {
-      const int zm = (wave >> 1) * 16, zn = (wave & 1) * 16;
-      const f16x8 th = tiles16::frag8_t(s.x.th, 0, zm, r, kq), dh = tiles16::frag8_t(s.x.dth, 0, zn, r, kq);
-      f32x4 a = {0.f, 0.f, 0.f, 0.f};
-      a = __builtin_amdgcn_mfma_f32_16x16x32_f16(th, dh, a, 0, 0, 0);
-      a = __builtin_amdgcn_mfma_f32_16x16x32_f16(th, tiles16::frag8_t(s.x.dtl, 0, zn, r, kq), a, 0, 0, 0);
-      a = __builtin_amdgcn_mfma_f32_16x16x32_f16(tiles16::frag8_t(s.x.tl, 0, zm, r, kq), dh, a, 0, 0, 0);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int row = zm + 4 * kq + e, col = zn + r;
-        const float z = pin(a[e]);
-        s.x.zh[row][col] = (f16)z;
-        s.x.zl[row][col] = (f16)(z - (float)(f16)z);
-      }
-    }
-    if (tid < C) {
-      float x = 0.f;
-      for (int j = 0; j < NCT; ++j) x += s.rw[j][tid];
-      s.kw[tid] = x;
-    }
-  } else {
-    mmx<NTG, C, C>(tid, [&](int m, int n, float x) { s.z[m][n] = x; },
-                   seg<C>([&](int m, int kk) { return s.t[kk][m]; }, [&](int kk, int n) { return s.dt[kk][n]; }));
-    const float kw = row_sum<NTG, C, K>(tid, [&](int rr, int i) { return s.k[rr][i] * s.dwt[rr][i]; });
-    if (tid % RL == 0) s.kw[tid / RL] = kw;
-  }
+  mmx<NTG, C, C>(tid, [&](int m, int n, float x) { s.z[m][n] = x; },
+                 seg<C>([&](int m, int kk) { return s.t[kk][m]; }, [&](int kk, int n) { return s.dt[kk][n]; }));
+  const float kw = row_sum<NTG, C, K>(tid, [&](int rr, int i) { return s.k[rr][i] * s.dwt[rr][i]; });
+  if (tid % RL == 0) s.kw[tid / RL] = kw;
+
   __syncthreads();
   // dA = -tril_-1(Z T^T) -> dt
-  if constexpr (F16W) {
-    if (wave < 4) {
-      const int am = (wave >> 1) * 16, an = (wave & 1) * 16;
-      const f16x8 zh = tiles16::frag8(&s.x.zh[am + r][8 * kq]), th = tiles16::frag8(&s.x.th[an + r][8 * kq]);
-      f32x4 a = {0.f, 0.f, 0.f, 0.f};
-      a = __builtin_amdgcn_mfma_f32_16x16x32_f16(zh, th, a, 0, 0, 0);
-      a = __builtin_amdgcn_mfma_f32_16x16x32_f16(zh, tiles16::frag8(&s.x.tl[an + r][8 * kq]), a, 0, 0, 0);
-      a = __builtin_amdgcn_mfma_f32_16x16x32_f16(tiles16::frag8(&s.x.zl[am + r][8 * kq]), th, a, 0, 0, 0);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int row = am + 4 * kq + e, col = an + r;
-        s.dt[row][col] = col < row ? -a[e] : 0.f;
-      }
-    }
-  } else {
-    mmx<NTG, C, C>(tid, [&](int m, int n, float x) { s.dt[m][n] = n < m ? -x : 0.f; },
-                   seg<C>([&](int m, int kk) { return s.z[m][kk]; }, [&](int kk, int n) { return s.t[n][kk]; }));
-  }
+  mmx<NTG, C, C>(tid, [&](int m, int n, float x) { s.dt[m][n] = n < m ? -x : 0.f; },
+                 seg<C>([&](int m, int kk) { return s.z[m][kk]; }, [&](int kk, int n) { return s.t[n][kk]; }));
+
   __syncthreads();
   // dKK = dA o beta_t M -> z;  dbeta and db
   for (int e = tid; e < C * C; e += NTG) {
@@ -2043,16 +1582,6 @@ __global__ __launch_bounds__(NTG) void grad_kernel(const BArgs p) {
     }
   }
   __syncthreads();
-  if constexpr (F16W) {
-    // dKK + dKK^T as fp16 pairs for the dk product (published by the
-    // barrier below)
-    for (int e = tid; e < C * C; e += NTG) {
-      const int t = e / C, j = e % C;
-      const float zz = pin(s.z[t][j] + s.z[j][t]);
-      s.x.zh[t][j] = (f16)zz;
-      s.x.zl[t][j] = (f16)(zz - (float)(f16)zz);
-    }
-  }
   if (wave == 0) {
     // dg_t = sum_{j >= t} db_j: lane l scans db[C - 1 - l]
     const float x = scan32(lane < C ? s.db[C - 1 - lane] : 0.f);
@@ -2070,35 +1599,14 @@ __global__ __launch_bounds__(NTG) void grad_kernel(const BArgs p) {
       aq[i] = f32x4{0.f, 0.f, 0.f, 0.f};
       ak[i] = aq[i];
     }
-    if constexpr (F16W) {
-      __syncthreads();  // the dKK + dKK^T pairs
-      // lane (r, kq): rows of dQK / dQK^T / dKK + dKK^T (A) and columns of
-      // K / Q (B), contraction indices 8 kq .. 8 kq + 7 of the C = 32
-#pragma unroll
-      for (int g = 0; g < NPW; ++g) {
-        if (g < ana) {
-          const f16x8 kt = tiles16::frag8_t(s.x.k, 0, an0[g], r, kq);
-          const f16x8 qt = tiles16::frag8_t(s.x.q, 0, an0[g], r, kq);
-          const int m = am0[g] + r;
-          aq[g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(tiles16::frag8(&s.x.yh[m][8 * kq]), kt, aq[g], 0, 0, 0);
-          aq[g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(tiles16::frag8(&s.x.yl[m][8 * kq]), kt, aq[g], 0, 0, 0);
-          ak[g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(tiles16::frag8_t(s.x.yh, 0, am0[g], r, kq), qt, ak[g], 0,
-                                                         0, 0);
-          ak[g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(tiles16::frag8_t(s.x.yl, 0, am0[g], r, kq), qt, ak[g], 0,
-                                                         0, 0);
-          ak[g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(tiles16::frag8(&s.x.zh[m][8 * kq]), kt, ak[g], 0, 0, 0);
-          ak[g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(tiles16::frag8(&s.x.zl[m][8 * kq]), kt, ak[g], 0, 0, 0);
-        }
-      }
-    } else {
-      seg_mfma<NPW>(aq, am0, an0, ana, r, kq,
-                    seg<C>([&](int m, int kk) { return s.y[m][kk]; }, [&](int kk, int n) { return s.k[kk][n]; }));
-      seg_mfma<NPW>(ak, am0, an0, ana, r, kq,
-                    seg<C>([&](int m, int kk) { return s.y[kk][m]; }, [&](int kk, int n) { return s.q[kk][n]; }));
-      seg_mfma<NPW>(ak, am0, an0, ana, r, kq,
-                    seg<C>([&](int m, int kk) { return s.z[m][kk] + s.z[kk][m]; },
-                           [&](int kk, int n) { return s.k[kk][n]; }));
-    }
+    seg_mfma<NPW>(aq, am0, an0, ana, r, kq,
+                  seg<C>([&](int m, int kk) { return s.y[m][kk]; }, [&](int kk, int n) { return s.k[kk][n]; }));
+    seg_mfma<NPW>(ak, am0, an0, ana, r, kq,
+                  seg<C>([&](int m, int kk) { return s.y[kk][m]; }, [&](int kk, int n) { return s.q[kk][n]; }));
+    seg_mfma<NPW>(ak, am0, an0, ana, r, kq,
+                  seg<C>([&](int m, int kk) { return s.z[m][kk] + s.z[kk][m]; },
+                         [&](int kk, int n) { return s.k[kk][n]; }));
+
 #pragma unroll
     for (int i = 0; i < NPW; ++i) {
       if (i < ana) {
@@ -2107,8 +1615,7 @@ __global__ __launch_bounds__(NTG) void grad_kernel(const BArgs p) {
           const int row = am0[i] + 4 * kq + e, col = an0[i] + r;
           if (row < nval) {
             const float dq = aq[i][e] + scale * s.gam[row] * accQ[i][e];
-            const float dwt = F16W ? aw[i][e] : s.dwt[row][col];
-            const float dk = ak[i][e] + s.D[row] * accK[i][e] + s.bt[row] * s.gam[row] * dwt;
+            const float dk = ak[i][e] + s.D[row] * accK[i][e] + s.bt[row] * s.gam[row] * s.dwt[row][col];
             stx<TIn>(p.dq, dqb + (int64_t)row * p.sdq[1] + col, dq);
             stx<TIn>(p.dk, dkb + (int64_t)row * p.sdk[1] + col, dk);
           }
@@ -2173,17 +1680,15 @@ int launch_k(const BArgs& a, int64_t nrec, hipStream_t s) {
   }
   if (nrec > 0) {
     const dim3 grid((unsigned)nrec);
-    const bool st16 = !std::is_same<TIn, float>::value && a.w16;
-    if (a.V == 128) {
-      if (st16) hipLaunchKernelGGL((grad_kernel<TIn, K, 32, true, 4>), grid, dim3(NTG), 0, s, a);
-      else hipLaunchKernelGGL((grad_kernel<TIn, K, 32, false, 4>), grid, dim3(NTG), 0, s, a);
-    } else if (a.V % 32 == 0) {
-      if (st16) hipLaunchKernelGGL((grad_kernel<TIn, K, 32, true, 0>), grid, dim3(NTG), 0, s, a);
-      else hipLaunchKernelGGL((grad_kernel<TIn, K, 32, false, 0>), grid, dim3(NTG), 0, s, a);
-    } else {
-      if (st16) hipLaunchKernelGGL((grad_kernel<TIn, K, 16, true, 0>), grid, dim3(NTG), 0, s, a);
-      else hipLaunchKernelGGL((grad_kernel<TIn, K, 16, false, 0>), grid, dim3(NTG), 0, s, a);
+    if constexpr (!std::is_same<TIn, float>::value) {
+      if (a.w16) {
+        hipLaunchKernelGGL((grad16_kernel<TIn, K>), grid, dim3(2 * K), 0, s, a);
+        return (int)hipGetLastError();
+      }
     }
+    if (a.V == 128) hipLaunchKernelGGL((grad_kernel<TIn, K, 32, 4>), grid, dim3(NTG), 0, s, a);
+    else if (a.V % 32 == 0) hipLaunchKernelGGL((grad_kernel<TIn, K, 32, 0>), grid, dim3(NTG), 0, s, a);
+    else hipLaunchKernelGGL((grad_kernel<TIn, K, 16, 0>), grid, dim3(NTG), 0, s, a);
   }
   return (int)hipGetLastError();
 }
@@ -2431,6 +1936,11 @@ static int bwd_launch_one(const GdnBwdParams& P, hipStream_t s) {
   a.xcd_remap = (units % 8 == 0) ? 1 : 0;
   // fp16 pair recurrences (the 16-bit walks)
   a.w16 = w16;
+  auto rows16 = [](const void* ptr, const int64_t* st) {
+    return reinterpret_cast<uintptr_t>(ptr) % 16 == 0 && st[0] % 8 == 0 && st[1] % 8 == 0 && st[2] % 8 == 0;
+  };
+  a.vec = (rows16(P.d_o, P.do_stride) ? bwd::VEC_DO : 0) | (rows16(P.dq, P.dq_stride) ? bwd::VEC_DQ : 0) |
+          (rows16(P.dk, P.dk_stride) ? bwd::VEC_DK : 0) | (rows16(P.dv, P.dv_stride) ? bwd::VEC_DV : 0);
 
   const int64_t nrec_launch = P.T > 0 ? nrec : 0;
   switch (P.qkv_dtype) {
