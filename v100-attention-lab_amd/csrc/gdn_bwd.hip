@@ -671,17 +671,9 @@ __device__ __forceinline__ void walk_backward(const BArgs& p, RSmem<K>& s, const
 template <typename TIn, int K>
 __global__ __launch_bounds__(NTP) void recur_kernel(const BArgs p) {
   __shared__ FRSmem<K> sm;
-  int blk = blockIdx.x;
-  const bool backward = blk >= p.units;
-  if (backward) blk -= p.units;
-  // consecutive units (the V-slices of one head) on one XCD: they read the
-  // same records
-  int unit = blk;
-  if (p.xcd_remap) unit = (blk & 7) * (p.units >> 3) + (blk >> 3);
-  const int vs = unit % p.nv;
-  const int bh = unit / p.nv;
-  const int bi = bh / p.H;
-  const int hi = bh % p.H;
+  const ScanUnit su = scan_unit<2>(p.cu, p.T, p.B, p.H, p.nv, blockIdx.x);
+  const int bi = su.bi, hi = su.hi, vs = su.vs;
+  const bool backward = su.dir != 0;
   const RowSpan rs = row_span(p.cu, p.T, bi);
   const int64_t slot0 = p.cu ? rs.t0 / C + bi : (int64_t)bi * p.nchmax;
   if (backward) walk_backward<TIn, K>(p, sm.r, rs, bi, hi, vs * BV, slot0);
@@ -1220,15 +1212,9 @@ __device__ __forceinline__ void walk_backward16(const BArgs& p, RMem<K>& s, cons
 template <typename TIn, int K>
 __global__ __launch_bounds__(NTP) void recur16_kernel(const BArgs p) {
   __shared__ w16::Mem<K> sm;
-  int blk = blockIdx.x;
-  const bool backward = blk >= p.units;
-  if (backward) blk -= p.units;
-  int unit = blk;
-  if (p.xcd_remap) unit = (blk & 7) * (p.units >> 3) + (blk >> 3);
-  const int vs = unit % p.nv;
-  const int bh = unit / p.nv;
-  const int bi = bh / p.H;
-  const int hi = bh % p.H;
+  const ScanUnit su = scan_unit<2>(p.cu, p.T, p.B, p.H, p.nv, blockIdx.x);
+  const int bi = su.bi, hi = su.hi, vs = su.vs;
+  const bool backward = su.dir != 0;
   const RowSpan rs = row_span(p.cu, p.T, bi);
   const int64_t slot0 = p.cu ? rs.t0 / C + bi : (int64_t)bi * p.nchmax;
   if (backward) w16::walk_backward16<TIn, K>(p, sm.r, rs, bi, hi, vs * BV, slot0);
@@ -1933,7 +1919,6 @@ static int bwd_launch_one(const GdnBwdParams& P, hipStream_t s) {
   a.scale = P.scale;
   a.g_dtype = P.g_dtype; a.beta_dtype = P.beta_dtype; a.do_dtype = P.do_dtype;
   a.cu = P.cu_seqlens;
-  a.xcd_remap = (units % 8 == 0) ? 1 : 0;
   // fp16 pair recurrences (the 16-bit walks)
   a.w16 = w16;
   auto rows16 = [](const void* ptr, const int64_t* st) {

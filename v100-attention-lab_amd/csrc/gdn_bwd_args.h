@@ -49,7 +49,6 @@ struct BArgs {
   float scale;
   int g_dtype, beta_dtype, do_dtype;
   const int64_t* cu;
-  int xcd_remap;
 };
 
 // Rows of dO, dq, dk, dv that start 16-byte aligned (the others are walked

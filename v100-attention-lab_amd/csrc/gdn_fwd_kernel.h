@@ -441,6 +441,81 @@ __device__ __forceinline__ RowSpan row_span(const int64_t* cu, int T, int bi) {
 
 __device__ __forceinline__ RowSpan row_span(const KArgs& p, int bi) { return row_span(p.cu, p.T, bi); }
 
+// Chunk slot -> (sequence, its rows, chunk).  False for a slot that holds
+// no chunk (the gaps between packed sequences).
+// p: B (sequences when cu is set), T, nchmax = ceil(T / C), cu.
+template <int C, typename Args>
+__device__ __forceinline__ bool slot_chunk(const Args& p, int64_t slot, RowSpan& rs, int& c, int& seq) {
+  if (p.cu == nullptr) {
+    seq = (int)(slot / p.nchmax);
+    c = (int)(slot % p.nchmax);
+    rs = row_span(nullptr, p.T, seq);
+    return seq < p.B && (int64_t)c * C < rs.T;
+  }
+  // the last sequence whose first slot floor(t0 / C) + i is <= slot
+  int lo = 0, hi = p.B - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (row_span(p.cu, p.T, mid).t0 / C + mid <= slot) lo = mid;
+    else hi = mid - 1;
+  }
+  rs = row_span(p.cu, p.T, lo);
+  seq = lo;
+  const int64_t cc = slot - (rs.t0 / C + lo);
+  c = (int)cc;
+  return cc >= 0 && cc * C < rs.T;
+}
+template <int C, typename Args>
+__device__ __forceinline__ bool slot_chunk(const Args& p, int64_t slot, RowSpan& rs, int& c) {
+  int seq;
+  return slot_chunk<C>(p, slot, rs, c, seq);
+}
+
+// Packed sequences, longest first.  Every scan workgroup walks one sequence,
+// so the last ones to start should be the short ones: in the order of the
+// offsets a long sequence at the end of a batch ran alone on its CUs (7
+// sequences of 3 to 2900 rows, 16 heads: backward walks 664 us, 314 us
+// longest first).  The rank-th longest of N <= 64 sequences (ties in order),
+// found by every wave for itself: all 64 lanes must be active.
+constexpr int kMaxRanked = 64;
+__device__ __forceinline__ int seq_of_rank(const int64_t* cu, int T, int N, int rank) {
+  const int lane = threadIdx.x & 63;
+  const int len = lane < N ? row_span(cu, T, lane).T : -1;
+  int r = 0;
+  for (int i = 0; i < N; ++i) {
+    const int li = __builtin_amdgcn_readlane(len, i);
+    r += (li > len || (li == len && i < lane)) ? 1 : 0;
+  }
+  return __builtin_ctzll(__ballot(lane < N && r == rank));
+}
+
+// Scan workgroup blk of B sequences x H heads x nv V-slices (x NDIR
+// directions, the forward ones first) -> (sequence, head, slice, direction).
+// Eight consecutive workgroups go to the eight XCDs: the V-slices of a head
+// share one, and with it its L2.
+struct ScanUnit {
+  int bi, hi, vs, dir;
+};
+template <int NDIR>
+__device__ __forceinline__ ScanUnit scan_unit(const int64_t* cu, int T, int B, int H, int nv, int blk) {
+  ScanUnit x;
+  int u = blk, per = B * H * nv;
+  int first = 0;  // the sequence of unit 0
+  if (cu != nullptr && B <= kMaxRanked) {
+    per = H * nv;
+    first = seq_of_rank(cu, T, B, blk / (per * NDIR));
+    u = blk % (per * NDIR);
+  }
+  x.dir = NDIR == 2 && u >= per ? 1 : 0;
+  u -= x.dir * per;
+  if (per % 8 == 0) u = (u & 7) * (per >> 3) + (u >> 3);
+  x.vs = u % nv;
+  const int bh = u / nv;
+  x.hi = bh % H;
+  x.bi = first + bh / H;
+  return x;
+}
+
 // Element offset of the first row of head h in a [B, T, H, *] tensor with
 // (b, t, h) strides s.
 __device__ __forceinline__ int64_t head_base(const RowSpan& r, int h, const int64_t* s) {

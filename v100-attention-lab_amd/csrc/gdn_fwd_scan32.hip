@@ -94,11 +94,11 @@ struct SArgs {
   int B, T, H, V, nv;  // B: sequences (units of row_span)
   int c0, L;           // this segment: chunks [c0, c0 + L) of every sequence
   int first;           // initial state from h0 (or zero) rather than final_state
-  int nrec;            // B * H * L
+  int nrec;            // record jobs (rec_coords)
+  int nchmax;          // ceil(T / C)
   float scale;
   int g_dtype, beta_dtype, o_dtype;
   const int64_t* cu;
-  int xcd_remap;
   int o_vec;           // o takes 16-byte stores (base and strides aligned for them)
 };
 
@@ -228,13 +228,25 @@ __device__ __forceinline__ unsigned long long ps_now() {
 // 1. records
 // ---------------------------------------------------------------------------
 
-// Record r of a segment is (sequence bi, head hi, chunk c0 + lc) with
-// r = (bi * H + hi) * L + lc.
-__device__ __forceinline__ void rec_coords(const SArgs& p, int r, int& bi, int& hi, int& lc) {
-  lc = r % p.L;
-  const int bh = r / p.L;
-  hi = bh % p.H;
-  bi = bh / p.H;
+// Record job r of a segment -> (sequence bi, head hi, its rows, chunk c0 + lc);
+// the record is number (bi H + hi) L + lc.  A dense batch has one job per
+// record.  Packed sequences have one per chunk slot and head (the B sequences
+// share ceil(T / C) + B slots, far fewer than B L): false where the slot's
+// chunk is not of this segment.
+__device__ __forceinline__ bool rec_coords(const SArgs& p, int r, RowSpan& rs, int& bi, int& hi, int& lc) {
+  if (p.cu == nullptr) {
+    lc = r % p.L;
+    const int bh = r / p.L;
+    hi = bh % p.H;
+    bi = bh / p.H;
+    rs = row_span(nullptr, p.T, bi);
+    return (p.c0 + lc) * C < rs.T;
+  }
+  hi = r % p.H;
+  int cc;
+  if (!slot_chunk<C>(p, r / p.H, rs, cc, bi)) return false;
+  lc = cc - p.c0;
+  return lc >= 0 && lc < p.L;
 }
 
 template <typename TIn, int K>
@@ -257,6 +269,7 @@ __global__ __launch_bounds__(256) void rec32_kernel(const SArgs p) {
   const char* kh[2];
   char* rp[2];
   uint32_t skb[2];
+  int64_t gof[2], bof[2];
 #pragma unroll
   for (int e = 0; e < 2; ++e) {
     const int r = (blockIdx.x * 4 + wave) * 2 + e;
@@ -264,17 +277,17 @@ __global__ __launch_bounds__(256) void rec32_kernel(const SArgs p) {
     kh[e] = nullptr;
     rp[e] = nullptr;
     skb[e] = 0;
-    if (r < p.nrec) {
-      int bi, hi, lc;
-      rec_coords(p, r, bi, hi, lc);
-      const RowSpan rs = row_span(p.cu, p.T, bi);
+    gof[e] = bof[e] = 0;
+    RowSpan rs;
+    int bi, hi, lc;
+    if (r < p.nrec && rec_coords(p, r, rs, bi, hi, lc)) {
       const int t0 = (p.c0 + lc) * C;
-      if (t0 < rs.T) {
-        nval[e] = min(C, rs.T - t0);
-        kh[e] = static_cast<const char*>(p.k) + (head_base(rs, hi, p.sk) + (int64_t)t0 * p.sk[1]) * EB;
-        skb[e] = (uint32_t)p.sk[1] * EB;
-        rp[e] = p.rec + (int64_t)r * rec_stride<TIn, K>();
-      }
+      nval[e] = min(C, rs.T - t0);
+      kh[e] = static_cast<const char*>(p.k) + (head_base(rs, hi, p.sk) + (int64_t)t0 * p.sk[1]) * EB;
+      skb[e] = (uint32_t)p.sk[1] * EB;
+      rp[e] = p.rec + ((int64_t)(bi * p.H + hi) * p.L + lc) * rec_stride<TIn, K>();
+      gof[e] = head_base(rs, hi, p.sg) + (int64_t)t0 * p.sg[1];
+      bof[e] = head_base(rs, hi, p.sb) + (int64_t)t0 * p.sb[1];
     }
   }
   // k rows (rows past the end re-read the last row: finite values whose
@@ -293,17 +306,9 @@ __global__ __launch_bounds__(256) void rec32_kernel(const SArgs p) {
     }
   }
   float gv = 0.f, bv = 0.f;
-  {
-    const int e = half;
-    const int r = (blockIdx.x * 4 + wave) * 2 + e;
-    if (r < p.nrec && c < nval[e]) {
-      int bi, hi, lc;
-      rec_coords(p, r, bi, hi, lc);
-      const RowSpan rs = row_span(p.cu, p.T, bi);
-      const int64_t t = (int64_t)(p.c0 + lc) * C + c;
-      gv = load_scalar(p.g, head_base(rs, hi, p.sg) + t * p.sg[1], p.g_dtype);
-      bv = load_scalar(p.beta, head_base(rs, hi, p.sb) + t * p.sb[1], p.beta_dtype);
-    }
+  if (c < (half ? nval[1] : nval[0])) {
+    gv = load_scalar(p.g, (half ? gof[1] : gof[0]) + (int64_t)c * p.sg[1], p.g_dtype);
+    bv = load_scalar(p.beta, (half ? bof[1] : bof[0]) + (int64_t)c * p.sb[1], p.beta_dtype);
   }
   // gates (lanes 0-31: record 0, lanes 32-63: record 1)
   const float b = scan32(gv);
@@ -587,13 +592,8 @@ __global__ __launch_bounds__((64 * scan_waves<BV, SPLIT>())) void scan32_kernel(
   const int n = lane & 15;
   const int gq = lane >> 4;
 
-  int unit = blockIdx.x;
-  if (p.xcd_remap) unit = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
-  const int vs = unit % p.nv;
-  const int bh = unit / p.nv;
-  const int bi = bh / p.H;
-  const int hi = bh % p.H;
-  const int v0 = vs * BV;
+  const ScanUnit su = scan_unit<1>(p.cu, p.T, p.B, p.H, p.nv, blockIdx.x);
+  const int bi = su.bi, hi = su.hi, v0 = su.vs * BV;
   const RowSpan rs = row_span(p.cu, p.T, bi);
   const int T = rs.T;
   const int nch_all = (T + C - 1) / C;
@@ -1285,7 +1285,6 @@ int scan32_launch(const GdnFwdParams& P, int bv, int seg_chunks, hipStream_t str
   a.g_dtype = P.g_dtype; a.beta_dtype = P.beta_dtype; a.o_dtype = P.o_dtype;
   a.cu = P.cu_seqlens;
   const int64_t units = (int64_t)P.B * P.H * a.nv;
-  a.xcd_remap = (units % 8 == 0) ? 1 : 0;
   {
     // 16-byte stores of o: 8 consecutive 16-bit elements or 4 fp32 ones
     // per lane (base 16-byte aligned, every stride a multiple of that many
@@ -1299,7 +1298,8 @@ int scan32_launch(const GdnFwdParams& P, int bv, int seg_chunks, hipStream_t str
   const int L = nchmax > 0 ? (seg_chunks < nchmax ? seg_chunks : nchmax) : 1;
   const int nseg = nchmax > 0 ? (nchmax + L - 1) / L : 1;
   a.L = L;
-  a.nrec = (int)((int64_t)P.B * P.H * L);
+  a.nchmax = nchmax;
+  a.nrec = (int)(P.cu_seqlens ? (int64_t)(nchmax + P.B) * P.H : (int64_t)P.B * P.H * L);
   for (int sg = 0; sg < nseg; ++sg) {
     a.c0 = sg * L;
     a.first = sg == 0;

@@ -243,35 +243,5 @@ __device__ __forceinline__ f32x4 ld4(const float (*x)[LD], int row, int col) {
   return *reinterpret_cast<const f32x4*>(&x[row][col]);
 }
 
-// Chunk slot -> (sequence, its rows, chunk).  False for a slot that holds
-// no chunk (the gaps between packed sequences).
-// p: B (sequences when cu is set), T, nchmax = ceil(T / C), cu.
-template <int C, typename Args>
-__device__ __forceinline__ bool slot_chunk(const Args& p, int64_t slot, RowSpan& rs, int& c, int& seq) {
-  if (p.cu == nullptr) {
-    seq = (int)(slot / p.nchmax);
-    c = (int)(slot % p.nchmax);
-    rs = row_span(nullptr, p.T, seq);
-    return seq < p.B && (int64_t)c * C < rs.T;
-  }
-  // the last sequence whose first slot floor(t0 / C) + i is <= slot
-  int lo = 0, hi = p.B - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (row_span(p.cu, p.T, mid).t0 / C + mid <= slot) lo = mid;
-    else hi = mid - 1;
-  }
-  rs = row_span(p.cu, p.T, lo);
-  seq = lo;
-  const int64_t cc = slot - (rs.t0 / C + lo);
-  c = (int)cc;
-  return cc >= 0 && cc * C < rs.T;
-}
-template <int C, typename Args>
-__device__ __forceinline__ bool slot_chunk(const Args& p, int64_t slot, RowSpan& rs, int& c) {
-  int seq;
-  return slot_chunk<C>(p, slot, rs, c, seq);
-}
-
 }  // namespace tiles
 }  // namespace gdn
