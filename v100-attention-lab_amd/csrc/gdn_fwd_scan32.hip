@@ -228,13 +228,169 @@ __device__ __forceinline__ unsigned long long ps_now() {
 // 1. records
 // ---------------------------------------------------------------------------
 
+// ---------------------------------------------------------------------------
+// short sequences: the step recurrence itself
+// ---------------------------------------------------------------------------
+
+// Sequences of at most this many rows are walked step by step, whatever the
+// batch holds beside them (packed runs give the bits of separate ones).  A
+// row costs about 1.1 us, the records and the scan of one chunk the same for 1
+// to 32 rows.  K = V = 128, us at 1 / 4 rows against those two launches:
+// 4 heads fp16 5.2 / 8.0 against 9.8, bf16 5.2 / 8.4 against 11.3; 256 heads
+// bf16 10.0 / 13.5 against 27; 2048 heads bf16 47 / 71 against 146.  At 6 rows
+// and 4 heads fp16 it is 11.5 against 9.8.
+constexpr int kShortRows = 4;
+
+// One wave: 16 columns (v0 ..) of the state of one sequence and head, row by
+// row in fp32.  Lane (rg = lane / 4, cl = lane % 4) holds the K / 16 keys of
+// group rg and columns 4 cl .. + 3.  With S the state before the row's decay,
+//   u = beta (v - e^g k S),  o = scale (e^g q S + (q.k) u),  S <- e^g S + k u:
+// k S, q S and q.k are summed over the 16 groups in one go (DPP and
+// v_permlane swaps), so a row is one dependent trip across the wave.  NT rows'
+// inputs are loaded at a time.  The arithmetic is spelled out (explicit fma),
+// so that every instance gives the same bits.
+template <typename TIn, int K, int NT>
+__device__ __forceinline__ void short_walk(const SArgs& p, const RowSpan& rs, int bi, int hi, int v0) {
+  constexpr int NK = K / 16;
+  const int lane = threadIdx.x & 63, rg = lane >> 2, cl = lane & 3;
+  const int k0 = NK * rg, c0 = v0 + 4 * cl;
+  // [K][V] states with unit stride along V or along K, rows 16-byte aligned,
+  // move in 16-byte pieces; any other strides element by element
+  auto piece = [](const void* ptr, const int64_t* sd, int unit, int other) {
+    return reinterpret_cast<uintptr_t>(ptr) % 16 == 0 && sd[unit] == 1 && ((sd[0] | sd[1] | sd[other]) & 3) == 0;
+  };
+  f32x4 S[NK];
+  if (p.h0 == nullptr) {
+#pragma unroll
+    for (int r = 0; r < NK; ++r) S[r] = f32x4{0.f, 0.f, 0.f, 0.f};
+  } else {
+    const float* const src = p.h0 + bi * p.sh0[0] + hi * p.sh0[1] + k0 * p.sh0[2] + c0 * p.sh0[3];
+    if (piece(p.h0, p.sh0, 3, 2)) {
+#pragma unroll
+      for (int r = 0; r < NK; ++r) S[r] = *reinterpret_cast<const f32x4*>(src + r * p.sh0[2]);
+    } else {
+#pragma unroll
+      for (int r = 0; r < NK; ++r)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) S[r][i] = src[r * p.sh0[2] + i * p.sh0[3]];
+    }
+  }
+  typedef uint32_t kw __attribute__((ext_vector_type(NK / 2)));
+  typedef uint32_t vw __attribute__((ext_vector_type(2)));
+  struct Row {
+    kw q, k;
+    vw v;
+    float g, beta;
+  } x[NT];
+  const TIn* const qp = static_cast<const TIn*>(p.q) + head_base(rs, hi, p.sq) + k0;
+  const TIn* const kp = static_cast<const TIn*>(p.k) + head_base(rs, hi, p.sk) + k0;
+  const TIn* const vp = static_cast<const TIn*>(p.v) + head_base(rs, hi, p.sv) + c0;
+  const int64_t gb = head_base(rs, hi, p.sg), bb = head_base(rs, hi, p.sb);
+  const int64_t ob = head_base(rs, hi, p.so) + c0;
+  auto f = [](uint32_t w, int e) __attribute__((always_inline)) {
+    const uint16_t h = (uint16_t)(e ? w >> 16 : w & 0xffffu);
+    if constexpr (std::is_same<TIn, f16>::value) return (float)__builtin_bit_cast(f16, h);
+    else return bf16_bits_to_float(h);
+  };
+  // over the lanes of equal lane % 4
+  auto sum = [](float a) __attribute__((always_inline)) {
+    auto ror = [](float b, auto ctrl) {
+      return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(b), decltype(ctrl)::value, 0xf, 0xf, false));
+    };
+    a += ror(a, std::integral_constant<int, 0x128>{});
+    a += ror(a, std::integral_constant<int, 0x124>{});
+    const auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(a), false, false);
+    a = __uint_as_float(b[0]) + __uint_as_float(b[1]);
+    const auto c = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(a), false, false);
+    return __uint_as_float(c[0]) + __uint_as_float(c[1]);
+  };
+  for (int t0 = 0; t0 < rs.T; t0 += NT) {
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+      const int64_t t = t0 + j;
+      if (t < rs.T) {
+        x[j].q = *reinterpret_cast<const kw*>(qp + t * p.sq[1]);
+        x[j].k = *reinterpret_cast<const kw*>(kp + t * p.sk[1]);
+        x[j].v = *reinterpret_cast<const vw*>(vp + t * p.sv[1]);
+        x[j].g = load_scalar(p.g, gb + t * p.sg[1], p.g_dtype);
+        x[j].beta = load_scalar(p.beta, bb + t * p.sb[1], p.beta_dtype);
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+      const int64_t t = t0 + j;
+      if (t < rs.T) {
+        float kf[NK], qf[NK], ks[4] = {0.f, 0.f, 0.f, 0.f}, qs[4] = {0.f, 0.f, 0.f, 0.f}, qk = 0.f;
+#pragma unroll
+        for (int r = 0; r < NK; ++r) {
+          kf[r] = f(x[j].k[r / 2], r & 1);
+          qf[r] = f(x[j].q[r / 2], r & 1);
+          qk = __builtin_fmaf(qf[r], kf[r], qk);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            ks[i] = __builtin_fmaf(kf[r], S[r][i], ks[i]);
+            qs[i] = __builtin_fmaf(qf[r], S[r][i], qs[i]);
+          }
+        }
+        qk = sum(qk);
+        const float e = expf(x[j].g);
+        float u[4], o[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          u[i] = x[j].beta * __builtin_fmaf(-e, sum(ks[i]), f(x[j].v[i / 2], i & 1));
+          o[i] = p.scale * __builtin_fmaf(qk, u[i], e * sum(qs[i]));
+        }
+#pragma unroll
+        for (int r = 0; r < NK; ++r)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) S[r][i] = __builtin_fmaf(kf[r], u[i], e * S[r][i]);
+        if (rg == 0) {
+          const int64_t at = ob + t * p.so[1];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) store_scalar(p.o, at + i, p.o_dtype, o[i]);
+        }
+      }
+    }
+  }
+  float* const dst = p.fs + bi * p.sfs[0] + hi * p.sfs[1] + k0 * p.sfs[2] + c0 * p.sfs[3];
+  if (piece(p.fs, p.sfs, 3, 2)) {
+#pragma unroll
+    for (int r = 0; r < NK; ++r) *reinterpret_cast<f32x4*>(dst + r * p.sfs[2]) = S[r];
+  } else if (piece(p.fs, p.sfs, 2, 3)) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int r = 0; r < NK; r += 4)
+        *reinterpret_cast<f32x4*>(dst + i * p.sfs[3] + r) = f32x4{S[r][i], S[r + 1][i], S[r + 2][i], S[r + 3][i]};
+  } else {
+#pragma unroll
+    for (int r = 0; r < NK; ++r)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) dst[r * p.sfs[2] + i * p.sfs[3]] = S[r][i];
+  }
+}
+
+// Workgroup blk of the short sequences: one wave per (sequence, head, 16
+// columns); a sequence of other lengths has nothing to do here.
+template <typename TIn, int K, int NT>
+__device__ __forceinline__ void short_job(const SArgs& p, int blk) {
+  const int nv = p.V / 16;
+  const int64_t unit = (int64_t)blk * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (unit >= (int64_t)p.B * p.H * nv) return;
+  const int vs = (int)(unit % nv), bh = (int)(unit / nv);
+  const RowSpan rs = row_span(p.cu, p.T, bh / p.H);
+  if (rs.T > 0 && rs.T <= kShortRows) short_walk<TIn, K, NT>(p, rs, bh / p.H, bh % p.H, 16 * vs);
+}
+inline int short_blocks(const SArgs& a) { return (int)(((int64_t)a.B * a.H * (a.V / 16) + 3) / 4); }
+
 // Record job r of a segment -> (sequence bi, head hi, its rows, chunk c0 + lc);
 // the record is number (bi H + hi) L + lc.  A dense batch has one job per
 // record.  Packed sequences have one per chunk slot and head (the B sequences
 // share ceil(T / C) + B slots, far fewer than B L): false where the slot's
 // chunk is not of this segment.
+template <bool PACKED>
 __device__ __forceinline__ bool rec_coords(const SArgs& p, int r, RowSpan& rs, int& bi, int& hi, int& lc) {
-  if (p.cu == nullptr) {
+  if constexpr (!PACKED) {
     lc = r % p.L;
     const int bh = r / p.L;
     hi = bh % p.H;
@@ -244,12 +400,15 @@ __device__ __forceinline__ bool rec_coords(const SArgs& p, int r, RowSpan& rs, i
   }
   hi = r % p.H;
   int cc;
-  if (!slot_chunk<C>(p, r / p.H, rs, cc, bi)) return false;
+  if (!slot_chunk<C>(p, r / p.H, rs, cc, bi) || rs.T <= kShortRows) return false;
   lc = cc - p.c0;
   return lc >= 0 && lc < p.L;
 }
 
-template <typename TIn, int K>
+// PACKED: cu_seqlens given (an instance of its own: a dense call's records are
+// bound by their latency, 9.6 us at 1024 of them, and packed geometry in the
+// same kernel cost them 0.7 us).
+template <typename TIn, int K, bool PACKED>
 __global__ __launch_bounds__(256) void rec32_kernel(const SArgs p) {
   constexpr int KB = K / 32;
   constexpr uint32_t EB = sizeof(TIn);
@@ -257,6 +416,13 @@ __global__ __launch_bounds__(256) void rec32_kernel(const SArgs p) {
   __shared__ __attribute__((aligned(16))) float s_at[4][2][C * C];
   __shared__ __attribute__((aligned(16))) float s_beta[4][2][C];
   __shared__ __attribute__((aligned(16))) float s_b[4][2][C];
+
+  if constexpr (PACKED) {
+    // the workgroups past the records walk the short sequences (a row at a
+    // time: more would cost the records a wave per SIMD in registers)
+    const int nblk = (p.nrec + 7) / 8;
+    if ((int)blockIdx.x >= nblk) return short_job<TIn, K, 1>(p, blockIdx.x - nblk);
+  }
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -269,7 +435,8 @@ __global__ __launch_bounds__(256) void rec32_kernel(const SArgs p) {
   const char* kh[2];
   char* rp[2];
   uint32_t skb[2];
-  int64_t gof[2], bof[2];
+  RowSpan rs[2] = {};
+  int hh[2], tt[2];
 #pragma unroll
   for (int e = 0; e < 2; ++e) {
     const int r = (blockIdx.x * 4 + wave) * 2 + e;
@@ -277,17 +444,14 @@ __global__ __launch_bounds__(256) void rec32_kernel(const SArgs p) {
     kh[e] = nullptr;
     rp[e] = nullptr;
     skb[e] = 0;
-    gof[e] = bof[e] = 0;
-    RowSpan rs;
-    int bi, hi, lc;
-    if (r < p.nrec && rec_coords(p, r, rs, bi, hi, lc)) {
-      const int t0 = (p.c0 + lc) * C;
-      nval[e] = min(C, rs.T - t0);
-      kh[e] = static_cast<const char*>(p.k) + (head_base(rs, hi, p.sk) + (int64_t)t0 * p.sk[1]) * EB;
+    hh[e] = tt[e] = 0;
+    int bi, lc;
+    if (r < p.nrec && rec_coords<PACKED>(p, r, rs[e], bi, hh[e], lc)) {
+      tt[e] = (p.c0 + lc) * C;
+      nval[e] = min(C, rs[e].T - tt[e]);
+      kh[e] = static_cast<const char*>(p.k) + (head_base(rs[e], hh[e], p.sk) + (int64_t)tt[e] * p.sk[1]) * EB;
       skb[e] = (uint32_t)p.sk[1] * EB;
-      rp[e] = p.rec + ((int64_t)(bi * p.H + hi) * p.L + lc) * rec_stride<TIn, K>();
-      gof[e] = head_base(rs, hi, p.sg) + (int64_t)t0 * p.sg[1];
-      bof[e] = head_base(rs, hi, p.sb) + (int64_t)t0 * p.sb[1];
+      rp[e] = p.rec + ((int64_t)(bi * p.H + hh[e]) * p.L + lc) * rec_stride<TIn, K>();
     }
   }
   // k rows (rows past the end re-read the last row: finite values whose
@@ -307,8 +471,11 @@ __global__ __launch_bounds__(256) void rec32_kernel(const SArgs p) {
   }
   float gv = 0.f, bv = 0.f;
   if (c < (half ? nval[1] : nval[0])) {
-    gv = load_scalar(p.g, (half ? gof[1] : gof[0]) + (int64_t)c * p.sg[1], p.g_dtype);
-    bv = load_scalar(p.beta, (half ? bof[1] : bof[0]) + (int64_t)c * p.sb[1], p.beta_dtype);
+    const int64_t t = c + (half ? tt[1] : tt[0]);
+    gv = load_scalar(p.g, (half ? head_base(rs[1], hh[1], p.sg) : head_base(rs[0], hh[0], p.sg)) + t * p.sg[1],
+                     p.g_dtype);
+    bv = load_scalar(p.beta, (half ? head_base(rs[1], hh[1], p.sb) : head_base(rs[0], hh[0], p.sb)) + t * p.sb[1],
+                     p.beta_dtype);
   }
   // gates (lanes 0-31: record 0, lanes 32-63: record 1)
   const float b = scan32(gv);
@@ -551,6 +718,14 @@ constexpr int dma_per_chunk() {
   return 2 * (C * K * 2 / 1024) + (C * BV * 2 + 1023) / 1024 + REC_BYTES / 1024;
 }
 
+// A dense batch of short sequences, four waves to a workgroup, no records.
+// Bound by the state's one trip in and out (256 heads, one row: 33.8 MB in
+// 10.0 us, 3.4 TB/s).
+template <typename TIn, int K>
+__global__ __launch_bounds__(256) void short32_kernel(const SArgs p) {
+  short_job<TIn, K, kShortRows>(p, blockIdx.x);
+}
+
 template <typename TIn, int K, int BV, bool SPLIT>
 __global__ __launch_bounds__((64 * scan_waves<BV, SPLIT>())) void scan32_kernel(const SArgs p) {
   using M = Mma<f16>;
@@ -599,6 +774,7 @@ __global__ __launch_bounds__((64 * scan_waves<BV, SPLIT>())) void scan32_kernel(
   const int nch_all = (T + C - 1) / C;
   const int nloc = max(0, min(p.L, nch_all - p.c0));  // chunks of this segment
   if (nloc == 0 && !p.first) return;                  // state unchanged
+  if (T > 0 && T <= kShortRows) return;               // walked by rec32_kernel's launch
   const f32x4 z4 = {0.f, 0.f, 0.f, 0.f};
 
   constexpr uint32_t EB = sizeof(TIn);
@@ -1236,7 +1412,15 @@ __global__ __launch_bounds__((64 * scan_waves<BV, SPLIT>())) void scan32_kernel(
 template <typename TIn, int K, int BV>
 int launch_kb(const SArgs& a, int units, hipStream_t s) {
   static_assert(sizeof(ScanSmem<K, BV>) <= kLdsLimit, "LDS budget");
-  if (a.nrec > 0) hipLaunchKernelGGL((rec32_kernel<TIn, K>), dim3((a.nrec + 7) / 8), dim3(256), 0, s, a);
+  if (a.cu == nullptr && a.T > 0 && a.T <= kShortRows) {
+    hipLaunchKernelGGL((short32_kernel<TIn, K>), dim3(short_blocks(a)), dim3(256), 0, s, a);
+    return (int)hipGetLastError();
+  }
+  if (a.nrec > 0) {
+    const dim3 grid((a.nrec + 7) / 8 + (a.cu != nullptr && a.first ? short_blocks(a) : 0));
+    if (a.cu != nullptr) hipLaunchKernelGGL((rec32_kernel<TIn, K, true>), grid, dim3(256), 0, s, a);
+    else hipLaunchKernelGGL((rec32_kernel<TIn, K, false>), grid, dim3(256), 0, s, a);
+  }
   if constexpr (scan_split_ok<TIn, K, BV>()) {
     if (a.L <= kSplitChunks) {
       hipLaunchKernelGGL((scan32_kernel<TIn, K, BV, true>), dim3(units), dim3(64 * scan_waves<BV, true>()), 0, s, a);
