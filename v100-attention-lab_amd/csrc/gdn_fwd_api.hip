@@ -184,6 +184,8 @@ static int launch_impl(const GdnFwdParams& P, hipStream_t s, int64_t scratch_byt
   a.xcd_remap = (units % 8 == 0) ? 1 : 0;
   a.cu = P.cu_seqlens;
 
+  if (!(P.flags & GDN_FLAG_PHASED_KERNEL) && f32_batch_runs(P) && pipe_offsets_fit(P))
+    return launch_f32_batch(a, P.K, s);
   const int grid = (int)units;
   if (!(P.flags & GDN_FLAG_PHASED_KERNEL) && pipe_supported(P.qkv_dtype, P.K, P.chunk_size, bv) &&
       pipe_offsets_fit(P)) {

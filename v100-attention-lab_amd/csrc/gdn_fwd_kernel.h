@@ -976,6 +976,10 @@ inline bool pipe_supported(int dtype, int K, int C, int BV) {
 }
 int launch_pipe_f16(const KArgs& a, int K, int bv, int grid, hipStream_t s);
 int launch_pipe_bf16(const KArgs& a, int K, int bv, int grid, hipStream_t s);
+// fp32 inputs with 32-row chunks and K in {64, 128} run in one launch of
+// batched chunks (gdn_fwd_f32_batch.hip).
+bool f32_batch_runs(const GdnFwdParams& P);
+int launch_f32_batch(KArgs a, int K, hipStream_t s);
 // 64-row chunks with K in {32, 64, 128} run as two launches (gdn_fwd_c64.hip)
 // over a caller-owned workspace of per-chunk records.
 bool c64_supported(int K, int C, int V);
