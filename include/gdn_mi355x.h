@@ -137,9 +137,12 @@ typedef struct GdnFwdParams {
  *     sequence (at least one), so any workspace of at least
  *     gdn_fwd_workspace_size() bytes runs the call; a longer sequence runs
  *     as several segments, its state passing through final_state in fp32.
- *     C = 64 needs params->workspace.
- *   - C = 32 without a workspace (or GDN_FLAG_FUSED_KERNEL), or K = 256 /
- *     GDN_FLAG_PHASED_KERNEL: one fused kernel, no workspace.
+ *     C = 64 needs params->workspace.  At C = 32 sequences of at most 4 rows
+ *     are walked step by step in fp32 (a dense batch of them in one launch,
+ *     with or without a workspace).
+ *   - C = 32 without a workspace (or GDN_FLAG_FUSED_KERNEL), fp32 inputs at
+ *     C = 32, or K = 256 / GDN_FLAG_PHASED_KERNEL: one fused kernel, no
+ *     workspace.
  * The state stays on chip in every path: no chunk state is written. */
 int gdn_fwd_launch(const GdnFwdParams* params, void* stream);
 

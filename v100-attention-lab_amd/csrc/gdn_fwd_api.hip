@@ -128,7 +128,7 @@ static int launch_impl(const GdnFwdParams& P, hipStream_t s, int64_t scratch_byt
   }
   const long long units = (long long)P.B * P.H * (P.V / bv);
   if (units > 0x7fffffffLL) return GDN_ERR_BAD_SHAPE;
-  bool scan32 = uses_scan32(P, bv) && (scratch_bytes > 0 || P.workspace != nullptr);
+  bool scan32 = uses_scan32(P, bv) && (scratch_bytes > 0 || P.workspace != nullptr || scan32_short(P));
   if (scratch_bytes > 0 && P.T > 0) {
     // The static scratch must hold one chunk's records per sequence and
     // head (longer sequences run in segments).  Where it cannot, the call
@@ -165,7 +165,7 @@ static int launch_impl(const GdnFwdParams& P, hipStream_t s, int64_t scratch_byt
   if (scan32) {
     // segment length: as many chunks per sequence as the workspace holds
     const int64_t per_chunk = (int64_t)P.B * P.H * scan32_record_bytes(P.qkv_dtype, P.K);
-    const int64_t L = W.workspace_bytes / per_chunk;
+    const int64_t L = W.workspace == nullptr ? 1 : W.workspace_bytes / per_chunk;  // none: short sequences
     if (P.T > 0 && (reinterpret_cast<uintptr_t>(W.workspace) % 256 != 0 || L < 1)) return GDN_ERR_WORKSPACE;
     return scan32_launch(W, bv, (int)(L < 1 ? 1 : L < 0x7fffffff ? L : 0x7fffffff), s);
   }
@@ -237,7 +237,7 @@ int64_t gdn_fwd_workspace_size(const GdnFwdParams* prm) {
   if (!valid_dtype(P.qkv_dtype)) return -1;
   if (uses_c64(P)) return c64_workspace_size(P.B, P.T, P.H, P.K, P.cu_seqlens ? P.B : 0, P.qkv_dtype);
   const int bv = P.block_v ? P.block_v : auto_block_v(P.B, P.H, P.K, P.V, P.chunk_size, P.qkv_dtype);
-  if (bv > 0 && P.V % bv == 0 && uses_scan32(P, bv)) {
+  if (bv > 0 && P.V % bv == 0 && uses_scan32(P, bv) && !scan32_short(P)) {
     const int64_t nch = (P.T + 31) / 32;
     const int64_t L = nch < kSegChunks ? nch : kSegChunks;
     const int64_t bytes = (int64_t)P.B * P.H * L * scan32_record_bytes(P.qkv_dtype, P.K);

@@ -994,6 +994,7 @@ int c64_launch(const GdnFwdParams& P, int seg_chunks, hipStream_t stream);
 // chunks per sequence whose records fit the caller's workspace.
 bool scan32_supported(int dtype, int K, int C, int BV, int V);
 int64_t scan32_record_bytes(int dtype, int K);  // per (chunk, head)
+bool scan32_short(const GdnFwdParams& P);       // a dense batch walked step by step: no records
 int scan32_launch(const GdnFwdParams& P, int bv, int seg_chunks, hipStream_t stream);
 
 }  // namespace gdn

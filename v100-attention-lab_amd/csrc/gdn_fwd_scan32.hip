@@ -1447,6 +1447,10 @@ bool scan32_supported(int dtype, int K, int C, int BV, int V) {
          (BV == 16 || BV == 32);
 }
 
+bool scan32_short(const GdnFwdParams& P) {
+  return P.cu_seqlens == nullptr && P.T > 0 && P.T <= s32::kShortRows;
+}
+
 int64_t scan32_record_bytes(int dtype, int K) {
   if (dtype != GDN_DTYPE_BF16) return s32::REC_BYTES;
   return K == 64 ? s32::rec_stride<bf16_t, 64>() : s32::rec_stride<bf16_t, 128>();

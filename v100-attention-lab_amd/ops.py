@@ -121,6 +121,21 @@ _PLANS = {}
 _PLANS_MAX = 256
 
 
+# Raw HIP stream of a device's current torch stream, and the current device,
+# without building the Python objects around them (about 1 us a call each).
+def _raw_stream(index):
+    return torch._C._cuda_getCurrentRawStream(index)
+
+
+def _launch(fn, P, dev):
+    """fn(&P, current stream of dev) with dev current."""
+    index = dev.index
+    if index is None or index != torch._C._cuda_getDevice():
+        with torch.cuda.device(dev):
+            return fn(ctypes.byref(P), _raw_stream(torch.cuda.current_device()))
+    return fn(ctypes.byref(P), _raw_stream(index))
+
+
 class _Plan:
     __slots__ = ("shape_o", "shape_fs", "out_dtype", "fs_vk", "o_hf", "params", "ws_bytes")
 
@@ -250,12 +265,7 @@ def _run(q, k, v, g, beta, h0, scale, chunk_size, block_v, output_dtype, kernel,
     if plan.ws_bytes > 0:
         ws = torch.empty(plan.ws_bytes, dtype=torch.uint8, device=dev)
         P.workspace, P.workspace_bytes = ws.data_ptr(), plan.ws_bytes
-    lib = _lib.load_library()
-    if dev.index == torch.cuda.current_device():
-        status = lib.gdn_fwd_launch(ctypes.byref(P), torch.cuda.current_stream(dev).cuda_stream)
-    else:
-        with torch.cuda.device(dev):
-            status = lib.gdn_fwd_launch(ctypes.byref(P), torch.cuda.current_stream(dev).cuda_stream)
+    status = _launch(_lib.load_library().gdn_fwd_launch, P, dev)
     if status != 0:
         raise RuntimeError(f"gdn_fwd_launch failed ({status}): {_lib.status_string(status)}")
     return o, fs
@@ -454,12 +464,7 @@ def gdn_prep(q: Optional[torch.Tensor] = None, k: Optional[torch.Tensor] = None,
         if t is not None:
             setattr(P, f"{name}_in", t.data_ptr())
             setattr(P, f"{name}_out", o.data_ptr())
-    lib = _lib.load_library()
-    if dev.index == torch.cuda.current_device():
-        status = lib.gdn_prep_launch(ctypes.byref(P), torch.cuda.current_stream(dev).cuda_stream)
-    else:
-        with torch.cuda.device(dev):
-            status = lib.gdn_prep_launch(ctypes.byref(P), torch.cuda.current_stream(dev).cuda_stream)
+    status = _launch(_lib.load_library().gdn_prep_launch, P, dev)
     if status != 0:
         raise RuntimeError(f"gdn_prep_launch failed ({status}): {_lib.status_string(status)}")
     return outs
@@ -555,6 +560,15 @@ def gdn_bwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Tensor,
     n_seq = None
     if cu_seqlens is not None:
         cu_seqlens, n_seq = _check_cu_seqlens(cu_seqlens, q.shape[1], q.device)
+    return _run_bwd(q, k, v, g, beta, h0, do, dfinal, scale, cu_seqlens, n_seq, need_dh0, max_segment_chunks)
+
+
+# Launch plans of the backward, as _PLANS: the validated, prefilled parameter
+# block and the workspace size of a signature.
+_BWD_PLANS = {}
+
+
+def _make_bwd_plan(q, k, v, g, beta, h0, do, dfinal, scale, n_seq, need_dh0, max_segment_chunks):
     B, T, H, K, V = _validate(q, k, v, g, beta, h0, 32, None, n_seq, check_device=False)
     if K not in BWD_SUPPORTED_K:
         raise ValueError(f"K={K} not supported by the backward (K in {BWD_SUPPORTED_K})")
@@ -565,41 +579,31 @@ def gdn_bwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Tensor,
         if tuple(dfinal.shape) != (B, H, K, V) or dfinal.dtype != torch.float32:
             raise ValueError(f"dfinal must be float32 [{B}, {H}, {K}, {V}]")
     _check_devices(q, k, v, g, beta, h0, do, dfinal)
-    # The kernels index dO rows by their (b, t, h) strides with a unit step
-    # along V.  autograd may hand over any layout, e.g. the stride-0 expansion
-    # of a scalar for o.sum().backward(): give the kernels a dense copy then.
-    if do.stride(-1) != 1:
-        do = do.contiguous()
-    dev = q.device
-    lib = _lib.load_library()
-    dq = torch.empty(q.shape, dtype=q.dtype, device=dev)
-    dk = torch.empty(k.shape, dtype=k.dtype, device=dev)
-    dv = torch.empty(v.shape, dtype=v.dtype, device=dev)
-    dg = torch.empty(g.shape, dtype=g.dtype, device=dev)
-    dbeta = torch.empty(beta.shape, dtype=beta.dtype, device=dev)
-    dh0 = torch.empty(B, H, K, V, dtype=torch.float32, device=dev) if need_dh0 else None
     P = _lib.GdnBwdParams()
-    P.q, P.k, P.v, P.g, P.beta = q.data_ptr(), k.data_ptr(), v.data_ptr(), g.data_ptr(), beta.data_ptr()
-    P.h0 = h0.data_ptr() if h0 is not None else None
-    P.d_o = do.data_ptr()
-    P.d_final_state = dfinal.data_ptr() if dfinal is not None else None
-    P.dq, P.dk, P.dv, P.dg, P.dbeta = dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), dg.data_ptr(), dbeta.data_ptr()
-    P.dh0 = dh0.data_ptr() if dh0 is not None else None
-    for name, t in (("q", q), ("k", k), ("v", v), ("do", do), ("dq", dq), ("dk", dk), ("dv", dv)):
+    P.d_o = do.data_ptr() & 15 or 16     # the size depends on dO's alignment
+    for name, t in (("q", q), ("k", k), ("v", v), ("do", do)):
         getattr(P, f"{name}_stride")[:] = t.stride()[:3]
-    for name, t in (("g", g), ("beta", beta), ("dg", dg), ("dbeta", dbeta)):
+    for name, t in (("g", g), ("beta", beta)):
         getattr(P, f"{name}_stride")[:] = t.stride()
+    # the gradients: new contiguous tensors
+    shapes = {"dq": q.shape, "dk": k.shape, "dv": v.shape, "dg": g.shape, "dbeta": beta.shape}
+    for name, shape in shapes.items():
+        strides = [1] * len(shape)
+        for i in range(len(shape) - 2, -1, -1):
+            strides[i] = strides[i + 1] * max(shape[i + 1], 1)
+        getattr(P, f"{name}_stride")[:] = strides[:3]
     P.h0_stride[:] = h0.stride() if h0 is not None else (0, 0, 0, 0)
     P.dfs_stride[:] = dfinal.stride() if dfinal is not None else (0, 0, 0, 0)
-    P.dh0_stride[:] = dh0.stride() if dh0 is not None else (0, 0, 0, 0)
+    P.dh0_stride[:] = (H * K * V, K * V, V, 1) if need_dh0 else (0, 0, 0, 0)
     P.B, P.T, P.H, P.K, P.V = B, T, H, K, V
     P.scale = float(scale)
     P.qkv_dtype = _DTYPE_CODE[q.dtype]
     P.g_dtype = _DTYPE_CODE[g.dtype]
     P.beta_dtype = _DTYPE_CODE[beta.dtype]
     P.do_dtype = _DTYPE_CODE[do.dtype]
-    P.cu_seqlens = cu_seqlens.data_ptr() if cu_seqlens is not None else None
+    P.cu_seqlens = 1 if n_seq is not None else None
     # the workspace this call's path takes (the 16-bit walks need less)
+    lib = _lib.load_library()
     if max_segment_chunks is None:
         ws_bytes = lib.gdn_bwd_workspace_size_params(ctypes.byref(P))
     else:
@@ -608,10 +612,53 @@ def gdn_bwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Tensor,
         ws_bytes = lib.gdn_bwd_segment_workspace_size(ctypes.byref(P), int(max_segment_chunks))
     if ws_bytes < 0:
         raise ValueError(f"backward does not support B={B} T={T} H={H} K={K} V={V}")
-    ws = torch.empty(max(ws_bytes, 256), dtype=torch.uint8, device=dev)
-    P.workspace, P.workspace_bytes = ws.data_ptr(), ws.numel()
-    with torch.cuda.device(dev):
-        status = lib.gdn_bwd_launch(ctypes.byref(P), torch.cuda.current_stream(dev).cuda_stream)
+    P.cu_seqlens = None
+    return bytes(P), max(ws_bytes, 256), (B, H, K, V) if need_dh0 else None
+
+
+def _run_bwd(q, k, v, g, beta, h0, do, dfinal, scale, cu, n_seq, need_dh0, max_segment_chunks=None):
+    """gdn_bwd with cu_seqlens already checked (cu int64, n_seq sequences)."""
+    # The kernels index dO rows by their (b, t, h) strides with a unit step
+    # along V.  autograd may hand over any layout, e.g. the stride-0 expansion
+    # of a scalar for o.sum().backward(): give the kernels a dense copy then.
+    if isinstance(do, torch.Tensor) and do.dim() == 4 and do.stride(-1) != 1 and do.device.type == "cuda":
+        do = do.contiguous()
+    try:
+        key = _signature(q, k, v, g, beta, h0, scale, need_dh0, None if dfinal is None else dfinal.dtype, None,
+                         None, None, n_seq, None, max_segment_chunks)
+        key += (do.shape, do.stride(), do.dtype, do.device, do.data_ptr() & 15)
+        if dfinal is not None:
+            key += (dfinal.shape, dfinal.stride(), dfinal.device)
+        plan = _BWD_PLANS.get(key)
+    except (AttributeError, TypeError):   # not tensors: the checks say which
+        key, plan = None, None
+    if plan is None:
+        plan = _make_bwd_plan(q, k, v, g, beta, h0, do, dfinal, scale, n_seq, need_dh0, max_segment_chunks)
+        if key is not None:
+            if len(_BWD_PLANS) >= _PLANS_MAX:
+                _BWD_PLANS.clear()
+            _BWD_PLANS[key] = plan
+    params, ws_bytes, dh0_shape = plan
+    qp, kp, vp = q.data_ptr(), k.data_ptr(), v.data_ptr()
+    if q.shape[1] > 0 and (qp | kp | vp) & 15:
+        for name, t in (("q", q), ("k", k), ("v", v)):
+            _check_rows(t, name)
+    dev = q.device
+    new = torch.empty
+    dq, dk, dv = (new(t.shape, dtype=t.dtype, device=dev) for t in (q, k, v))
+    dg, dbeta = (new(t.shape, dtype=t.dtype, device=dev) for t in (g, beta))
+    dh0 = new(dh0_shape, dtype=torch.float32, device=dev) if dh0_shape is not None else None
+    ws = new(ws_bytes, dtype=torch.uint8, device=dev)
+    P = _lib.GdnBwdParams.from_buffer_copy(params)
+    P.q, P.k, P.v, P.g, P.beta = qp, kp, vp, g.data_ptr(), beta.data_ptr()
+    P.h0 = h0.data_ptr() if h0 is not None else None
+    P.d_o = do.data_ptr()
+    P.d_final_state = dfinal.data_ptr() if dfinal is not None else None
+    P.dq, P.dk, P.dv, P.dg, P.dbeta = (t.data_ptr() for t in (dq, dk, dv, dg, dbeta))
+    P.dh0 = dh0.data_ptr() if dh0 is not None else None
+    P.cu_seqlens = cu.data_ptr() if cu is not None else None
+    P.workspace, P.workspace_bytes = ws.data_ptr(), ws_bytes
+    status = _launch(_lib.load_library().gdn_bwd_launch, P, dev)
     if status != 0:
         raise RuntimeError(f"gdn_bwd_launch failed ({status}): {_lib.status_string(status)}")
     return dq, dk, dv, dg, dbeta, dh0
@@ -641,8 +688,15 @@ class _GdnFunction(torch.autograd.Function):
         if dfs_kv is not None and dfs_kv.dtype != torch.float32:
             dfs_kv = dfs_kv.float()
         need_dh0 = h0 is not None and ctx.needs_input_grad[5]
-        dq, dk, dv, dg, dbeta, dh0 = gdn_bwd(q, k, v, g, beta, h0, do_bthv, dfs_kv, ctx.scale,
-                                             cu_seqlens=cu, need_dh0=need_dh0)
+        n_seq = None
+        if cu is not None:
+            # checked by the forward (a second read of the offsets would make
+            # the host wait for the device once more)
+            n_seq = cu.numel() - 1
+            if cu.dtype != torch.int64 or not cu.is_contiguous():
+                cu = cu.to(torch.int64).contiguous()
+        dq, dk, dv, dg, dbeta, dh0 = _run_bwd(q, k, v, g, beta, h0, do_bthv, dfs_kv, ctx.scale, cu, n_seq,
+                                              need_dh0)
         return dq, dk, dv, dg, dbeta, dh0, None, None, None, None, None, None, None, None, None
 
 
