@@ -708,11 +708,31 @@ namespace w16 {
 // 3 of t swapped, so that the rows of a 32-lane pass of a transposing read
 // (t = 0..3 and 8..11, + 4 h) fill 256 contiguous bytes.
 __device__ __forceinline__ int dperm(int t) { return (t & ~12) | ((t & 4) << 1) | ((t & 8) >> 1); }
-// lane (r, kq) receives dO[8 kq + j][r], j = 0..7: row r of dO^T
-__device__ __forceinline__ f16x8 dot_frag8(const f16* x, int r, int kq) {
+// 4 elements of a 16-bit input as they are in LDS -> fp32; bf16 values times
+// sc (a power of two: exact)
+template <typename TIn>
+__device__ __forceinline__ f32x4 to_f4(const f16x4& x, float sc) {
+  f32x4 y;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const f16 e = x[i];
+    if constexpr (std::is_same<TIn, f16>::value) y[i] = (float)e;
+    else y[i] = bf16_bits_to_float(__builtin_bit_cast(uint16_t, e)) * sc;
+  }
+  return y;
+}
+// lane (r, kq) receives dO[8 kq + j][r], j = 0..7: row r of dO^T (bf16 times
+// sc), as an operand
+template <typename TIn>
+__device__ __forceinline__ f16x8 dot_frag8(const f16* x, int r, int kq, float sc) {
   const int t = 8 * kq + (r >> 2), col = 4 * (r & 3);
   const f16x4 lo = read_tr4(x + dperm(t) * BV + col), hi = read_tr4(x + dperm(t + 4) * BV + col);
-  return f16x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+  if constexpr (std::is_same<TIn, f16>::value) {
+    return f16x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+  } else {
+    const f32x4 a = to_f4<TIn>(lo, sc), b = to_f4<TIn>(hi, sc);
+    return f16x8{(f16)a[0], (f16)a[1], (f16)a[2], (f16)a[3], (f16)b[0], (f16)b[1], (f16)b[2], (f16)b[3]};
+  }
 }
 
 // Rows t0 .. t0 + C - 1 of a row-major 16-bit input (rows ld elements apart,
@@ -731,22 +751,30 @@ __device__ __forceinline__ void dma_rows(const uint16_t* src, int64_t ld, int nv
     dma16(src + min(t, nval - 1) * ld + 8 * (pc ^ swz<W>(t)), dst + 512 * j);
   }
 }
-// Once a wave's copies of dma_rows have landed: bf16 -> fp16, rows >= nval
-// -> zero, each lane on the pieces it copied itself.
-template <typename TIn, int W, int NW>
-__device__ __forceinline__ void fix_rows(f16* dst, int nval, int lw, int lane) {
+// Once a wave's copies of dma_rows have landed: rows >= nval -> zero, each
+// lane on the pieces it copied itself.
+template <int W, int NW>
+__device__ __forceinline__ void zero_rows(f16* dst, int nval, int lw, int lane) {
   constexpr int NJ = C * W / 512;
 #pragma unroll
   for (int jj = 0; jj < NJ / NW; ++jj) {
     const int pos = 512 * (NW * jj + lw) + 8 * lane;
-    f16x8* const a = reinterpret_cast<f16x8*>(dst + pos);
-    if (pos / W >= nval) {
-      *a = f16x8{};
-    } else if constexpr (!std::is_same<TIn, f16>::value) {
-      f16 x[8];
-      InTraits<TIn>::to_op(*reinterpret_cast<const uint4*>(a), x);
-      *a = f16x8{x[0], x[1], x[2], x[3], x[4], x[5], x[6], x[7]};
-    }
+    if (pos / W >= nval) *reinterpret_cast<f16x8*>(dst + pos) = f16x8{};
+  }
+}
+// 8 elements of a 16-bit input as it is in LDS -> an fp16 operand.  bf16
+// (exact in fp16's range) is converted here, between the products, by every
+// wave that reads it: 12 instructions a fragment.  Converted in LDS before the
+// barrier that publishes the tile, the two walks took 625 us against 555 (B4
+// T4096 H16 K = V = 128, bf16).
+template <typename TIn>
+__device__ __forceinline__ f16x8 op8(const f16x8& x) {
+  if constexpr (std::is_same<TIn, f16>::value) {
+    return x;
+  } else {
+    f16 y[8];
+    InTraits<TIn>::to_op(__builtin_bit_cast(uint4, x), y);
+    return f16x8{y[0], y[1], y[2], y[3], y[4], y[5], y[6], y[7]};
   }
 }
 
@@ -762,21 +790,13 @@ __device__ __forceinline__ void dma_dot(const uint16_t* src, int64_t ld, int nva
     dma4(src + min(dperm(pos / BV), nval - 1) * ld + pos % BV, dst + 128 * j);
   }
 }
-// bf16 values times sc (a power of two: exact) -> fp16, rows >= nval -> zero
-template <typename TIn>
-__device__ __forceinline__ void fix_dot(f16* dst, int nval, float sc, int lw, int lane) {
+// rows >= nval -> zero
+__device__ __forceinline__ void zero_dot(f16* dst, int nval, int lw, int lane) {
   constexpr int NJ = C * BV / 128;
 #pragma unroll
   for (int jj = 0; jj < NJ / 2; ++jj) {
     const int pos = 128 * (2 * jj + lw) + 2 * lane;
-    uint32_t* const a = reinterpret_cast<uint32_t*>(dst + pos);
-    if (dperm(pos / BV) >= nval) {
-      *a = 0u;
-    } else if constexpr (!std::is_same<TIn, f16>::value) {
-      const uint32_t w = *a;
-      const f16 lo = (f16)(bf16_bits_to_float(w & 0xffffu) * sc), hi = (f16)(bf16_bits_to_float(w >> 16) * sc);
-      *a = (uint32_t)__builtin_bit_cast(uint16_t, lo) | ((uint32_t)__builtin_bit_cast(uint16_t, hi) << 16);
-    }
+    if (dperm(pos / BV) >= nval) *reinterpret_cast<uint32_t*>(dst + pos) = 0u;
   }
 }
 
@@ -787,17 +807,9 @@ __device__ __forceinline__ void dma_v(const uint16_t* src, int64_t ld, int nval,
   const int pos = 8 * lane;
   dma16(src + min(pos / BV, nval - 1) * ld + pos % BV, dst);
 }
-template <typename TIn>
-__device__ __forceinline__ void fix_v(f16* dst, int nval, float sc, int lane) {
+__device__ __forceinline__ void zero_v(f16* dst, int nval, int lane) {
   const int pos = 8 * lane;
-  f16x8* const a = reinterpret_cast<f16x8*>(dst + pos);
-  if (pos / BV >= nval) {
-    *a = f16x8{};
-  } else if constexpr (!std::is_same<TIn, f16>::value) {
-    f16 x[8];
-    InTraits<TIn>::to_op_sc(*reinterpret_cast<const uint4*>(a), x, sc);
-    *a = f16x8{x[0], x[1], x[2], x[3], x[4], x[5], x[6], x[7]};
-  }
+  if (pos / BV >= nval) *reinterpret_cast<f16x8*>(dst + pos) = f16x8{};
 }
 
 // A chunk's inputs of the forward walk in LDS.
@@ -931,9 +943,9 @@ __device__ __forceinline__ void walk_forward16(const BArgs& p, FMem<K>& s, const
   auto settle = [&](int cn, int b) __attribute__((always_inline)) {
     wait_dma();
     const int nval = min(C, rs.T - cn * C);
-    if (!std::is_same<TIn, f16>::value || nval < C) {
-      fix_rows<TIn, K, 1>(s.in[b].k, nval, 0, lane);
-      fix_v<TIn>(s.in[b].v, nval, rsc.v, lane);
+    if (nval < C) {
+      zero_rows<K, 1>(s.in[b].k, nval, 0, lane);
+      zero_v(s.in[b].v, nval, lane);
     }
   };
   State<K> S;
@@ -956,15 +968,15 @@ __device__ __forceinline__ void walk_forward16(const BArgs& p, FMem<K>& s, const
       f32x4 ak = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int kb = 0; kb < K; kb += 32) {
-        const f16x8 kf = frag8_s<K>(in.k, um0 + r, kb + 8 * kq);
+        const f16x8 kf = op8<TIn>(frag8_s<K>(in.k, um0 + r, kb + 8 * kq));
         ak = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, frag8(&s.sh[r][kb + 8 * kq]), ak, 0, 0, 0);
         ak = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, frag8(&s.sl[r][kb + 8 * kq]), ak, 0, 0, 0);
       }
       const int t = um0 + 4 * kq;
-      const f16x4 vv = frag4_t(reinterpret_cast<const f16 (*)[BV]>(in.v), um0, 0, r, kq);
+      const f32x4 vv = to_f4<TIn>(frag4_t(reinterpret_cast<const f16 (*)[BV]>(in.v), um0, 0, r, kq), rsc.v);
       float y[4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) y[i] = in.gv[3][t + i] * ((float)vv[i] - in.gv[1][t + i] * ak[i]);
+      for (int i = 0; i < 4; ++i) y[i] = in.gv[3][t + i] * (vv[i] - in.gv[1][t + i] * ak[i]);
       store_pair4(&s.yh[r][t], &s.yl[r][t], y);
     } else if (issuer && c + 2 < nch) {
       fetch(c + 2, b2);
@@ -995,7 +1007,7 @@ __device__ __forceinline__ void walk_forward16(const BArgs& p, FMem<K>& s, const
     for (int j = 0; j < State<K>::NST; ++j) {
       const int m0 = 16 * (wave + 4 * j);
       if (m0 < K) {
-        const f16x8 kt = frag8_ts<K>(in.k, 0, m0, r, kq);
+        const f16x8 kt = op8<TIn>(frag8_ts<K>(in.k, 0, m0, r, kq));
         f32x4 a = {0.f, 0.f, 0.f, 0.f};
         a = __builtin_amdgcn_mfma_f32_16x16x32_f16(kt, frag8(&s.dh[r][8 * kq]), a, 0, 0, 0);
         a = __builtin_amdgcn_mfma_f32_16x16x32_f16(kt, frag8(&s.dl[r][8 * kq]), a, 0, 0, 0);
@@ -1072,13 +1084,13 @@ __device__ __forceinline__ void walk_backward16(const BArgs& p, RMem<K>& s, cons
   auto settle = [&](int cn) __attribute__((always_inline)) {
     wait_dma();
     const int nval = min(C, rs.T - cn * C);
-    if (!std::is_same<TIn, f16>::value || nval < C) {
+    if (nval < C) {
       RIn<K>& d = s.in[cn & 1];
       if (!loader) {
-        fix_rows<TIn, K, 2>(d.q, nval, wave, lane);
+        zero_rows<K, 2>(d.q, nval, wave, lane);
       } else {
-        fix_rows<TIn, K, 2>(d.k, nval, lw, lane);
-        fix_dot<TIn>(d.dot, nval, rsd.v, lw, lane);
+        zero_rows<K, 2>(d.k, nval, lw, lane);
+        zero_dot(d.dot, nval, lw, lane);
       }
     }
   };
@@ -1104,12 +1116,12 @@ __device__ __forceinline__ void walk_backward16(const BArgs& p, RMem<K>& s, cons
       // du = scale P^T dO + diag(D) K dS', rows 16 w ..
       const int um0 = 16 * wave;
       f32x4 a1 = {0.f, 0.f, 0.f, 0.f}, a2 = {0.f, 0.f, 0.f, 0.f};
-      const f16x8 df = dot_frag8(in.dot, r, kq);
+      const f16x8 df = dot_frag8<TIn>(in.dot, r, kq, rsd.v);
       a1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(frag8_ts<C>(in.ph, 0, um0, r, kq), df, a1, 0, 0, 0);
       a1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(frag8_ts<C>(in.pl, 0, um0, r, kq), df, a1, 0, 0, 0);
 #pragma unroll
       for (int kb = 0; kb < K; kb += 32) {
-        const f16x8 kf = frag8_s<K>(in.k, um0 + r, kb + 8 * kq);
+        const f16x8 kf = op8<TIn>(frag8_s<K>(in.k, um0 + r, kb + 8 * kq));
         a2 = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, frag8(&s.sh[r][kb + 8 * kq]), a2, 0, 0, 0);
         a2 = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, frag8(&s.sl[r][kb + 8 * kq]), a2, 0, 0, 0);
       }
@@ -1127,9 +1139,9 @@ __device__ __forceinline__ void walk_backward16(const BArgs& p, RMem<K>& s, cons
       // (diag(gam) dO)^T as pairs: lane (r, kq) of loader wave lw -> column
       // r, rows t4 .. t4 + 3 (a 32-lane pass reads rows 0..3, 8..11 + 16 lw)
       const int t4 = 16 * lw + ((kq & 1) << 3) + ((kq & 2) << 1);
-      const f16x4 dv = read_tr4(in.dot + dperm(t4 + (r >> 2)) * BV + 4 * (r & 3));
-      const float x[4] = {in.gv[1][t4] * (float)dv[0], in.gv[1][t4 + 1] * (float)dv[1],
-                          in.gv[1][t4 + 2] * (float)dv[2], in.gv[1][t4 + 3] * (float)dv[3]};
+      const f32x4 dv = to_f4<TIn>(read_tr4(in.dot + dperm(t4 + (r >> 2)) * BV + 4 * (r & 3)), rsd.v);
+      const float x[4] = {in.gv[1][t4] * dv[0], in.gv[1][t4 + 1] * dv[1], in.gv[1][t4 + 2] * dv[2],
+                          in.gv[1][t4 + 3] * dv[3]};
       store_pair4(&s.gh[r][t4], &s.gl[r][t4], x);
       copy_state_rows<K, 128>(s.sh, reinterpret_cast<f16*>(p.ckD) + (ri * p.V + v0) * (int64_t)K, ll);
       // chunk c + 1's rows of T^T du: a chunk late, so that the drain at its
@@ -1147,7 +1159,7 @@ __device__ __forceinline__ void walk_backward16(const BArgs& p, RMem<K>& s, cons
         const int m0 = 16 * (wave + 4 * j);
         aq[j] = f32x4{0.f, 0.f, 0.f, 0.f};
         if (m0 < K) {
-          const f16x8 qt = frag8_ts<K>(in.q, 0, m0, r, kq);
+          const f16x8 qt = op8<TIn>(frag8_ts<K>(in.q, 0, m0, r, kq));
           aq[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(qt, frag8(&s.gh[r][8 * kq]), aq[j], 0, 0, 0);
           aq[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(qt, frag8(&s.gl[r][8 * kq]), aq[j], 0, 0, 0);
         }
@@ -1179,7 +1191,7 @@ __device__ __forceinline__ void walk_backward16(const BArgs& p, RMem<K>& s, cons
     for (int j = 0; j < State<K>::NST; ++j) {
       const int m0 = 16 * (wave + 4 * j);
       if (m0 < K) {
-        const f16x8 kt = frag8_ts<K>(in.k, 0, m0, r, kq);
+        const f16x8 kt = op8<TIn>(frag8_ts<K>(in.k, 0, m0, r, kq));
         f32x4 b = {0.f, 0.f, 0.f, 0.f};
         b = __builtin_amdgcn_mfma_f32_16x16x32_f16(kt, frag8(&s.zh[r][8 * kq]), b, 0, 0, 0);
         b = __builtin_amdgcn_mfma_f32_16x16x32_f16(kt, frag8(&s.zl[r][8 * kq]), b, 0, 0, 0);
