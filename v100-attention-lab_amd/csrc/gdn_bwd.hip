@@ -34,7 +34,8 @@
 //      the gates, T and P, the last two as fp16 pairs;
 //   2. recur_kernel (fp32) or recur16_kernel (16-bit q, k, v, dO: fp16 MFMA
 //      on hi + lo pairs), one workgroup per (sequence, head, 16-column V
-//      slice) and direction, both directions in one launch: the forward
+//      slice; 32 columns in large 16-bit launches) and direction, both
+//      directions in one launch: the forward
 //      walk stores each chunk's start state S and u; the backward walk
 //      stores each chunk's dS' and du and finally dh0.  The 16-bit walks
 //      store S and dS' in fp16 (half the bytes of the largest arrays of
@@ -58,6 +59,7 @@ namespace bwd {
 
 constexpr int NTP = 256;  // threads: prep_kernel and recur_kernel (4 waves)
 constexpr int NTG = 512;  // threads: grad_kernel (8 waves)
+constexpr int kCUs = 256;  // of an MI355X
 
 // ---------------------------------------------------------------------------
 // 1. prep: the state-independent half of a chunk's forward
@@ -687,7 +689,9 @@ __global__ __launch_bounds__(NTP) void recur_kernel(const BArgs p) {
 //     accumulators of the four waves (rows 16 (w + 4 j) of K); an fp16 hi /
 //     lo copy of its transpose in LDS feeds the products through it.  K^T,
 //     Q^T, P^T and W^T are read from row-major LDS copies by transposing
-//     reads.  Per chunk: the u (du) tiles on waves 0-1, then the state
+//     reads.  A workgroup takes NB blocks of 16 columns: a wave does a row
+//     tile's products for every block, from one read of its k, q, T or P
+//     operand.  Per chunk: the u (du) tiles on waves 0-1, then the state
 //     update on all four waves; the inputs of the chunks ahead arrive in
 //     LDS by LDS-DMA copies that waves 2-3 (and, for q, waves 0-1) issue
 //     and drain themselves.
@@ -812,24 +816,39 @@ __device__ __forceinline__ void zero_v(f16* dst, int nval, int lane) {
   if (pos / BV >= nval) *reinterpret_cast<f16x8*>(dst + pos) = f16x8{};
 }
 
+// Rows of N halves of the pairs the walks form, in LDS: padded, or, where two
+// blocks of columns need the room, permuted like the inputs' rows (one block
+// permuted: 0.2 % slower, train step B2 T4096 H16 K = V = 128 fp16).
+template <int N, int NB>
+constexpr int LDP = NB == 1 ? N + HP : N;
+template <int N, int NB>
+__device__ __forceinline__ int poff(int row, int col) {
+  return NB == 1 ? row * LDP<N, NB> + col : soff<N>(row, col);
+}
+template <int N, int NB>
+__device__ __forceinline__ f16x8 pfrag8(const f16* x, int row, int col) {
+  return frag8(x + poff<N, NB>(row, col));
+}
+
 // A chunk's inputs of the forward walk in LDS.
-template <int K>
+template <int K, int NB>
 struct alignas(16) FIn {
   f16 k[C * K];               // K rows, swz<K>
   f16 th[C * C], tl[C * C];   // T as fp16 pairs, swz<C>
-  f16 v[C * BV];              // V rows of the slice
+  f16 v[NB][C * BV];          // V rows of the slice, by blocks of BV columns
   float gv[4][C];             // b, gam, D, beta
 };
 
 // The forward walk's inputs are triple-buffered (chunk c in in[c % 3]): a
 // chunk's copies are issued two chunks ahead and have a whole chunk to land.
-template <int K>
+template <int K, int NB>
 struct alignas(16) FMem {
-  f16 sh[BV][K + HP], sl[BV][K + HP];  // S^T
-  f16 yh[BV][C + HP], yl[BV][C + HP];  // (diag(beta) (V - diag(gam) K S))^T
-  f16 dh[BV][C + HP], dl[BV][C + HP];  // (diag(D) u)^T
-  float uf[C][BV];                     // u rows, on their way to uu
-  FIn<K> in[3];
+  static constexpr int W = NB * BV;
+  f16 sh[W * LDP<K, NB>], sl[W * LDP<K, NB>];    // S^T
+  f16 yh[W * LDP<C, NB>], yl[W * LDP<C, NB>];    // (diag(beta) (V - diag(gam) K S))^T
+  f16 dh[W * LDP<C, NB>], dl[W * LDP<C, NB>];    // (diag(D) u)^T
+  float uf[C][W];                    // u rows, on their way to uu
+  FIn<K, NB> in[3];
 };
 
 // A chunk's inputs of the backward walk in LDS.
@@ -837,51 +856,89 @@ template <int K>
 struct alignas(16) RIn {
   f16 q[C * K], k[C * K];     // Q, K rows, swz<K>
   f16 th[C * C], tl[C * C];   // T, swz<C>
-  f16 ph[C * C], pl[C * C];   // P, swz<C>
-  f16 dot[C * BV];            // dO rows of the slice, row t at dperm(t)
   float gv[4][C];
 };
+// and those that only a chunk's first phase reads
+template <int NB>
+struct alignas(16) RIn1 {
+  f16 ph[C * C], pl[C * C];   // P, swz<C>
+  f16 dot[NB][C * BV];        // dO rows of the slice, row t at dperm(t)
+};
 
-template <int K>
+// At 32 columns the first phase's inputs have one buffer, refilled in the
+// second phase: 79 KB at K = 128, so that two workgroups share a CU.
+template <int K, int NB>
 struct alignas(16) RMem {
-  f16 sh[BV][K + HP], sl[BV][K + HP];  // dS'^T
-  f16 gh[BV][C + HP], gl[BV][C + HP];  // (diag(gam) dO)^T
-  f16 uh[BV][C + HP], ul[BV][C + HP];  // du^T
-  f16 zh[BV][C + HP], zl[BV][C + HP];  // (diag(beta gam) T^T du)^T
-  float duf[C][BV];                    // T^T du rows, on their way to du
+  static constexpr int W = NB * BV, NI1 = NB == 1 ? 2 : 1;
+  f16 sh[W * LDP<K, NB>], sl[W * LDP<K, NB>];    // dS'^T
+  f16 gh[W * LDP<C, NB>], gl[W * LDP<C, NB>];    // (diag(gam) dO)^T
+  f16 uh[W * LDP<C, NB>], ul[W * LDP<C, NB>];    // du^T
+  f16 zh[W * LDP<C, NB>], zl[W * LDP<C, NB>];    // (diag(beta gam) T^T du)^T
+  float duf[C][W];                   // T^T du rows, on their way to du
   RIn<K> in[2];
+  RIn1<NB> in1[NI1];
 };
 
-template <int K>
+template <int K, int NB>
 union Mem {
-  FMem<K> f;
-  RMem<K> r;
+  FMem<K, NB> f;
+  RMem<K, NB> r;
 };
 
-template <int K>
-struct State {
-  static constexpr int NST = (K / 16 + 3) / 4;
-  f32x4 st[NST];
-  // times sc (a power of two: exact)
-  __device__ __forceinline__ void load(const float* src, const int64_t (&sd)[4], int bi, int hi, int v0, int wave,
-                                       int r, int kq, float sc = 1.f) {
+// One range scale per block of BV columns, whatever the walk's width (the
+// gradient kernel reads them by block): the largest magnitudes in one pass.
+// Every thread calls it.
+template <typename TIn, int NB>
+__device__ __forceinline__ void block_scales(RangeScale (&rs)[NB], const TIn* x, int64_t ld, int rows, const float* h0,
+                                             int64_t sk, int64_t sc, int K) {
+  if constexpr (NB == 1) {
+    rs[0] = slice_range_scale<TIn>(reinterpret_cast<const char*>(x), ld * (int64_t)sizeof(TIn), rows, BV, h0, sk, sc,
+                                   K, 1.f);
+  } else if constexpr (std::is_same<TIn, bf16_t>::value) {
+    __shared__ uint32_t red[NB][16];
+    constexpr int PIECES = NB * BV / 8;  // 16-byte pieces of a row, a fixed one per thread
+    static_assert(NTP % PIECES == 0, "a fixed piece per thread");
+    const int piece = threadIdx.x % PIECES;
+    const uint32_t m = column_absmax_bits(reinterpret_cast<const char*>(x) + 16 * piece, ld * (int64_t)sizeof(TIn),
+                                          rows, threadIdx.x / PIECES, NTP / PIECES);
 #pragma unroll
-    for (int j = 0; j < NST; ++j) {
-      const int m0 = 16 * (wave + 4 * j);
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        st[j][i] = (src && m0 < K) ? src[bi * sd[0] + hi * sd[1] + (m0 + 4 * kq + i) * sd[2] + (v0 + r) * sd[3]] * sc
-                                   : 0.f;
+    for (int cb = 0; cb < NB; ++cb) {
+      const uint32_t h = state_absmax_bits(h0 ? h0 + cb * BV * sc : nullptr, sk, sc, K, BV);
+      rs[cb] = range_scale_of(__uint_as_float(block_max_bits(max(piece / (BV / 8) == cb ? m : 0u, h), red[cb])), 1.f);
     }
   }
-  template <int LD>
-  __device__ __forceinline__ void put(f16 (*sh)[LD], f16 (*sl)[LD], int wave, int r, int kq) const {
+}
+
+template <int K, int NB>
+struct State {
+  static constexpr int NST = (K / 16 + 3) / 4;
+  f32x4 st[NB][NST];
+  // each block times its scale (a power of two: exact)
+  __device__ __forceinline__ void load(const float* src, const int64_t (&sd)[4], int bi, int hi, int v0, int wave,
+                                       int r, int kq, const RangeScale (&sc)[NB]) {
+#pragma unroll
+    for (int cb = 0; cb < NB; ++cb)
+#pragma unroll
+      for (int j = 0; j < NST; ++j) {
+        const int m0 = 16 * (wave + 4 * j);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          st[cb][j][i] = (src && m0 < K) ? src[bi * sd[0] + hi * sd[1] + (m0 + 4 * kq + i) * sd[2] +
+                                               (v0 + BV * cb + r) * sd[3]] * sc[cb].v
+                                         : 0.f;
+      }
+  }
+  __device__ __forceinline__ void put(f16* sh, f16* sl, int wave, int r, int kq) const {
 #pragma unroll
     for (int j = 0; j < NST; ++j) {
       const int m0 = 16 * (wave + 4 * j);
       if (m0 < K) {
-        const float x[4] = {st[j][0], st[j][1], st[j][2], st[j][3]};
-        store_pair4(&sh[r][m0 + 4 * kq], &sl[r][m0 + 4 * kq], x);
+#pragma unroll
+        for (int cb = 0; cb < NB; ++cb) {
+          const float x[4] = {st[cb][j][0], st[cb][j][1], st[cb][j][2], st[cb][j][3]};
+          const int at = poff<K, NB>(BV * cb + r, m0 + 4 * kq);
+          store_pair4(sh + at, sl + at, x);
+        }
       }
     }
   }
@@ -890,15 +947,15 @@ struct State {
 // The state's fp16 values -> rows of the [V][K] chunk-state array (row =
 // state column), 16 bytes a lane (NT lanes).  They are the hi parts of the walk's
 // S^T pair copy (x rounded to nearest), copied as they are.
-template <int K, int NT, int LD>
-__device__ __forceinline__ void copy_state_rows(const f16 (*sh)[LD], f16* dst, int tid) {
-  constexpr int NV = BV * K / 8;
+template <int K, int NB, int NT>
+__device__ __forceinline__ void copy_state_rows(const f16* sh, f16* dst, int tid) {
+  constexpr int NV = NB * BV * K / 8;
 #pragma unroll
   for (int i = 0; i < (NV + NT - 1) / NT; ++i) {
     const int e = tid + i * NT;
     if (NV % NT == 0 || e < NV)
       *reinterpret_cast<f16x8*>(dst + (int64_t)(e / (K / 8)) * K + 8 * (e % (K / 8))) =
-          *reinterpret_cast<const f16x8*>(&sh[e / (K / 8)][8 * (e % (K / 8))]);
+          pfrag8<K, NB>(sh, e / (K / 8), 8 * (e % (K / 8)));
   }
 }
 
@@ -912,8 +969,8 @@ __device__ __forceinline__ void copy_state_rows(const f16 (*sh)[LD], f16* dst, i
 // while the other waits for the copies of chunk c + 1 it issued a chunk
 // earlier (its only memory operations in flight).  Waves 0 and 1 hold the
 // chain's products (Y, u).
-template <typename TIn, int K>
-__device__ __forceinline__ void walk_forward16(const BArgs& p, FMem<K>& s, const RowSpan& rs, int bi, int hi,
+template <typename TIn, int K, int NB>
+__device__ __forceinline__ void walk_forward16(const BArgs& p, FMem<K, NB>& s, const RowSpan& rs, int bi, int hi,
                                                int v0, int64_t slot0) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -921,22 +978,27 @@ __device__ __forceinline__ void walk_forward16(const BArgs& p, FMem<K>& s, const
   const int nch = (rs.T + C - 1) / C;
   const TIn* const kg = static_cast<const TIn*>(p.k) + head_base(rs, hi, p.sk);
   const TIn* const vg = static_cast<const TIn*>(p.v) + head_base(rs, hi, p.sv) + v0;
-  const RangeScale rsc = slice_range_scale<TIn>(
-      reinterpret_cast<const char*>(vg), p.sv[1] * (int64_t)sizeof(TIn), rs.T, BV,
-      p.h0 ? p.h0 + bi * p.sh0[0] + hi * p.sh0[1] + v0 * p.sh0[3] : nullptr, p.sh0[2], p.sh0[3], K, 1.f);
-  if (tid == 0) p.scl[((int64_t)bi * p.H + hi) * p.nv + v0 / BV] = rsc.fs;
+  constexpr int W = NB * BV;
+  RangeScale rsc[NB];
+  block_scales<TIn, NB>(rsc, vg, p.sv[1], rs.T,
+                        p.h0 ? p.h0 + bi * p.sh0[0] + hi * p.sh0[1] + v0 * p.sh0[3] : nullptr, p.sh0[2], p.sh0[3], K);
+#pragma unroll
+  for (int cb = 0; cb < NB; ++cb)
+    if (tid == 0) p.scl[((int64_t)bi * p.H + hi) * p.nv + v0 / BV + cb] = rsc[cb].fs;
   const bool loader = wave >= 2;
   const int lw = wave - 2;
   // a loader: chunk cn's inputs -> in[b]
   auto fetch = [&](int cn, int b) __attribute__((always_inline)) {
-    FIn<K>& d = s.in[b];
+    FIn<K, NB>& d = s.in[b];
     const int64_t ri = (slot0 + cn) * p.H + hi;
     const int nval = min(C, rs.T - cn * C);
     const uint16_t* const rh = reinterpret_cast<const uint16_t*>(p.r16 + ri * (int64_t)Rec16::SIZE);
     dma_rows<K, 1>(reinterpret_cast<const uint16_t*>(kg) + (int64_t)cn * C * p.sk[1], p.sk[1], nval, d.k, 0, lane);
     dma_rows<C, 1>(rh + Rec16::TH, C, C, d.th, 0, lane);
     dma_rows<C, 1>(rh + Rec16::TL, C, C, d.tl, 0, lane);
-    dma_v(reinterpret_cast<const uint16_t*>(vg) + (int64_t)cn * C * p.sv[1], p.sv[1], nval, d.v, lane);
+#pragma unroll
+    for (int cb = 0; cb < NB; ++cb)
+      dma_v(reinterpret_cast<const uint16_t*>(vg) + (int64_t)cn * C * p.sv[1] + BV * cb, p.sv[1], nval, d.v[cb], lane);
     if (lane < C) dma16(p.rec + ri * (int64_t)RecT::SIZE + RecT::G + 4 * lane, &d.gv[0][0]);
   };
   // the loader that fetched chunk cn, before the barrier that publishes it
@@ -945,11 +1007,12 @@ __device__ __forceinline__ void walk_forward16(const BArgs& p, FMem<K>& s, const
     const int nval = min(C, rs.T - cn * C);
     if (nval < C) {
       zero_rows<K, 1>(s.in[b].k, nval, 0, lane);
-      zero_v(s.in[b].v, nval, lane);
+#pragma unroll
+      for (int cb = 0; cb < NB; ++cb) zero_v(s.in[b].v[cb], nval, lane);
     }
   };
-  State<K> S;
-  S.load(p.h0, p.sh0, bi, hi, v0, wave, r, kq, rsc.v);
+  State<K, NB> S;
+  S.load(p.h0, p.sh0, bi, hi, v0, wave, r, kq, rsc);
   S.put(s.sh, s.sl, wave, r, kq);
   if (loader && lw < nch) {
     fetch(lw, lw);
@@ -958,26 +1021,37 @@ __device__ __forceinline__ void walk_forward16(const BArgs& p, FMem<K>& s, const
   bar();
   for (int c = 0, b = 0; c < nch; ++c, b = b == 2 ? 0 : b + 1) {
     const int64_t ri = (slot0 + c) * p.H + hi;
-    FIn<K>& in = s.in[b];
+    FIn<K, NB>& in = s.in[b];
     const int b1 = b == 2 ? 0 : b + 1, b2 = b1 == 2 ? 0 : b1 + 1;
     const bool issuer = loader && lw == (c & 1);
     if (!loader) {
       // Y = diag(beta) (V - diag(gam) K S), rows 16 w .. (k exact in fp16), as
       // Y^T pairs
       const int um0 = 16 * wave;
-      f32x4 ak = {0.f, 0.f, 0.f, 0.f};
+      f32x4 ak[NB];
+#pragma unroll
+      for (int cb = 0; cb < NB; ++cb) ak[cb] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int kb = 0; kb < K; kb += 32) {
         const f16x8 kf = op8<TIn>(frag8_s<K>(in.k, um0 + r, kb + 8 * kq));
-        ak = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, frag8(&s.sh[r][kb + 8 * kq]), ak, 0, 0, 0);
-        ak = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, frag8(&s.sl[r][kb + 8 * kq]), ak, 0, 0, 0);
+#pragma unroll
+        for (int cb = 0; cb < NB; ++cb)
+          ak[cb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, pfrag8<K, NB>(s.sh, BV * cb + r, kb + 8 * kq), ak[cb], 0,
+                                                          0, 0);
+#pragma unroll
+        for (int cb = 0; cb < NB; ++cb)
+          ak[cb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, pfrag8<K, NB>(s.sl, BV * cb + r, kb + 8 * kq), ak[cb], 0,
+                                                          0, 0);
       }
       const int t = um0 + 4 * kq;
-      const f32x4 vv = to_f4<TIn>(frag4_t(reinterpret_cast<const f16 (*)[BV]>(in.v), um0, 0, r, kq), rsc.v);
-      float y[4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) y[i] = in.gv[3][t + i] * (vv[i] - in.gv[1][t + i] * ak[i]);
-      store_pair4(&s.yh[r][t], &s.yl[r][t], y);
+      for (int cb = 0; cb < NB; ++cb) {
+        const f32x4 vv = to_f4<TIn>(frag4_t(reinterpret_cast<const f16 (*)[BV]>(in.v[cb]), um0, 0, r, kq), rsc[cb].v);
+        float y[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) y[i] = in.gv[3][t + i] * (vv[i] - in.gv[1][t + i] * ak[cb][i]);
+        store_pair4(s.yh + poff<C, NB>(BV * cb + r, t), s.yl + poff<C, NB>(BV * cb + r, t), y);
+      }
     } else if (issuer && c + 2 < nch) {
       fetch(c + 2, b2);
     }
@@ -985,43 +1059,54 @@ __device__ __forceinline__ void walk_forward16(const BArgs& p, FMem<K>& s, const
     if (!loader) {
       // u = T Y, rows 16 w ..
       const int um0 = 16 * wave;
-      f32x4 au = {0.f, 0.f, 0.f, 0.f};
-      const f16x8 th = frag8_s<C>(in.th, um0 + r, 8 * kq), yh = frag8(&s.yh[r][8 * kq]);
-      au = __builtin_amdgcn_mfma_f32_16x16x32_f16(th, yh, au, 0, 0, 0);
-      au = __builtin_amdgcn_mfma_f32_16x16x32_f16(th, frag8(&s.yl[r][8 * kq]), au, 0, 0, 0);
-      au = __builtin_amdgcn_mfma_f32_16x16x32_f16(frag8_s<C>(in.tl, um0 + r, 8 * kq), yh, au, 0, 0, 0);
       const int t = um0 + 4 * kq;
-      float du[4];
+      f16x8 yhs[NB];
+      const f16x8 th = frag8_s<C>(in.th, um0 + r, 8 * kq);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        du[i] = in.gv[2][t + i] * au[i];
-        s.uf[t + i][r] = au[i] * rsc.fs;
+      for (int cb = 0; cb < NB; ++cb) yhs[cb] = pfrag8<C, NB>(s.yh, BV * cb + r, 8 * kq);
+      const f16x8 tl = frag8_s<C>(in.tl, um0 + r, 8 * kq);
+#pragma unroll
+      for (int cb = 0; cb < NB; ++cb) {
+        f32x4 au = {0.f, 0.f, 0.f, 0.f};
+        const f16x8 yh = yhs[cb];
+        au = __builtin_amdgcn_mfma_f32_16x16x32_f16(th, yh, au, 0, 0, 0);
+        au = __builtin_amdgcn_mfma_f32_16x16x32_f16(th, pfrag8<C, NB>(s.yl, BV * cb + r, 8 * kq), au, 0, 0, 0);
+        au = __builtin_amdgcn_mfma_f32_16x16x32_f16(tl, yh, au, 0, 0, 0);
+        float du[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          du[i] = in.gv[2][t + i] * au[i];
+          s.uf[t + i][BV * cb + r] = au[i] * rsc[cb].fs;
+        }
+        store_pair4(s.dh + poff<C, NB>(BV * cb + r, t), s.dl + poff<C, NB>(BV * cb + r, t), du);
       }
-      store_pair4(&s.dh[r][t], &s.dl[r][t], du);
     } else if (issuer) {
-      copy_state_rows<K, 64>(s.sh, reinterpret_cast<f16*>(p.ckS) + (ri * p.V + v0) * (int64_t)K, lane);
+      copy_state_rows<K, NB, 64>(s.sh, reinterpret_cast<f16*>(p.ckS) + (ri * p.V + v0) * (int64_t)K, lane);
     }
     bar();
     // S <- gam_C S + K^T diag(D) u
 #pragma unroll
-    for (int j = 0; j < State<K>::NST; ++j) {
+    for (int j = 0; j < State<K, NB>::NST; ++j) {
       const int m0 = 16 * (wave + 4 * j);
       if (m0 < K) {
         const f16x8 kt = op8<TIn>(frag8_ts<K>(in.k, 0, m0, r, kq));
-        f32x4 a = {0.f, 0.f, 0.f, 0.f};
-        a = __builtin_amdgcn_mfma_f32_16x16x32_f16(kt, frag8(&s.dh[r][8 * kq]), a, 0, 0, 0);
-        a = __builtin_amdgcn_mfma_f32_16x16x32_f16(kt, frag8(&s.dl[r][8 * kq]), a, 0, 0, 0);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) S.st[j][i] = in.gv[1][C - 1] * S.st[j][i] + a[i];
+        for (int cb = 0; cb < NB; ++cb) {
+          f32x4 a = {0.f, 0.f, 0.f, 0.f};
+          a = __builtin_amdgcn_mfma_f32_16x16x32_f16(kt, pfrag8<C, NB>(s.dh, BV * cb + r, 8 * kq), a, 0, 0, 0);
+          a = __builtin_amdgcn_mfma_f32_16x16x32_f16(kt, pfrag8<C, NB>(s.dl, BV * cb + r, 8 * kq), a, 0, 0, 0);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) S.st[cb][j][i] = in.gv[1][C - 1] * S.st[cb][j][i] + a[i];
+        }
       }
     }
     S.put(s.sh, s.sl, wave, r, kq);
     if (issuer) {
       // u rows -> uu: 16 bytes a lane
-      static_assert(C * BV % (4 * 64) == 0, "whole u pieces per lane");
+      static_assert(C * W % (4 * 64) == 0, "whole u pieces per lane");
 #pragma unroll
-      for (int i = 0; i < C * BV / (4 * 64); ++i) {
-        const int e = lane + 64 * i, row = e / (BV / 4), c4 = 4 * (e % (BV / 4));
+      for (int i = 0; i < C * W / (4 * 64); ++i) {
+        const int e = lane + 64 * i, row = e / (W / 4), c4 = 4 * (e % (W / 4));
         *reinterpret_cast<f32x4*>(p.uu + (ri * C + row) * (int64_t)p.V + v0 + c4) =
             *reinterpret_cast<const f32x4*>(&s.uf[row][c4]);
       }
@@ -1042,8 +1127,8 @@ __device__ __forceinline__ void walk_forward16(const BArgs& p, FMem<K>& s, const
 // Waves 2 and 3 (the loaders) copy the previous chunk's inputs but its q
 // rows and store the chunk's dS' rows and du rows; waves 0 and 1 hold the
 // chain's products (du, z) and copy the q rows once their du is done.
-template <typename TIn, int K>
-__device__ __forceinline__ void walk_backward16(const BArgs& p, RMem<K>& s, const RowSpan& rs, int bi, int hi,
+template <typename TIn, int K, int NB>
+__device__ __forceinline__ void walk_backward16(const BArgs& p, RMem<K, NB>& s, const RowSpan& rs, int bi, int hi,
                                                 int v0, int64_t slot0) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1053,10 +1138,14 @@ __device__ __forceinline__ void walk_backward16(const BArgs& p, RMem<K>& s, cons
   const TIn* const qg = static_cast<const TIn*>(p.q) + head_base(rs, hi, p.sq);
   const TIn* const kg = static_cast<const TIn*>(p.k) + head_base(rs, hi, p.sk);
   const TIn* const dg = static_cast<const TIn*>(p.d_o) + head_base(rs, hi, p.sdo) + v0;
-  const RangeScale rsd = slice_range_scale<TIn>(
-      reinterpret_cast<const char*>(dg), p.sdo[1] * (int64_t)sizeof(TIn), rs.T, BV,
-      p.dfs ? p.dfs + bi * p.sdfs[0] + hi * p.sdfs[1] + v0 * p.sdfs[3] : nullptr, p.sdfs[2], p.sdfs[3], K, 1.f);
-  if (tid == 0) p.scl[p.units + ((int64_t)bi * p.H + hi) * p.nv + v0 / BV] = rsd.fs;
+  constexpr int W = NB * BV, NI1 = RMem<K, NB>::NI1;
+  RangeScale rsd[NB];
+  block_scales<TIn, NB>(rsd, dg, p.sdo[1], rs.T,
+                        p.dfs ? p.dfs + bi * p.sdfs[0] + hi * p.sdfs[1] + v0 * p.sdfs[3] : nullptr, p.sdfs[2],
+                        p.sdfs[3], K);
+#pragma unroll
+  for (int cb = 0; cb < NB; ++cb)
+    if (tid == 0) p.scl[p.units + ((int64_t)bi * p.H + hi) * p.nv + v0 / BV + cb] = rsd[cb].fs;
   const bool loader = wave >= 2;
   const int lw = wave - 2, ll = tid - 128;
   // chunk cn's inputs -> in[cn & 1]: q rows from waves 0 and 1 (issued at
@@ -1075,10 +1164,21 @@ __device__ __forceinline__ void walk_backward16(const BArgs& p, RMem<K>& s, cons
     dma_rows<K, 2>(reinterpret_cast<const uint16_t*>(kg) + (int64_t)cn * C * p.sk[1], p.sk[1], nval, d.k, lw, lane);
     dma_rows<C, 2>(rh + Rec16::TH, C, C, d.th, lw, lane);
     dma_rows<C, 2>(rh + Rec16::TL, C, C, d.tl, lw, lane);
+  };
+  // the loaders: what the chunk's first phase alone reads, and the gates
+  auto fetch1 = [&](int cn) __attribute__((always_inline)) {
+    RIn1<NB>& d = s.in1[cn & (NI1 - 1)];
+    const int64_t ri = (slot0 + cn) * p.H + hi;
+    const uint16_t* const rh = reinterpret_cast<const uint16_t*>(p.r16 + ri * (int64_t)Rec16::SIZE);
+    const int nval = min(C, rs.T - cn * C);
     dma_rows<C, 2>(rh + Rec16::PH, C, C, d.ph, lw, lane);
     dma_rows<C, 2>(rh + Rec16::PL, C, C, d.pl, lw, lane);
-    dma_dot(reinterpret_cast<const uint16_t*>(dg) + (int64_t)cn * C * p.sdo[1], p.sdo[1], nval, d.dot, lw, lane);
-    if (lw == 0 && lane < C) dma16(p.rec + ri * (int64_t)RecT::SIZE + RecT::G + 4 * lane, &d.gv[0][0]);
+#pragma unroll
+    for (int cb = 0; cb < NB; ++cb)
+      dma_dot(reinterpret_cast<const uint16_t*>(dg) + (int64_t)cn * C * p.sdo[1] + BV * cb, p.sdo[1], nval, d.dot[cb],
+              lw, lane);
+    if (lw == 0 && lane < C)
+      dma16(p.rec + ri * (int64_t)RecT::SIZE + RecT::G + 4 * lane, &s.in[cn & 1].gv[0][0]);
   };
   // every wave, before the barrier that publishes chunk cn: its own copies
   auto settle = [&](int cn) __attribute__((always_inline)) {
@@ -1090,60 +1190,88 @@ __device__ __forceinline__ void walk_backward16(const BArgs& p, RMem<K>& s, cons
         zero_rows<K, 2>(d.q, nval, wave, lane);
       } else {
         zero_rows<K, 2>(d.k, nval, lw, lane);
-        zero_dot(d.dot, nval, lw, lane);
+#pragma unroll
+        for (int cb = 0; cb < NB; ++cb) zero_dot(s.in1[cn & (NI1 - 1)].dot[cb], nval, lw, lane);
       }
     }
   };
   // a loader: chunk cn's rows of T^T du (still in duf) -> du, 16 bytes a lane
   auto store_duf = [&](int cn) __attribute__((always_inline)) {
-    static_assert(C * BV == 4 * 128, "four entries per loader lane");
-    const int row = ll / (BV / 4), c4 = 4 * (ll % (BV / 4));
-    *reinterpret_cast<f32x4*>(p.du + (((slot0 + cn) * p.H + hi) * C + row) * (int64_t)p.V + v0 + c4) =
-        *reinterpret_cast<const f32x4*>(&s.duf[row][c4]);
+    static_assert(C * BV == 4 * 128, "four entries per loader lane and block");
+#pragma unroll
+    for (int i = 0; i < NB; ++i) {
+      const int e = ll + 128 * i, row = e / (W / 4), c4 = 4 * (e % (W / 4));
+      *reinterpret_cast<f32x4*>(p.du + (((slot0 + cn) * p.H + hi) * C + row) * (int64_t)p.V + v0 + c4) =
+          *reinterpret_cast<const f32x4*>(&s.duf[row][c4]);
+    }
   };
-  State<K> S;
-  S.load(p.dfs, p.sdfs, bi, hi, v0, wave, r, kq, rsd.v);
+  State<K, NB> S;
+  S.load(p.dfs, p.sdfs, bi, hi, v0, wave, r, kq, rsd);
   S.put(s.sh, s.sl, wave, r, kq);
   if (nch > 0) {
     fetch(nch - 1);
+    if (loader) fetch1(nch - 1);
     settle(nch - 1);
   }
   bar();
   for (int c = nch - 1; c >= 0; --c) {
     const int64_t ri = (slot0 + c) * p.H + hi;
     RIn<K>& in = s.in[c & 1];
+    RIn1<NB>& in1 = s.in1[c & (NI1 - 1)];
     if (!loader) {
       // du = scale P^T dO + diag(D) K dS', rows 16 w ..
       const int um0 = 16 * wave;
-      f32x4 a1 = {0.f, 0.f, 0.f, 0.f}, a2 = {0.f, 0.f, 0.f, 0.f};
-      const f16x8 df = dot_frag8<TIn>(in.dot, r, kq, rsd.v);
-      a1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(frag8_ts<C>(in.ph, 0, um0, r, kq), df, a1, 0, 0, 0);
-      a1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(frag8_ts<C>(in.pl, 0, um0, r, kq), df, a1, 0, 0, 0);
+      f32x4 a1[NB], a2[NB];
+      f16x8 df[NB];
+#pragma unroll
+      for (int cb = 0; cb < NB; ++cb) df[cb] = dot_frag8<TIn>(in1.dot[cb], r, kq, rsd[cb].v);
+      const f16x8 ph = frag8_ts<C>(in1.ph, 0, um0, r, kq), pl = frag8_ts<C>(in1.pl, 0, um0, r, kq);
+#pragma unroll
+      for (int cb = 0; cb < NB; ++cb) {
+        a1[cb] = a2[cb] = f32x4{0.f, 0.f, 0.f, 0.f};
+        a1[cb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ph, df[cb], a1[cb], 0, 0, 0);
+        a1[cb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pl, df[cb], a1[cb], 0, 0, 0);
+      }
 #pragma unroll
       for (int kb = 0; kb < K; kb += 32) {
         const f16x8 kf = op8<TIn>(frag8_s<K>(in.k, um0 + r, kb + 8 * kq));
-        a2 = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, frag8(&s.sh[r][kb + 8 * kq]), a2, 0, 0, 0);
-        a2 = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, frag8(&s.sl[r][kb + 8 * kq]), a2, 0, 0, 0);
+#pragma unroll
+        for (int cb = 0; cb < NB; ++cb)
+          a2[cb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, pfrag8<K, NB>(s.sh, BV * cb + r, kb + 8 * kq), a2[cb], 0,
+                                                          0, 0);
+#pragma unroll
+        for (int cb = 0; cb < NB; ++cb)
+          a2[cb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, pfrag8<K, NB>(s.sl, BV * cb + r, kb + 8 * kq), a2[cb], 0,
+                                                          0, 0);
       }
       const int t = um0 + 4 * kq;
-      float du[4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        du[i] = scale * a1[i] + in.gv[2][t + i] * a2[i];
+      for (int cb = 0; cb < NB; ++cb) {
+        float du[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          du[i] = scale * a1[cb][i] + in.gv[2][t + i] * a2[cb][i];
+        }
+        store_pair4(s.uh + poff<C, NB>(BV * cb + r, t), s.ul + poff<C, NB>(BV * cb + r, t), du);
       }
-      store_pair4(&s.uh[r][t], &s.ul[r][t], du);
       if (c >= 1) fetch(c - 1);
     } else {
       // the previous chunk's copies first: they have until the chunk's end
-      if (c >= 1) fetch(c - 1);
+      if (c >= 1) {
+        fetch(c - 1);
+        if (NI1 == 2) fetch1(c - 1);
+      }
       // (diag(gam) dO)^T as pairs: lane (r, kq) of loader wave lw -> column
       // r, rows t4 .. t4 + 3 (a 32-lane pass reads rows 0..3, 8..11 + 16 lw)
       const int t4 = 16 * lw + ((kq & 1) << 3) + ((kq & 2) << 1);
-      const f32x4 dv = to_f4<TIn>(read_tr4(in.dot + dperm(t4 + (r >> 2)) * BV + 4 * (r & 3)), rsd.v);
-      const float x[4] = {in.gv[1][t4] * dv[0], in.gv[1][t4 + 1] * dv[1], in.gv[1][t4 + 2] * dv[2],
-                          in.gv[1][t4 + 3] * dv[3]};
-      store_pair4(&s.gh[r][t4], &s.gl[r][t4], x);
-      copy_state_rows<K, 128>(s.sh, reinterpret_cast<f16*>(p.ckD) + (ri * p.V + v0) * (int64_t)K, ll);
+#pragma unroll
+      for (int cb = 0; cb < NB; ++cb) {
+        const f32x4 dv = to_f4<TIn>(read_tr4(in1.dot[cb] + dperm(t4 + (r >> 2)) * BV + 4 * (r & 3)), rsd[cb].v);
+        const float x[4] = {in.gv[1][t4] * dv[0], in.gv[1][t4 + 1] * dv[1], in.gv[1][t4 + 2] * dv[2],
+                            in.gv[1][t4 + 3] * dv[3]};
+        store_pair4(s.gh + poff<C, NB>(BV * cb + r, t4), s.gl + poff<C, NB>(BV * cb + r, t4), x);
+      }
+      copy_state_rows<K, NB, 128>(s.sh, reinterpret_cast<f16*>(p.ckD) + (ri * p.V + v0) * (int64_t)K, ll);
       // chunk c + 1's rows of T^T du: a chunk late, so that the drain at its
       // end did not wait for their stores
       if (c + 1 < nch) store_duf(c + 1);
@@ -1152,51 +1280,66 @@ __device__ __forceinline__ void walk_backward16(const BArgs& p, RMem<K>& s, cons
     // W^T du = K^T diag(beta gam) T^T du = K^T z: T^T du and z on waves 0-1
     // (rows 16 w .., T transposed by the reads) while waves 2-3 form their
     // Q^T diag(gam) dO term
-    f32x4 aq[State<K>::NST];
+    f32x4 aq[NB][State<K, NB>::NST];
     auto q_term = [&]() __attribute__((always_inline)) {
 #pragma unroll
-      for (int j = 0; j < State<K>::NST; ++j) {
+      for (int j = 0; j < State<K, NB>::NST; ++j) {
         const int m0 = 16 * (wave + 4 * j);
-        aq[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int cb = 0; cb < NB; ++cb) aq[cb][j] = f32x4{0.f, 0.f, 0.f, 0.f};
         if (m0 < K) {
           const f16x8 qt = op8<TIn>(frag8_ts<K>(in.q, 0, m0, r, kq));
-          aq[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(qt, frag8(&s.gh[r][8 * kq]), aq[j], 0, 0, 0);
-          aq[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(qt, frag8(&s.gl[r][8 * kq]), aq[j], 0, 0, 0);
+#pragma unroll
+          for (int cb = 0; cb < NB; ++cb) {
+            f32x4 x = aq[cb][j];
+            x = __builtin_amdgcn_mfma_f32_16x16x32_f16(qt, pfrag8<C, NB>(s.gh, BV * cb + r, 8 * kq), x, 0, 0, 0);
+            x = __builtin_amdgcn_mfma_f32_16x16x32_f16(qt, pfrag8<C, NB>(s.gl, BV * cb + r, 8 * kq), x, 0, 0, 0);
+            aq[cb][j] = x;
+          }
         }
       }
     };
     if (!loader) {
       const int um0 = 16 * wave;
       const f16x8 tth = frag8_ts<C>(in.th, 0, um0, r, kq), ttl = frag8_ts<C>(in.tl, 0, um0, r, kq);
-      const f16x8 uh = frag8(&s.uh[r][8 * kq]);
-      f32x4 az = {0.f, 0.f, 0.f, 0.f};
-      az = __builtin_amdgcn_mfma_f32_16x16x32_f16(tth, uh, az, 0, 0, 0);
-      az = __builtin_amdgcn_mfma_f32_16x16x32_f16(tth, frag8(&s.ul[r][8 * kq]), az, 0, 0, 0);
-      az = __builtin_amdgcn_mfma_f32_16x16x32_f16(ttl, uh, az, 0, 0, 0);
       const int t = um0 + 4 * kq;
-      float z[4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        z[i] = in.gv[1][t + i] * in.gv[3][t + i] * az[i];
-        s.duf[t + i][r] = az[i] * rsd.fs;
+      for (int cb = 0; cb < NB; ++cb) {
+        const f16x8 uh = pfrag8<C, NB>(s.uh, BV * cb + r, 8 * kq);
+        f32x4 az = {0.f, 0.f, 0.f, 0.f};
+        az = __builtin_amdgcn_mfma_f32_16x16x32_f16(tth, uh, az, 0, 0, 0);
+        az = __builtin_amdgcn_mfma_f32_16x16x32_f16(tth, pfrag8<C, NB>(s.ul, BV * cb + r, 8 * kq), az, 0, 0, 0);
+        az = __builtin_amdgcn_mfma_f32_16x16x32_f16(ttl, uh, az, 0, 0, 0);
+        float z[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          z[i] = in.gv[1][t + i] * in.gv[3][t + i] * az[i];
+          s.duf[t + i][BV * cb + r] = az[i] * rsd[cb].fs;
+        }
+        store_pair4(s.zh + poff<C, NB>(BV * cb + r, t), s.zl + poff<C, NB>(BV * cb + r, t), z);
       }
-      store_pair4(&s.zh[r][t], &s.zl[r][t], z);
     } else {
+      // the first phase's inputs: every wave has read chunk c's by now
+      if (NI1 == 1 && c >= 1) fetch1(c - 1);
       q_term();
     }
     bar();
     if (!loader) q_term();
     // dS <- scale Q^T diag(gam) dO + gam_C dS' - K^T z
 #pragma unroll
-    for (int j = 0; j < State<K>::NST; ++j) {
+    for (int j = 0; j < State<K, NB>::NST; ++j) {
       const int m0 = 16 * (wave + 4 * j);
       if (m0 < K) {
         const f16x8 kt = op8<TIn>(frag8_ts<K>(in.k, 0, m0, r, kq));
-        f32x4 b = {0.f, 0.f, 0.f, 0.f};
-        b = __builtin_amdgcn_mfma_f32_16x16x32_f16(kt, frag8(&s.zh[r][8 * kq]), b, 0, 0, 0);
-        b = __builtin_amdgcn_mfma_f32_16x16x32_f16(kt, frag8(&s.zl[r][8 * kq]), b, 0, 0, 0);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) S.st[j][i] = scale * aq[j][i] + in.gv[1][C - 1] * S.st[j][i] - b[i];
+        for (int cb = 0; cb < NB; ++cb) {
+          f32x4 b = {0.f, 0.f, 0.f, 0.f};
+          b = __builtin_amdgcn_mfma_f32_16x16x32_f16(kt, pfrag8<C, NB>(s.zh, BV * cb + r, 8 * kq), b, 0, 0, 0);
+          b = __builtin_amdgcn_mfma_f32_16x16x32_f16(kt, pfrag8<C, NB>(s.zl, BV * cb + r, 8 * kq), b, 0, 0, 0);
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            S.st[cb][j][i] = scale * aq[cb][j][i] + in.gv[1][C - 1] * S.st[cb][j][i] - b[i];
+        }
       }
     }
     S.put(s.sh, s.sl, wave, r, kq);
@@ -1207,13 +1350,15 @@ __device__ __forceinline__ void walk_backward16(const BArgs& p, RMem<K>& s, cons
   wait_dma();
   if (p.dh0 != nullptr) {
 #pragma unroll
-    for (int j = 0; j < State<K>::NST; ++j) {
+    for (int j = 0; j < State<K, NB>::NST; ++j) {
       const int m0 = 16 * (wave + 4 * j);
       if (m0 < K) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-          p.dh0[bi * p.sdh0[0] + hi * p.sdh0[1] + (m0 + 4 * kq + i) * p.sdh0[2] + (v0 + r) * p.sdh0[3]] =
-              S.st[j][i] * rsd.fs;
+        for (int cb = 0; cb < NB; ++cb)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            p.dh0[bi * p.sdh0[0] + hi * p.sdh0[1] + (m0 + 4 * kq + i) * p.sdh0[2] + (v0 + BV * cb + r) * p.sdh0[3]] =
+                S.st[cb][j][i] * rsd[cb].fs;
       }
     }
   }
@@ -1221,16 +1366,16 @@ __device__ __forceinline__ void walk_backward16(const BArgs& p, RMem<K>& s, cons
 
 }  // namespace w16
 
-template <typename TIn, int K>
+template <typename TIn, int K, int NB>
 __global__ __launch_bounds__(NTP) void recur16_kernel(const BArgs p) {
-  __shared__ w16::Mem<K> sm;
-  const ScanUnit su = scan_unit<2>(p.cu, p.T, p.B, p.H, p.nv, blockIdx.x);
-  const int bi = su.bi, hi = su.hi, vs = su.vs;
+  __shared__ w16::Mem<K, NB> sm;
+  const ScanUnit su = scan_unit<2>(p.cu, p.T, p.B, p.H, p.nv / NB, blockIdx.x);
+  const int bi = su.bi, hi = su.hi, v0 = su.vs * NB * BV;
   const bool backward = su.dir != 0;
   const RowSpan rs = row_span(p.cu, p.T, bi);
   const int64_t slot0 = p.cu ? rs.t0 / C + bi : (int64_t)bi * p.nchmax;
-  if (backward) w16::walk_backward16<TIn, K>(p, sm.r, rs, bi, hi, vs * BV, slot0);
-  else w16::walk_forward16<TIn, K>(p, sm.f, rs, bi, hi, vs * BV, slot0);
+  if (backward) w16::walk_backward16<TIn, K, NB>(p, sm.r, rs, bi, hi, v0, slot0);
+  else w16::walk_forward16<TIn, K, NB>(p, sm.f, rs, bi, hi, v0, slot0);
 }
 
 // ---------------------------------------------------------------------------
@@ -1657,6 +1802,30 @@ inline Layout layout(int B, int T, int H, int K, int V, int n_seq, bool w16) {
   return L;
 }
 
+// 32 columns a workgroup of the 16-bit walks instead of 16 (the same sums in
+// the same order) where that takes fewer rounds of the resident workgroups.
+// A walk then passes its k, q, T and P through LDS once for 32 columns, and
+// its chain's products come in pairs, independent of each other; but a
+// chunk's step takes longer, so as many rounds of them lose.  By LDS, two (16
+// columns) and two (32) share a CU at K = 128, three and two at 64, four and
+// three at 32.  Backward call, H = 16, bf16 / fp16, 16 -> 32 columns, K = V =
+// 128: one round of 512 (B2 T4096) 472 -> 517 / 433 -> 443 us, two to one
+// (B4) 885 -> 782 / 829 -> 716, eight to four (B16 T512) 516 -> 435 / 435 ->
+// 375.  K = 64, T2048: two to one (B1 H56 V128) 304 -> 276 / 281 -> 249,
+// two to two (B4 H17 V128) 357 -> 403 / 330 -> 343, three to two (B8 V128)
+// 623 -> 563 / 581 -> 500.  Packed sequences keep the 16: their longest one's
+// chain is the launch's tail, and the host does not know its length (3000
+// rows beside five of 3: 276 -> 356 us; seven of 3 to 2900 rows: 519 -> 510).
+template <int K>
+bool wide_walks(int V, int64_t units, bool packed) {
+  // LDS comes in blocks of 1280 bytes; 128 hold the range scales' maxima
+  constexpr int64_t lds = 160 * 1024, blk = 1280;
+  constexpr int64_t n1 = kCUs * (lds / ((sizeof(w16::Mem<K, 1>) + 128 + blk - 1) / blk * blk));
+  constexpr int64_t n2 = kCUs * (lds / ((sizeof(w16::Mem<K, 2>) + 128 + blk - 1) / blk * blk));
+  static_assert(n1 == kCUs * (K == 128 ? 2 : K == 64 ? 3 : 4) && n2 == kCUs * (K == 32 ? 3 : 2), "as measured");
+  return !packed && V % (2 * BV) == 0 && (units + n2 - 1) / n2 < (2 * units + n1 - 1) / n1;
+}
+
 template <typename TIn, int K>
 int launch_k(const BArgs& a, int64_t nrec, hipStream_t s) {
   if constexpr (!std::is_same<TIn, float>::value) {
@@ -1671,7 +1840,9 @@ int launch_k(const BArgs& a, int64_t nrec, hipStream_t s) {
     if (nrec > 0) hipLaunchKernelGGL((prep_kernel<TIn, K>), dim3((unsigned)nrec), dim3(NTP), 0, s, a);
   }
   if constexpr (!std::is_same<TIn, float>::value) {
-    if (a.w16) hipLaunchKernelGGL((recur16_kernel<TIn, K>), dim3(2 * a.units), dim3(NTP), 0, s, a);
+    if (a.w16 && wide_walks<K>(a.V, a.units, a.cu != nullptr))
+      hipLaunchKernelGGL((recur16_kernel<TIn, K, 2>), dim3(a.units), dim3(NTP), 0, s, a);
+    else if (a.w16) hipLaunchKernelGGL((recur16_kernel<TIn, K, 1>), dim3(2 * a.units), dim3(NTP), 0, s, a);
     else hipLaunchKernelGGL((recur_kernel<TIn, K>), dim3(2 * a.units), dim3(NTP), 0, s, a);
   } else {
     hipLaunchKernelGGL((recur_kernel<TIn, K>), dim3(2 * a.units), dim3(NTP), 0, s, a);

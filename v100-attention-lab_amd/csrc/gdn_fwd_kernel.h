@@ -199,6 +199,21 @@ __device__ __forceinline__ uint32_t block_max_bits(uint32_t m, uint32_t* red) {
   return m;
 }
 
+// Bits of the largest magnitude of a 16-byte piece of 8 bf16 columns at v
+// over rows r, r + rstep, ... (`rstride` bytes apart), eight loads in flight.
+__device__ __forceinline__ uint32_t column_absmax_bits(const char* v, int64_t rstride, int rows, int r, int rstep) {
+  uint32_t m = 0;
+  for (; r + 7 * rstep < rows; r += 8 * rstep) {
+    uint4 x[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) x[u] = *reinterpret_cast<const uint4*>(v + (int64_t)(r + u * rstep) * rstride);
+#pragma unroll
+    for (int u = 0; u < 8; ++u) m = max(m, bf16x8_absmax_bits(x[u]));
+  }
+  for (; r < rows; r += rstep) m = max(m, bf16x8_absmax_bits(*reinterpret_cast<const uint4*>(v + (int64_t)r * rstride)));
+  return m;
+}
+
 // Largest magnitude of v[rows x cols] (bf16, rows `rstride` bytes apart,
 // cols a multiple of 8, 16-byte aligned rows) and of h0[K x cols] (fp32,
 // element strides sk and sc; nullable), over the whole workgroup: every
@@ -209,27 +224,15 @@ __device__ __forceinline__ float slice_absmax_bf16(const char* v, int64_t rstrid
   const int tid = threadIdx.x, nthr = blockDim.x;
   uint32_t m = 0;
   const int pieces = cols >> 3;
-  auto piece_max = [](const uint4& x) { return bf16x8_absmax_bits(x); };
   if (nthr % pieces == 0) {
-    // a fixed 16-byte column piece per thread, rows nthr / pieces apart,
-    // eight loads in flight
-    const int rstep = nthr / pieces;
-    const char* const vc = v + (tid % pieces) * 16;
-    int r = tid / pieces;
-    for (; r + 7 * rstep < rows; r += 8 * rstep) {
-      uint4 x[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) x[u] = *reinterpret_cast<const uint4*>(vc + (int64_t)(r + u * rstep) * rstride);
-#pragma unroll
-      for (int u = 0; u < 8; ++u) m = max(m, piece_max(x[u]));
-    }
-    for (; r < rows; r += rstep) m = max(m, piece_max(*reinterpret_cast<const uint4*>(vc + (int64_t)r * rstride)));
+    // a fixed 16-byte column piece per thread, rows nthr / pieces apart
+    m = column_absmax_bits(v + (tid % pieces) * 16, rstride, rows, tid / pieces, nthr / pieces);
   } else {
     const int64_t nv = (int64_t)rows * pieces;
     for (int64_t i = tid; i < nv; i += nthr) {
       const int64_t r = i / pieces;
       const int c = (int)(i - r * pieces);
-      m = max(m, piece_max(*reinterpret_cast<const uint4*>(v + r * rstride + c * 16)));
+      m = max(m, bf16x8_absmax_bits(*reinterpret_cast<const uint4*>(v + r * rstride + c * 16)));
     }
   }
   return __uint_as_float(block_max_bits(max(m, state_absmax_bits(h0, sk, sc, K, cols)), red));
