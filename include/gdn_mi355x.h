@@ -137,9 +137,10 @@ typedef struct GdnFwdParams {
  *     sequence (at least one), so any workspace of at least
  *     gdn_fwd_workspace_size() bytes runs the call; a longer sequence runs
  *     as several segments, its state passing through final_state in fp32.
- *     C = 64 needs params->workspace.  At C = 32 sequences of at most 4 rows
- *     are walked step by step in fp32 (a dense batch of them in one launch,
- *     with or without a workspace).
+ *     C = 64 needs params->workspace.
+ *   - of these, C = 32 sequences of at most 4 rows are walked step by step in
+ *     fp32: a dense batch of them (T <= 4) in one launch that takes no
+ *     workspace (gdn_fwd_workspace_size is 0, params->workspace is not read).
  *   - C = 32 without a workspace (or GDN_FLAG_FUSED_KERNEL), fp32 inputs at
  *     C = 32, or K = 256 / GDN_FLAG_PHASED_KERNEL: one fused kernel, no
  *     workspace.
@@ -160,7 +161,8 @@ int gdn_fwd_launch(const GdnFwdParams* params, void* stream);
  *     and 3 KB + 2 C K bytes for bf16, which also carry the chunk's k rows
  *     in fp16).  If one chunk per sequence does not fit (fp16:
  *     B * H > 10922; bf16 at K = 128: B * H > 2978), the call runs on the
- *     fused kernel, which needs no workspace.
+ *     fused kernel, which needs no workspace.  Dense batches of at most 4
+ *     rows take no records and run as in gdn_fwd_launch whatever B * H is.
  *   - 64-row chunks: likewise in segments (records of 33 KB per chunk and
  *     head for 16-bit inputs, 66 KB for fp32 at K = 128).  If one chunk
  *     per sequence does not fit (B * H > 992 for 16-bit inputs), the call
@@ -179,10 +181,11 @@ int gdn_fwd_launch_noalloc(const GdnFwdParams* params, void* stream);
 int64_t gdn_fwd_scratch_bytes(void);
 
 /* Bytes of workspace gdn_fwd_launch needs for these params (0 for the fused
- * kernels; the records of a segment of at most 256 chunks per sequence for
- * 32-row chunks, at most 64 chunks for 64-row chunks; B = the number of
- * sequences when cu_seqlens is set); -1 if the shape is invalid.  No counterpart in the reference, whose Triton
- * launch needs none. */
+ * kernels and for dense 16-bit batches of at most 4 rows at C = 32; the
+ * records of a segment of at most 256 chunks per sequence for 32-row chunks,
+ * at most 64 chunks for 64-row chunks; B = the number of sequences when
+ * cu_seqlens is set); -1 if the shape is invalid.  No counterpart in the
+ * reference, whose Triton launch needs none. */
 int64_t gdn_fwd_workspace_size(const GdnFwdParams* params);
 
 /* The block_v the launcher picks when params->block_v == 0 (for logging and

@@ -510,3 +510,20 @@ def test_traffic_profile_tracks_sources(monkeypatch):
     monkeypatch.setattr(bench, "sources_digest", lambda config: "0" * 16)
     nbytes, note = bench.load_traffic("cfg2")
     assert nbytes is None and note.startswith("stale")
+
+
+@pytest.mark.parametrize("T", [1, 4])
+@pytest.mark.parametrize("dtype", [1, 2])
+@pytest.mark.parametrize("kw", [dict(workspace=0x100000), dict(workspace=0x100010), dict(workspace=None),
+                                dict(workspace=0x100000, workspace_bytes=4096), dict(B=4096)])
+def test_short_rows_take_any_workspace(lib, pkg, T, dtype, kw):
+    """Dense batches of at most 4 rows need no workspace: the size query says
+    0, and a launch with an empty, a small, an unaligned or no buffer (or from
+    gdn_fwd_launch_noalloc, whatever B * H is) passes every check."""
+    if torch.cuda.is_available():
+        pytest.skip("made-up addresses: only where nothing can be launched")
+    P = _params(pkg._lib, T=T, qkv_dtype=dtype, o_dtype=dtype, **kw)
+    assert lib.gdn_fwd_workspace_size(ctypes.byref(P)) == 0
+    for fn in (lib.gdn_fwd_launch, lib.gdn_fwd_launch_noalloc):
+        status = fn(ctypes.byref(P), None)
+        assert 0 < status < 1000, status    # HIP's own error: no device

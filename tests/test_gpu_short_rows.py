@@ -4,6 +4,8 @@ against the fp64 recurrence (the walk is fp32 throughout: 2e-6 on fp32 outputs,
 one rounding more on 16-bit ones), and bit-equal between packed and separate
 runs."""
 
+import ctypes
+
 import pytest
 import torch
 
@@ -62,3 +64,35 @@ def test_short_rows_packed(pkg, cuda, dtype, lens):
         assert torch.equal(o[:, a:b], so) and torch.equal(fs[i], sf[0]), i
         so, sf = pkg.gdn_fwd(*(t[:, a:b] for t in (q, k, v, g, beta)), h0[i:i + 1], max_segment_chunks=2)
         assert torch.equal(o2[:, a:b], so) and torch.equal(fs2[i], sf[0]), i
+
+
+@pytest.mark.parametrize("dtype,T,H", [(torch.float16, 1, 3), (torch.bfloat16, 4, 3), (torch.bfloat16, 2, 3000)])
+def test_short_rows_workspace(pkg, cuda, dtype, T, H):
+    """The C entry points with no workspace, an empty one, an unaligned one and
+    one of a few bytes, and gdn_fwd_launch_noalloc (3000 bf16 heads: more
+    records than its array holds), all give gdn_fwd's bits."""
+    L, B, K, V = pkg._lib, 1, 128, 16
+    lib = L.load_library()
+    q, k, v, g, beta, h0 = (t.to(cuda) for t in _inputs(B, T, H, K, V, dtype, seed=T))
+    want = pkg.gdn_fwd(q, k, v, g, beta, h0)
+    ws = torch.empty(1024, dtype=torch.uint8, device=cuda)
+    P = L.GdnFwdParams()
+    code = {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}
+    for n, t in (("q", q), ("k", k), ("v", v), ("g", g), ("beta", beta), ("h0", h0)):
+        setattr(P, n, t.data_ptr())
+        getattr(P, f"{n}_stride")[:] = t.stride() if n in ("g", "beta", "h0") else t.stride()[:3]
+    P.o_stride[:], P.fs_stride[:] = v.stride()[:3], h0.stride()
+    P.B, P.T, P.H, P.K, P.V, P.scale, P.chunk_size = B, T, H, K, V, 1.0, 32
+    P.qkv_dtype = P.o_dtype = code[dtype]
+    P.g_dtype, P.beta_dtype = code[g.dtype], code[beta.dtype]
+    assert lib.gdn_fwd_workspace_size(ctypes.byref(P)) == 0
+    for fn, ptr, nbytes in ((lib.gdn_fwd_launch, None, 0), (lib.gdn_fwd_launch, ws.data_ptr(), 0),
+                            (lib.gdn_fwd_launch, ws.data_ptr() + 16, 0), (lib.gdn_fwd_launch, ws.data_ptr(), 512),
+                            (lib.gdn_fwd_launch_noalloc, None, 0)):
+        o, fs = torch.full_like(v, float("nan")), torch.full_like(h0, float("nan"))
+        P.o, P.final_state, P.workspace, P.workspace_bytes = o.data_ptr(), fs.data_ptr(), ptr, nbytes
+        print(f"[short] {dtype} T={T} H={H} {fn.__name__} workspace {nbytes}", flush=True)
+        rc = fn(ctypes.byref(P), torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        assert rc == 0, L.status_string(rc)
+        assert torch.equal(o, want[0]) and torch.equal(fs, want[1])

@@ -128,7 +128,13 @@ static int launch_impl(const GdnFwdParams& P, hipStream_t s, int64_t scratch_byt
   }
   const long long units = (long long)P.B * P.H * (P.V / bv);
   if (units > 0x7fffffffLL) return GDN_ERR_BAD_SHAPE;
-  bool scan32 = uses_scan32(P, bv) && (scratch_bytes > 0 || P.workspace != nullptr || scan32_short(P));
+  if (uses_scan32(P, bv) && scan32_short(P)) {
+    // walked step by step, no records: params->workspace is not looked at (a
+    // caller may pass what it keeps for other calls, or an empty buffer)
+    (void)hipGetLastError();
+    return scan32_launch(P, bv, 1, s);
+  }
+  bool scan32 = uses_scan32(P, bv) && (scratch_bytes > 0 || P.workspace != nullptr);
   if (scratch_bytes > 0 && P.T > 0) {
     // The static scratch must hold one chunk's records per sequence and
     // head (longer sequences run in segments).  Where it cannot, the call
@@ -165,7 +171,7 @@ static int launch_impl(const GdnFwdParams& P, hipStream_t s, int64_t scratch_byt
   if (scan32) {
     // segment length: as many chunks per sequence as the workspace holds
     const int64_t per_chunk = (int64_t)P.B * P.H * scan32_record_bytes(P.qkv_dtype, P.K);
-    const int64_t L = W.workspace == nullptr ? 1 : W.workspace_bytes / per_chunk;  // none: short sequences
+    const int64_t L = W.workspace_bytes / per_chunk;
     if (P.T > 0 && (reinterpret_cast<uintptr_t>(W.workspace) % 256 != 0 || L < 1)) return GDN_ERR_WORKSPACE;
     return scan32_launch(W, bv, (int)(L < 1 ? 1 : L < 0x7fffffff ? L : 0x7fffffff), s);
   }
