@@ -527,3 +527,21 @@ def test_short_rows_take_any_workspace(lib, pkg, T, dtype, kw):
     for fn in (lib.gdn_fwd_launch, lib.gdn_fwd_launch_noalloc):
         status = fn(ctypes.byref(P), None)
         assert 0 < status < 1000, status    # HIP's own error: no device
+
+
+@pytest.mark.parametrize("bad,msg", [(lambda c: c.cpu(), "must be on"), (lambda c: c.double(), "int64 or int32"),
+                                     (lambda c: c[:1], "1-D"), (lambda c: c[None], "1-D")])
+def test_backward_checks_saved_offsets(pkg, bad, msg):
+    """Offsets that come out of a saved-tensor hook on another device, in
+    another type or shape are refused before a kernel gets their address."""
+    meta = lambda *s, **kw: torch.empty(*s, device="meta", **kw)
+    q = meta(1, 64, 2, 64, dtype=torch.float16)
+    v = meta(1, 64, 2, 32, dtype=torch.float16)
+    cu = bad(torch.empty(3, dtype=torch.int64) if msg == "must be on" else meta(3, dtype=torch.int64))
+
+    class Ctx:
+        saved_tensors = (q, q, v, meta(1, 64, 2), meta(1, 64, 2), None, cu)
+        scale, fs_vk, o_hf, needs_input_grad = 1.0, False, False, [True] * 15
+
+    with pytest.raises(ValueError, match="cu_seqlens.*" + msg):
+        pkg.ops._GdnFunction.backward(Ctx, v, meta(2, 2, 64, 32))

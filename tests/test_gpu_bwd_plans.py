@@ -47,3 +47,14 @@ def test_packed_autograd_offsets(pkg, cuda, cdtype):
     want = pkg.gdn_bwd(q, k, v, g, beta, None, do, torch.zeros(3, 2, 64, 32, device=cuda), cu_seqlens=cu, need_dh0=False)
     for a, b in zip(got, want):
         assert torch.equal(a, b)
+
+
+def test_packed_autograd_moved_offsets(pkg, cuda):
+    """Saved-tensor hooks that hand the offsets back on the host: refused."""
+    q, k, v, g, beta, _, do, _ = _inputs(cuda, seed=3)
+    cu = torch.tensor([0, 3, 40, 70], dtype=torch.int64, device=cuda)
+    leaves = [t.clone().requires_grad_(True) for t in (q, k, v, g, beta)]
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, lambda t: t.cpu() if t.dtype == torch.int64 else t):
+        o, _ = pkg.chunk_gated_delta_rule(*leaves, cu_seqlens=cu)
+    with pytest.raises(ValueError, match="cu_seqlens must be on"):
+        torch.autograd.grad(o, leaves, do)

@@ -210,22 +210,30 @@ def _make_plan(q, k, v, g, beta, h0, scale, chunk_size, block_v, output_dtype, k
     return plan
 
 
-def _check_cu_seqlens(cu, T, dev):
-    """Validates FLA-style packed-sequence offsets; returns (int64 tensor, N).
-    Reads the offsets on the host (one small copy), as FLA's own varlen
-    preparation does."""
+def _offsets(cu, dev):
+    """Packed-sequence offsets as the kernels read them: a contiguous int64
+    tensor on dev.  Returns (tensor, N); the values are not read (the kernels
+    clamp them to the rows they have)."""
     if not isinstance(cu, torch.Tensor) or cu.dim() != 1 or cu.numel() < 2:
         raise ValueError("cu_seqlens must be a 1-D tensor of N + 1 row offsets (N >= 1)")
     if cu.dtype not in (torch.int64, torch.int32):
         raise ValueError(f"cu_seqlens must be int64 or int32, got {cu.dtype}")
     if cu.device != dev:
         raise ValueError(f"cu_seqlens must be on {dev}, got {cu.device}")
+    if cu.dtype != torch.int64 or not cu.is_contiguous():
+        cu = cu.to(torch.int64).contiguous()
+    return cu, cu.numel() - 1
+
+
+def _check_cu_seqlens(cu, T, dev):
+    """Validates FLA-style packed-sequence offsets; returns (int64 tensor, N).
+    Reads the offsets on the host (one small copy), as FLA's own varlen
+    preparation does."""
+    cu, n_seq = _offsets(cu, dev)
     c = cu.tolist()
     if c[0] != 0 or c[-1] != T or any(b < a for a, b in zip(c, c[1:])):
         raise ValueError(f"cu_seqlens must rise from 0 to T={T} without decreasing, got {c}")
-    if cu.dtype != torch.int64 or not cu.is_contiguous():
-        cu = cu.to(torch.int64).contiguous()
-    return cu, len(c) - 1
+    return cu, n_seq
 
 
 def _run(q, k, v, g, beta, h0, scale, chunk_size, block_v, output_dtype, kernel, fs_vk,
@@ -690,11 +698,10 @@ class _GdnFunction(torch.autograd.Function):
         need_dh0 = h0 is not None and ctx.needs_input_grad[5]
         n_seq = None
         if cu is not None:
-            # checked by the forward (a second read of the offsets would make
-            # the host wait for the device once more)
-            n_seq = cu.numel() - 1
-            if cu.dtype != torch.int64 or not cu.is_contiguous():
-                cu = cu.to(torch.int64).contiguous()
+            # the values were checked by the forward (a second read of them
+            # would make the host wait for the device once more); where the
+            # tensor lives was not: saved-tensor hooks may hand back another
+            cu, n_seq = _offsets(cu, q.device)
         dq, dk, dv, dg, dbeta, dh0 = _run_bwd(q, k, v, g, beta, h0, do_bthv, dfs_kv, ctx.scale, cu, n_seq,
                                               need_dh0)
         return dq, dk, dv, dg, dbeta, dh0, None, None, None, None, None, None, None, None, None
