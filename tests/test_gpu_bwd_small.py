@@ -1,0 +1,72 @@
+"""GPU tests of the 16-bit backward where gradients, rows or inputs are far
+smaller than the largest of their sequence: each output's rows stay within the
+bound of their own magnitude (2-norm), against reverse-mode differentiation of
+the fp64 recurrence."""
+
+import pytest
+import torch
+
+from oracle import gdn_oracle as ref
+
+pytestmark = pytest.mark.gpu
+
+# one rounding to the storage dtype
+EPS = {torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}
+NAMES = ("dq", "dk", "dv", "dg", "dbeta", "dh0")
+
+
+def _inputs(T, H, K, V, dtype, seed, gate=1.0):
+    gen = torch.Generator().manual_seed(seed)
+    n = lambda *s: torch.randn(*s, generator=gen)
+    return {"q": ref.l2norm(n(1, T, H, K)), "k": ref.l2norm(n(1, T, H, K)), "v": n(1, T, H, V),
+            "g": gate * torch.nn.functional.logsigmoid(n(1, T, H)), "beta": torch.sigmoid(n(1, T, H)),
+            "h0": 0.1 * n(1, H, K, V), "do": n(1, T, H, V), "dfs": n(1, H, K, V)}
+
+
+def _grads(pkg, dev, x, dtype, scale):
+    x = {n: t.to(dtype) if n in ("q", "k", "v", "do") else t for n, t in x.items()}
+    d = {n: t.to(dev) for n, t in x.items()}
+    got = pkg.gdn_bwd(d["q"], d["k"], d["v"], d["g"], d["beta"], d["h0"], d["do"], d["dfs"], scale=scale)
+    torch.cuda.synchronize()
+    dq, dk, dv, dbeta, dg, dh0 = ref.recurrent_grads(x["q"], x["k"], x["v"], x["beta"], x["g"], x["h0"], x["do"],
+                                                     x["dfs"], scale=scale)
+    return dict(zip(NAMES, (t.cpu().double() for t in got))), dict(zip(NAMES, (dq, dk, dv, dg, dbeta, dh0)))
+
+
+def _err(got, want, rows=slice(None)):
+    """Relative 2-norm error over some rows."""
+    a, b = got[:, rows], want[:, rows]
+    return ((a - b).norm() / b.norm()).item()
+
+
+@pytest.mark.parametrize("K,V", [(128, 64), (64, 48), (32, 32)])
+def test_small_du(pkg, cuda, K, V):
+    """bf16 dO near 2^-14 beside a final state's gradient near 1, a small scale
+    and gates that leave each row to itself: du of the first chunk is near
+    2^-20 of the walk's unit, and dv = beta T^T du keeps its own precision.
+    Bound: one rounding, and 2^-10 for dO's elements below 2^-17 (subnormal in
+    fp16) and P (entries near 2^-4 to 2^-25)."""
+    dtype = torch.bfloat16
+    x = _inputs(96, 2, K, V, dtype, seed=K + V, gate=20.0)
+    x["do"] *= 2.0 ** -14
+    print(f"[small] du {dtype} K={K} V={V}", flush=True)
+    got, want = _grads(pkg, cuda, x, dtype, scale=0.125)
+    err = _err(got["dv"], want["dv"], slice(0, 32))
+    print(f"  dv {err:.2e}", flush=True)
+    assert err <= EPS[dtype] + 2.0 ** -10
+
+
+@pytest.mark.parametrize("K,V", [(128, 48), (128, 96), (64, 64)])
+def test_small_gradients_f16(pkg, cuda, K, V):
+    """fp16 gradients near 2^-13 (the walks do not shift fp16): dbeta, an fp32
+    output.  Bound: 2^-10, of which the carried state gradient (an fp16 pair to
+    2^-25, entries near 2^-14) is half."""
+    dtype = torch.float16
+    x = _inputs(300, 4, K, V, dtype, seed=5, gate=0.3)
+    x["do"] *= 2.0 ** -13
+    x["dfs"] *= 2.0 ** -13
+    print(f"[small] {dtype} K={K} V={V}", flush=True)
+    got, want = _grads(pkg, cuda, x, dtype, scale=0.3)
+    err = _err(got["dbeta"], want["dbeta"])
+    print(f"  dbeta {err:.2e}", flush=True)
+    assert err <= 2.0 ** -10

@@ -363,7 +363,7 @@ __global__ __launch_bounds__(256) void prep16_kernel(const BArgs p, int64_t nrec
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         f16 hh, ll;
-        tiles16::split_f16(xc[j + i], hh, ll);
+        tiles16::split_f16_up(xc[j + i], hh, ll);
         h[i] = hh;
         l[i] = ll;
       }
@@ -845,7 +845,7 @@ template <int K, int NB>
 struct alignas(16) FMem {
   static constexpr int W = NB * BV;
   f16 sh[W * LDP<K, NB>], sl[W * LDP<K, NB>];    // S^T
-  f16 yh[W * LDP<C, NB>], yl[W * LDP<C, NB>];    // (diag(beta) (V - diag(gam) K S))^T
+  f16 yh[W * LDP<C, NB>], yl[W * LDP<C, NB>];    // (diag(beta) (V - diag(gam) K S))^T, yl times 2^11
   f16 dh[W * LDP<C, NB>], dl[W * LDP<C, NB>];    // (diag(D) u)^T
   float uf[C][W];                    // u rows, on their way to uu
   FIn<K, NB> in[3];
@@ -872,7 +872,7 @@ struct alignas(16) RMem {
   static constexpr int W = NB * BV, NI1 = NB == 1 ? 2 : 1;
   f16 sh[W * LDP<K, NB>], sl[W * LDP<K, NB>];    // dS'^T
   f16 gh[W * LDP<C, NB>], gl[W * LDP<C, NB>];    // (diag(gam) dO)^T
-  f16 uh[W * LDP<C, NB>], ul[W * LDP<C, NB>];    // du^T
+  f16 uh[W * LDP<C, NB>], ul[W * LDP<C, NB>];    // du^T, ul times 2^11
   f16 zh[W * LDP<C, NB>], zl[W * LDP<C, NB>];    // (diag(beta gam) T^T du)^T
   float duf[C][W];                   // T^T du rows, on their way to du
   RIn<K> in[2];
@@ -1050,7 +1050,7 @@ __device__ __forceinline__ void walk_forward16(const BArgs& p, FMem<K, NB>& s, c
         float y[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) y[i] = in.gv[3][t + i] * (vv[i] - in.gv[1][t + i] * ak[cb][i]);
-        store_pair4(s.yh + poff<C, NB>(BV * cb + r, t), s.yl + poff<C, NB>(BV * cb + r, t), y);
+        store_pair4_up(s.yh + poff<C, NB>(BV * cb + r, t), s.yl + poff<C, NB>(BV * cb + r, t), y);
       }
     } else if (issuer && c + 2 < nch) {
       fetch(c + 2, b2);
@@ -1067,14 +1067,15 @@ __device__ __forceinline__ void walk_forward16(const BArgs& p, FMem<K, NB>& s, c
       const f16x8 tl = frag8_s<C>(in.tl, um0 + r, 8 * kq);
 #pragma unroll
       for (int cb = 0; cb < NB; ++cb) {
-        f32x4 au = {0.f, 0.f, 0.f, 0.f};
+        f32x4 au = {0.f, 0.f, 0.f, 0.f}, al = {0.f, 0.f, 0.f, 0.f};
         const f16x8 yh = yhs[cb];
         au = __builtin_amdgcn_mfma_f32_16x16x32_f16(th, yh, au, 0, 0, 0);
-        au = __builtin_amdgcn_mfma_f32_16x16x32_f16(th, pfrag8<C, NB>(s.yl, BV * cb + r, 8 * kq), au, 0, 0, 0);
-        au = __builtin_amdgcn_mfma_f32_16x16x32_f16(tl, yh, au, 0, 0, 0);
+        al = __builtin_amdgcn_mfma_f32_16x16x32_f16(th, pfrag8<C, NB>(s.yl, BV * cb + r, 8 * kq), al, 0, 0, 0);
+        al = __builtin_amdgcn_mfma_f32_16x16x32_f16(tl, yh, al, 0, 0, 0);
         float du[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
+          au[i] = __builtin_fmaf(kLowDown, al[i], au[i]);
           du[i] = in.gv[2][t + i] * au[i];
           s.uf[t + i][BV * cb + r] = au[i] * rsc[cb].fs;
         }
@@ -1252,7 +1253,7 @@ __device__ __forceinline__ void walk_backward16(const BArgs& p, RMem<K, NB>& s, 
         for (int i = 0; i < 4; ++i) {
           du[i] = scale * a1[cb][i] + in.gv[2][t + i] * a2[cb][i];
         }
-        store_pair4(s.uh + poff<C, NB>(BV * cb + r, t), s.ul + poff<C, NB>(BV * cb + r, t), du);
+        store_pair4_up(s.uh + poff<C, NB>(BV * cb + r, t), s.ul + poff<C, NB>(BV * cb + r, t), du);
       }
       if (c >= 1) fetch(c - 1);
     } else {
@@ -1306,13 +1307,14 @@ __device__ __forceinline__ void walk_backward16(const BArgs& p, RMem<K, NB>& s, 
 #pragma unroll
       for (int cb = 0; cb < NB; ++cb) {
         const f16x8 uh = pfrag8<C, NB>(s.uh, BV * cb + r, 8 * kq);
-        f32x4 az = {0.f, 0.f, 0.f, 0.f};
+        f32x4 az = {0.f, 0.f, 0.f, 0.f}, al = {0.f, 0.f, 0.f, 0.f};
         az = __builtin_amdgcn_mfma_f32_16x16x32_f16(tth, uh, az, 0, 0, 0);
-        az = __builtin_amdgcn_mfma_f32_16x16x32_f16(tth, pfrag8<C, NB>(s.ul, BV * cb + r, 8 * kq), az, 0, 0, 0);
-        az = __builtin_amdgcn_mfma_f32_16x16x32_f16(ttl, uh, az, 0, 0, 0);
+        al = __builtin_amdgcn_mfma_f32_16x16x32_f16(tth, pfrag8<C, NB>(s.ul, BV * cb + r, 8 * kq), al, 0, 0, 0);
+        al = __builtin_amdgcn_mfma_f32_16x16x32_f16(ttl, uh, al, 0, 0, 0);
         float z[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
+          az[i] = __builtin_fmaf(kLowDown, al[i], az[i]);
           z[i] = in.gv[1][t + i] * in.gv[3][t + i] * az[i];
           s.duf[t + i][BV * cb + r] = az[i] * rsd[cb].fs;
         }

@@ -73,7 +73,7 @@ struct RecT {
   static constexpr int SIZE = G + 4 * C;
 };
 // The same chunk's operands of the 16-bit recurrences, in halves: T and P as
-// [C][C], each an fp16 pair hi + lo.
+// [C][C], each an fp16 pair hi + lo (T's low half times 2^11, split_f16_up).
 struct Rec16 {
   static constexpr int TH = 0, TL = C * C, PH = 2 * C * C, PL = 3 * C * C;
   static constexpr int SIZE = 4 * C * C;

@@ -41,6 +41,24 @@ __device__ __forceinline__ void store_pair4(f16* hi, f16* lo, const float (&x)[4
   *reinterpret_cast<f16x4*>(lo) = f16x4{l[0], l[1], l[2], l[3]};
 }
 
+// The same with the low half times 2^11 (kLowUp): a value below 2^-14, whose
+// hi half is subnormal, keeps what it rounds off (to 2^-36 instead of 2^-25),
+// and no low half overflows (it is at most 2^4 before).  Products of a low half
+// are summed apart and take kLowDown.
+constexpr float kLowUp = 2048.f, kLowDown = 1.f / 2048.f;
+__device__ __forceinline__ void split_f16_up(float x, f16& hi, f16& lo) {
+  x = pin(x);
+  hi = (f16)x;
+  lo = (f16)((x - (float)hi) * kLowUp);
+}
+__device__ __forceinline__ void store_pair4_up(f16* hi, f16* lo, const float (&x)[4]) {
+  f16 h[4], l[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) split_f16_up(x[i], h[i], l[i]);
+  *reinterpret_cast<f16x4*>(hi) = f16x4{h[0], h[1], h[2], h[3]};
+  *reinterpret_cast<f16x4*>(lo) = f16x4{l[0], l[1], l[2], l[3]};
+}
+
 // Row m0 + r of X^T, contraction indices t0 + 8 kq .. t0 + 8 kq + 7, from
 // row-major X in LDS by two ds_read_b64_tr_b16: in each group of 16 lanes,
 // lane i receives as element j halfword i % 4 of the 8 bytes addressed by
