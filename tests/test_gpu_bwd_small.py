@@ -70,3 +70,40 @@ def test_small_gradients_f16(pkg, cuda, K, V):
     err = _err(got["dbeta"], want["dbeta"])
     print(f"  dbeta {err:.2e}", flush=True)
     assert err <= 2.0 ** -10
+
+
+@pytest.mark.parametrize("K,V", [(128, 128), (64, 128), (128, 48), (32, 80)])
+@pytest.mark.parametrize("p", [14, 18, 22])
+def test_small_do(pkg, cuda, K, V, p):
+    """bf16 dO 2^-p below a final state's gradient near 1, gates near 1 a row:
+    dq depends on dO alone and keeps its own precision wherever dO lies in
+    the walk's unit (one rounding of each element, 2^-10 for the fp16 states)."""
+    dtype = torch.bfloat16
+    x = _inputs(96, 2, K, V, dtype, seed=K + V + p, gate=0.3)
+    x["do"] *= 2.0 ** -p
+    print(f"[small] do 2^-{p} K={K} V={V}", flush=True)
+    got, want = _grads(pkg, cuda, x, dtype, scale=0.3)
+    err = _err(got["dq"], want["dq"])
+    print(f"  dq {err:.2e}", flush=True)
+    assert err <= EPS[dtype] + 2.0 ** -10
+
+
+@pytest.mark.parametrize("K,V", [(128, 128), (64, 128), (32, 64)])
+@pytest.mark.parametrize("p", [10])
+def test_small_do_rows(pkg, cuda, K, V, p):
+    """bf16: most rows of dO 2^-p below every seventh: dq of every row keeps the
+    bound of its own magnitude (as above).  Slices of different range, too."""
+    dtype = torch.bfloat16
+    x = _inputs(70, 2, K, V, dtype, seed=K + V + p, gate=0.3)
+    for spread in (0, 3, 9):
+        y = dict(x)
+        y["do"] = x["do"] * torch.where(torch.arange(70) % 7 == 0, 1.0, 2.0 ** -p).view(1, -1, 1, 1)
+        for n in ("v", "h0", "do", "dfs"):
+            y[n] = y[n].clone()
+            y[n][..., 16:32] *= 2.0 ** (6 + spread)    # out of the range that is left as it is
+        print(f"[small] rows 2^-{p} K={K} V={V} spread {spread}", flush=True)
+        got, want = _grads(pkg, cuda, y, dtype, scale=0.3)
+        a, b = got["dq"], want["dq"]
+        err = ((a - b).norm(dim=-1) / b.norm(dim=-1)).max().item()
+        print(f"  dq {err:.2e}", flush=True)
+        assert err <= EPS[dtype] + 2.0 ** -10

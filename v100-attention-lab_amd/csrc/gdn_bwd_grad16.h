@@ -82,12 +82,26 @@ __device__ __forceinline__ float max_wave(float x) {
   x = fmaxf(x, dpp_ror<0x121>(x));
   return reduce_groups(x, [](float a, float b) { return fmaxf(a, b); });
 }
-// Sum over the 8 lanes 8 j .. 8 j + 7 (DPP row_half_mirror, quad_perm).
+// Sum (maximum) over the 8 lanes 8 j .. 8 j + 7 (DPP row_half_mirror, quad_perm).
 __device__ __forceinline__ float sum8(float x) {
   x += dpp_ror<0x141>(x);
   x += dpp_ror<0x4e>(x);
   x += dpp_ror<0xb1>(x);
   return x;
+}
+__device__ __forceinline__ float max8(float x) {
+  x = fmaxf(x, dpp_ror<0x141>(x));
+  x = fmaxf(x, dpp_ror<0x4e>(x));
+  x = fmaxf(x, dpp_ror<0xb1>(x));
+  return x;
+}
+
+// Exponent of the unit that puts a row of largest magnitude m near 2^13 (of
+// fp16's 2^16): what is 2^-27 of the row still keeps fp16's 11 bits.  Inf and
+// NaN: 0.
+__device__ __forceinline__ int row_unit(float m) {
+  const int e = (int)((__float_as_uint(m) >> 23) & 255) - 127;
+  return e == 128 ? 0 : max(e, -120) - 13;
 }
 
 // Exponent of |m| (0 for zero; at most 100, also for inf and NaN).
@@ -122,6 +136,7 @@ struct alignas(16) GradMem {
   float am[3][16];          // row sums of dA M KK
   float dgc[NW];
   float mx[6];              // largest magnitude of each C x C tile
+  int er[2][3][C];          // row units of dO, z, u (of a group of V steps: double-buffered)
 };
 
 // One workgroup of K / 32 waves per (chunk, head): wave w owns 32 keys of the
@@ -137,11 +152,16 @@ struct alignas(16) GradMem {
 // fp16 states of bf16 inputs are in their slices' shifted units (2^eS, 2^eD
 // take S and dS' back): u and z, dO are brought to the same units.  Where the
 // slices' 2^(eS + eD) lie within a factor of 16, the ratio to the largest
-// goes into z, dO and dS'; else (SLOW) each slice's products are summed by
-// themselves and added in fp32 in true units.
+// goes into z, dO and (for u dS'^T, where they differ: spread) u; else (SLOW)
+// each slice's products are summed by themselves and added in fp32 in true
+// units.
+// Each row of z, u and bf16 dO is then taken to a unit of its own (row_unit,
+// from the rows in registers, before they are staged), which leaves with the
+// accumulators: a row far below the largest of its sequence keeps its digits.
+// V beyond NW steps: a group of steps raises the units of the one before.
 template <typename TIn, int K, bool SLOW>
 __device__ __forceinline__ void grad16_chunk(const BArgs& p, GradMem<K>& s, const RowSpan& rs, int c, int hi,
-                                             int64_t slot, int64_t sclb, int emax) {
+                                             int64_t slot, int64_t sclb, int emax, bool spread) {
   constexpr bool SHIFT = std::is_same<TIn, bf16_t>::value;
   constexpr int NW = K / 32, MAXJ = (6 + NW - 1) / NW;
   constexpr int RING = GradMem<K>::RING;
@@ -159,10 +179,11 @@ __device__ __forceinline__ void grad16_chunk(const BArgs& p, GradMem<K>& s, cons
   float gate[NG];
 #pragma unroll
   for (int i = 0; i < NG; ++i) gate[i] = rec[RecT::G + ((tid + 64 * NW * i) & (4 * C - 1))];
-  // q, k rows of this wave's keys, held until after the V walk
-  const int64_t row[2] = {min(n, nval - 1), min(16 + n, nval - 1)};
+  // q, k rows of this wave's keys, for after the V walk (loaded behind its last
+  // step but one: held through the walk they put 16 more registers in scratch)
   u32x4 qk[2][2];
-  {
+  auto load_qk = [&]() __attribute__((always_inline)) {
+    const int64_t row[2] = {min(n, nval - 1), min(16 + n, nval - 1)};
     const TIn* const qp = static_cast<const TIn*>(p.q) + head_base(rs, hi, p.sq) + (int64_t)t0 * p.sq[1] + key0;
     const TIn* const kp = static_cast<const TIn*>(p.k) + head_base(rs, hi, p.sk) + (int64_t)t0 * p.sk[1] + key0;
 #pragma unroll
@@ -170,7 +191,7 @@ __device__ __forceinline__ void grad16_chunk(const BArgs& p, GradMem<K>& s, cons
       qk[0][tt] = *reinterpret_cast<const u32x4*>(qp + row[tt] * p.sq[1]);
       qk[1][tt] = *reinterpret_cast<const u32x4*>(kp + row[tt] * p.sk[1]);
     }
-  }
+  };
 
   // ---- a V step's rows: thread tid takes columns 4 (tid % 8) .. + 3 of rows
   // tid / 8 + 8 NW i (columns past V load column 0, rows past the chunk's end
@@ -249,13 +270,74 @@ __device__ __forceinline__ void grad16_chunk(const BArgs& p, GradMem<K>& s, cons
   // (3-5), job j on wave j % NW
   auto tile_t = [](int job) { return job % 3 == 0 ? 0 : 1; };
   auto tile_j = [](int job) { return job % 3 == 2 ? 1 : 0; };
+  // this thread's rows' units, of the V steps so far
+  int eo[NR], ez[NR], eu[NR];
+  // what takes step x's dO and z, and u, to the slice's unit
+  auto unit_z = [&](const Raw& x) __attribute__((always_inline)) {
+    return !SHIFT ? 0 : SLOW ? -exponent(x.fd) : exponent(x.fs) - emax;
+  };
+  auto unit_u = [&](const Raw& x) __attribute__((always_inline)) { return SHIFT ? -exponent(x.fs) : 0; };
+  auto row_units = [&](int s0, int par) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < NR; ++i) {
+      float mo = 0.f, mz = 0.f, mu = 0.f;
+      auto amax = [](const auto& x) __attribute__((always_inline)) {
+        return fmaxf(fmaxf(fabsf(x[0]), fabsf(x[1])), fmaxf(fabsf(x[2]), fabsf(x[3])));
+      };
+#pragma unroll
+      for (int j = 0; j < NW; ++j) {
+        if (s0 + j < ns) {
+          const Raw& x = raw[j];
+          if constexpr (SHIFT) {
+            const uint32_t m = max(bf16x2_absmax_bits(x.o[i][0]), bf16x2_absmax_bits(x.o[i][1]));
+            mo = fmaxf(mo, ldexpf(__uint_as_float(m), unit_z(x)));
+          }
+          mz = fmaxf(mz, ldexpf(amax(x.z[i]), unit_z(x)));
+          mu = fmaxf(mu, ldexpf(amax(x.u[i]), unit_u(x)));
+        }
+      }
+      const int a = SHIFT ? row_unit(max8(mo)) : 0, b = row_unit(max8(mz)), c = row_unit(max8(mu));
+      eo[i] = s0 > 0 ? max(eo[i], a) : a;
+      ez[i] = s0 > 0 ? max(ez[i], b) : b;
+      eu[i] = s0 > 0 ? max(eu[i], c) : c;
+      if ((tid & 7) == 0) {
+        const int t = r0 + 8 * NW * i;
+        s.er[par][0][t] = eo[i];
+        s.er[par][1][t] = ez[i];
+        s.er[par][2][t] = eu[i];
+      }
+    }
+  };
+  // the accumulators times 2^f(which, row) of their rows' units and 2^es (the
+  // C x C ones 2^ej)
+  auto rescale = [&](auto&& f, int es, int ej) __attribute__((always_inline)) {
+#pragma unroll
+    for (int tt = 0; tt < 2; ++tt) {
+      const int fo = f(0, 16 * tt + n) + es, fz = f(1, 16 * tt + n) + es, fu = f(2, 16 * tt + n) + es;
+#pragma unroll
+      for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          aQ[kt][tt][e] = ldexpf(aQ[kt][tt][e], fo);
+          aW[kt][tt][e] = ldexpf(aW[kt][tt][e], fz);
+          aK[kt][tt][e] = ldexpf(aK[kt][tt][e], fu);
+        }
+    }
+#pragma unroll
+    for (int job = 0; job < 6; ++job) {
+      if (job % NW == wave) {
+        const int fu = f(2, 16 * tile_j(job) + n) + ej;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          aJ[job / NW][e] = ldexpf(aJ[job / NW][e], f(job < 3 ? 0 : 1, 16 * tile_t(job) + 4 * g + e) + fu);
+      }
+    }
+  };
   // step st's rows as operands -> in[st & 1], dv = diag(beta) z and v.z
   auto stage = [&](const Raw& x, int st) __attribute__((always_inline)) {
     auto& in = s.in[st & 1];
     const int v = 32 * st + c4;
-    const int eS = SHIFT ? exponent(x.fs) : 0, eD = SHIFT ? exponent(x.fd) : 0;
-    // z and dO carry the slice's ratio to the largest unit
-    const int xz = SLOW ? -eD : eS - emax;
+    const int xz = unit_z(x), xu = unit_u(x);
 #pragma unroll
     for (int i = 0; i < NR; ++i) {
       const int t = r0 + 8 * NW * i;
@@ -277,14 +359,15 @@ __device__ __forceinline__ void grad16_chunk(const BArgs& p, GradMem<K>& s, cons
         unpack8<TIn>(ob, o);
         f16x4 h;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          z[e] = ldexpf(z[e], xz);
-          u[e] = ldexpf(u[e], -eS);
-          h[e] = (f16)ldexpf(o[e], xz);
-        }
+        for (int e = 0; e < 4; ++e) h[e] = (f16)ldexpf(o[e], xz - eo[i]);
         *reinterpret_cast<f16x4*>(&in.o[at]) = h;
       } else {
         *reinterpret_cast<u32x2*>(&in.o[at]) = ob;
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        z[e] = ldexpf(z[e], xz - ez[i]);
+        u[e] = ldexpf(u[e], xu - eu[i]);
       }
       tiles16::store_pair4(&in.uh[at], &in.ul[at], u);
       tiles16::store_pair4(&in.zh[at], &in.zl[at], z);
@@ -296,12 +379,15 @@ __device__ __forceinline__ void grad16_chunk(const BArgs& p, GradMem<K>& s, cons
     for (int sub = 0; sub < (SLOW ? 2 : 1); ++sub) {
       const bool use = 32 * st + 8 * g < V && (!SLOW || (g >> 1) == sub);
       // SLOW: the slice's unit, its products summed in fp32 in true units
-      const int unit = SLOW ? __builtin_amdgcn_readfirstlane(__shfl(eS + eD, 32 * sub, 64)) : 0;
-      auto add = [&](f32x4& acc, auto&& f) __attribute__((always_inline)) {
+      // (less row_unit's 2^13 a row: products of rows near its largest would
+      // leave fp32's range before the true ones do); else this lane's slice's
+      // ratio to the largest
+      const int unit = SLOW ? __builtin_amdgcn_readfirstlane(__shfl(eS + eD, 32 * sub, 64)) : SHIFT ? eS + eD - emax : 0;
+      auto add = [&](f32x4& acc, int rows, auto&& f) __attribute__((always_inline)) {
         if constexpr (SLOW) {
           const f32x4 x = f(zero4);
 #pragma unroll
-          for (int e = 0; e < 4; ++e) acc[e] += ldexpf(x[e], unit);
+          for (int e = 0; e < 4; ++e) acc[e] += ldexpf(x[e], unit - 13 * rows);
         } else {
           acc = f(acc);
         }
@@ -317,7 +403,6 @@ __device__ __forceinline__ void grad16_chunk(const BArgs& p, GradMem<K>& s, cons
         const f16x4 d0 = w16::read_tr4(d), d1 = w16::read_tr4(d + 128);
         sS[kt] = f16x8{a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], a1[2], a1[3]};
         sD[kt] = f16x8{d0[0], d0[1], d0[2], d0[3], d1[0], d1[1], d1[2], d1[3]};
-        if constexpr (SHIFT && !SLOW) sD[kt] *= (f16)ldexpf(1.f, eS + eD - emax);
         if constexpr (SLOW) {
           sS[kt] = use ? sS[kt] : f16x8{};
           sD[kt] = use ? sD[kt] : f16x8{};
@@ -339,37 +424,52 @@ __device__ __forceinline__ void grad16_chunk(const BArgs& p, GradMem<K>& s, cons
           uh[tt] = use ? uh[tt] : f16x8{};
           ul[tt] = use ? ul[tt] : f16x8{};
         }
+        // the ratio on u (its rows' units leave it the room)
+        f16x8 dh = uh[tt], dl = ul[tt];
+        if constexpr (SHIFT && !SLOW) {
+          if (spread) {
+            dh *= (f16)ldexpf(1.f, unit);
+            dl *= (f16)ldexpf(1.f, unit);
+          }
+        }
 #pragma unroll
         for (int kt = 0; kt < 2; ++kt) {
-          add(aW[kt][tt], [&](f32x4 x) { return mma(sS[kt], zl, mma(sS[kt], zh, x)); });
-          add(aQ[kt][tt], [&](f32x4 x) { return mma(sS[kt], of, x); });
-          add(aK[kt][tt], [&](f32x4 x) { return mma(sD[kt], ul[tt], mma(sD[kt], uh[tt], x)); });
+          add(aW[kt][tt], 1, [&](f32x4 x) { return mma(sS[kt], zl, mma(sS[kt], zh, x)); });
+          add(aQ[kt][tt], 1, [&](f32x4 x) { return mma(sS[kt], of, x); });
+          add(aK[kt][tt], 1, [&](f32x4 x) { return mma(sD[kt], dl, mma(sD[kt], dh, x)); });
         }
 #pragma unroll
         for (int job = 0; job < 6; ++job) {
           if (tile_t(job) == tt && job % NW == wave) {
             const int jt = tile_j(job);
-            if (job < 3) add(aJ[job / NW], [&](f32x4 x) { return mma(of, ul[jt], mma(of, uh[jt], x)); });
-            else add(aJ[job / NW], [&](f32x4 x) { return mma(zl, uh[jt], mma(zh, ul[jt], mma(zh, uh[jt], x))); });
+            if (job < 3) add(aJ[job / NW], 2, [&](f32x4 x) { return mma(of, ul[jt], mma(of, uh[jt], x)); });
+            else add(aJ[job / NW], 2, [&](f32x4 x) { return mma(zl, uh[jt], mma(zh, ul[jt], mma(zh, uh[jt], x))); });
           }
         }
       }
     }
   };
   w16::bar();  // the gates
-  int b = 0;
+  int b = 0, par = 0;
   for (int s0 = 0; s0 < ns; s0 += NW) {
+    par = (s0 / NW) & 1;
+    row_units(s0, par);
 #pragma unroll
     for (int i = 0; i < NW; ++i) {
       const int st = s0 + i;
       if (st < ns) {
         stage(raw[i], st);
         // this wave's copies of step st are in: only those of the steps
-        // after it may be in flight (4 each)
+        // after it may be in flight (4 each), or the 4 loads of q and k
         if (st + 2 < ns) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
-        else if (st + 1 < ns) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+        else if (ns > 1) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
         else w16::wait_dma();
         w16::bar();
+        // (the units of the group before are read before the barriers of this
+        // group's later steps, and overwritten after them)
+        if (st == max(ns - 2, 0)) load_qk();
+        if (i == 0 && s0 > 0)
+          rescale([&](int x, int t) { return s.er[par ^ 1][x][t] - s.er[par][x][t]; }, 0, 0);
         // the scales of this lane's operand columns (lanes 0 and 4 loaded
         // those of the step's two slices)
         const int eS = SHIFT ? __shfl(exponent(raw[i].fs), 2 * (g & 2), 64) : 0;
@@ -386,21 +486,10 @@ __device__ __forceinline__ void grad16_chunk(const BArgs& p, GradMem<K>& s, cons
     for (int i = 0; i < NW; ++i)
       if (s0 + NW + i < ns) load(raw[i], s0 + NW + i);
   }
-  if constexpr (SHIFT && !SLOW) {
-    // back to true units
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        aW[i >> 1][i & 1][e] = ldexpf(aW[i >> 1][i & 1][e], emax);
-        aQ[i >> 1][i & 1][e] = ldexpf(aQ[i >> 1][i & 1][e], emax);
-        aK[i >> 1][i & 1][e] = ldexpf(aK[i >> 1][i & 1][e], emax);
-      }
-#pragma unroll
-      for (int i = 0; i < MAXJ; ++i) aJ[i][e] = ldexpf(aJ[i][e], emax);
-    }
-    dgc = ldexpf(dgc, emax);
-  }
+  // back to true units (the slices' are in SLOW sums already)
+  rescale([&](int x, int t) { return s.er[par][x][t]; }, SLOW ? 13 : SHIFT ? emax : 0,
+          SLOW ? 26 : SHIFT ? emax : 0);
+  if constexpr (SHIFT && !SLOW) dgc = ldexpf(dgc, emax);
 
   // ---- q and k rows -> this wave's own ring, row dots
   f16* const qs = &s.st[wave][0][0][0];
@@ -453,10 +542,10 @@ __device__ __forceinline__ void grad16_chunk(const BArgs& p, GradMem<K>& s, cons
   }
   w16::bar();
 
-  // dQK and dKK leave as fp16 pairs in units 2^ey, 2^ez that put the largest
+  // dQK and dKK leave as fp16 pairs in units 2^eq, 2^ek that put the largest
   // entry of dO u^T, z u^T near 1: gradients of any size keep their pairs
-  const int ey = unit_exponent(scale * fmaxf(fmaxf(s.mx[0], s.mx[1]), s.mx[2]));
-  const int ez = unit_exponent(fmaxf(fmaxf(s.mx[3], s.mx[4]), s.mx[5]));
+  const int eq = unit_exponent(scale * fmaxf(fmaxf(s.mx[0], s.mx[1]), s.mx[2]));
+  const int ek = unit_exponent(fmaxf(fmaxf(s.mx[3], s.mx[4]), s.mx[5]));
 
   // ---- the C x C tiles: lane (n, g) holds rows t = 16 tt + 4 g + i, column
   // j = 16 jt + n
@@ -497,7 +586,7 @@ __device__ __forceinline__ void grad16_chunk(const BArgs& p, GradMem<K>& s, cons
       col = sum_groups(col);
       if (g == 0) s.cs[job][n] = col;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) x[i] = ldexpf(x[i], isq ? -ey : -ez);
+      for (int i = 0; i < 4; ++i) x[i] = ldexpf(x[i], isq ? -eq : -ek);
       tiles16::store_pair4(isq ? &s.m.yh[j][tb] : &s.m.zh[j][tb], isq ? &s.m.yl[j][tb] : &s.m.zl[j][tb], x);
       if (job % 3 == 1) {
         // the upper tile (rows 0-15, columns 16-31) is zero
@@ -573,8 +662,8 @@ __device__ __forceinline__ void grad16_chunk(const BArgs& p, GradMem<K>& s, cons
       e = mma(kT[kt], zcl, mma(kT[kt], zch, e));
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        dq[4 * kt + i] = ldexpf(a[i], ey) + scale * gam * aQ[kt][tt][i];
-        dk[4 * kt + i] = ldexpf(b[i], ey) + ldexpf(e[i], ez) + (D * aK[kt][tt][i] - bg * aW[kt][tt][i]);
+        dq[4 * kt + i] = ldexpf(a[i], eq) + scale * gam * aQ[kt][tt][i];
+        dk[4 * kt + i] = ldexpf(b[i], eq) + ldexpf(e[i], ek) + (D * aK[kt][tt][i] - bg * aW[kt][tt][i]);
       }
     }
     if (t < nval) {
@@ -609,12 +698,21 @@ __global__ __launch_bounds__(2 * K, 2) void grad16_kernel(const BArgs p) {
       up = max(up, __shfl_xor(up, o, 64));
     }
     const int emax = __builtin_amdgcn_readfirstlane(up);
-    if (__builtin_amdgcn_readfirstlane(up - lo) > 4)
-      grad16_chunk<TIn, K, true>(p, s, rs, c, hi, slot, sclb, emax);
-    else
-      grad16_chunk<TIn, K, false>(p, s, rs, c, hi, slot, sclb, emax);
+    const int spread = __builtin_amdgcn_readfirstlane(up - lo);
+    if (spread > 4) {
+      // the arguments (the kernel's first and only ones) by an address that the
+      // compiler cannot see through: reads that both branches share would
+      // be held in registers across either (with them the other branch kept 70
+      // registers in scratch: 323 -> 359 us, B4 T4096 H16 K = V = 128)
+      typedef const __attribute__((address_space(4))) BArgs KernArgs;
+      KernArgs* args = (KernArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+      asm volatile("" : "+s"(args));
+      grad16_chunk<TIn, K, true>(*(const BArgs*)args, s, rs, c, hi, slot, sclb, emax, true);
+    } else {
+      grad16_chunk<TIn, K, false>(p, s, rs, c, hi, slot, sclb, emax, spread > 0);
+    }
   } else {
-    grad16_chunk<TIn, K, false>(p, s, rs, c, hi, slot, sclb, 0);
+    grad16_chunk<TIn, K, false>(p, s, rs, c, hi, slot, sclb, 0, false);
   }
 }
 
