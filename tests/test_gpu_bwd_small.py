@@ -89,7 +89,7 @@ def test_small_do(pkg, cuda, K, V, p):
 
 
 @pytest.mark.parametrize("K,V", [(128, 128), (64, 128), (32, 64)])
-@pytest.mark.parametrize("p", [10])
+@pytest.mark.parametrize("p", [10, 17, 24])
 def test_small_do_rows(pkg, cuda, K, V, p):
     """bf16: most rows of dO 2^-p below every seventh: dq of every row keeps the
     bound of its own magnitude (as above).  Slices of different range, too."""

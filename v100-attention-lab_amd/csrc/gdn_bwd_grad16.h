@@ -96,18 +96,12 @@ __device__ __forceinline__ float max8(float x) {
   return x;
 }
 
-// Exponent of the unit that puts a row of largest magnitude m near 2^13 (of
-// fp16's 2^16): what is 2^-27 of the row still keeps fp16's 11 bits.  Inf and
-// NaN: 0.
-__device__ __forceinline__ int row_unit(float m) {
+// Exponent of the unit that puts values of largest magnitude m near 2^13 (of
+// fp16's 2^16): what is 2^-27 of the largest still keeps fp16's 11 bits.  Inf
+// and NaN: 0.
+__device__ __forceinline__ int unit_of(float m) {
   const int e = (int)((__float_as_uint(m) >> 23) & 255) - 127;
   return e == 128 ? 0 : max(e, -120) - 13;
-}
-
-// Exponent of |m| (0 for zero; at most 100, also for inf and NaN).
-__device__ __forceinline__ int unit_exponent(float m) {
-  const int e = (int)((__float_as_uint(m) >> 23) & 255) - 127;
-  return e == -127 ? 0 : min(e, 100);
 }
 
 template <int K>
@@ -135,7 +129,7 @@ struct alignas(16) GradMem {
   float rs[6][16], cs[6][16];  // row and column sums of the C x C tiles
   float am[3][16];          // row sums of dA M KK
   float dgc[NW];
-  float mx[6];              // largest magnitude of each C x C tile
+  float mx[6];              // largest magnitude of each tile of dQK, dKK
   int er[2][3][C];          // row units of dO, z, u (of a group of V steps: double-buffered)
 };
 
@@ -155,7 +149,7 @@ struct alignas(16) GradMem {
 // goes into z, dO and (for u dS'^T, where they differ: spread) u; else (SLOW)
 // each slice's products are summed by themselves and added in fp32 in true
 // units.
-// Each row of z, u and bf16 dO is then taken to a unit of its own (row_unit,
+// Each row of z, u and bf16 dO is then taken to a unit of its own (unit_of,
 // from the rows in registers, before they are staged), which leaves with the
 // accumulators: a row far below the largest of its sequence keeps its digits.
 // V beyond NW steps: a group of steps raises the units of the one before.
@@ -296,7 +290,7 @@ __device__ __forceinline__ void grad16_chunk(const BArgs& p, GradMem<K>& s, cons
           mu = fmaxf(mu, ldexpf(amax(x.u[i]), unit_u(x)));
         }
       }
-      const int a = SHIFT ? row_unit(max8(mo)) : 0, b = row_unit(max8(mz)), c = row_unit(max8(mu));
+      const int a = SHIFT ? unit_of(max8(mo)) : 0, b = unit_of(max8(mz)), c = unit_of(max8(mu));
       eo[i] = s0 > 0 ? max(eo[i], a) : a;
       ez[i] = s0 > 0 ? max(ez[i], b) : b;
       eu[i] = s0 > 0 ? max(eu[i], c) : c;
@@ -379,7 +373,7 @@ __device__ __forceinline__ void grad16_chunk(const BArgs& p, GradMem<K>& s, cons
     for (int sub = 0; sub < (SLOW ? 2 : 1); ++sub) {
       const bool use = 32 * st + 8 * g < V && (!SLOW || (g >> 1) == sub);
       // SLOW: the slice's unit, its products summed in fp32 in true units
-      // (less row_unit's 2^13 a row: products of rows near its largest would
+      // (less unit_of's 2^13 a row: products of rows near its largest would
       // leave fp32's range before the true ones do); else this lane's slice's
       // ratio to the largest
       const int unit = SLOW ? __builtin_amdgcn_readfirstlane(__shfl(eS + eD, 32 * sub, 64)) : SHIFT ? eS + eD - emax : 0;
@@ -535,17 +529,31 @@ __device__ __forceinline__ void grad16_chunk(const BArgs& p, GradMem<K>& s, cons
 #pragma unroll
   for (int job = 0; job < 6; ++job) {
     if (job % NW == wave) {
-      const f32x4 a = aJ[job / NW];
-      const float m = max_wave(fmaxf(fmaxf(fabsf(a[0]), fabsf(a[1])), fmaxf(fabsf(a[2]), fabsf(a[3]))));
+      // dO u^T -> dQK, z u^T -> dA o M (dKK = diag(beta) of it)
+      const int tb = 16 * tile_t(job) + 4 * g, j = 16 * tile_j(job) + n;
+      const f32x4 bt4 = *reinterpret_cast<const f32x4*>(&s.gt[0][tb]);
+      const f32x4 be4 = *reinterpret_cast<const f32x4*>(&s.gt[3][tb]);
+      const float bj = s.gt[0][j];
+      float m = 0.f;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int t = tb + i;
+        const float e = aJ[job / NW][i], d = expf(bt4[i] - bj);
+        const float x = job < 3 ? (j <= t ? scale * d * e : 0.f) : (j < t ? -e * d : 0.f);
+        aJ[job / NW][i] = x;
+        m = fmaxf(m, fabsf(job < 3 ? x : be4[i] * x));
+      }
+      m = max_wave(m);
       if (lane == 0) s.mx[job] = m;
     }
   }
   w16::bar();
 
-  // dQK and dKK leave as fp16 pairs in units 2^eq, 2^ek that put the largest
-  // entry of dO u^T, z u^T near 1: gradients of any size keep their pairs
-  const int eq = unit_exponent(scale * fmaxf(fmaxf(s.mx[0], s.mx[1]), s.mx[2]));
-  const int ek = unit_exponent(fmaxf(fmaxf(s.mx[3], s.mx[4]), s.mx[5]));
+  // dQK and dKK leave as fp16 pairs in units 2^eq, 2^ek of their largest entry:
+  // gradients of any size, and rows far below the chunk's largest, keep their
+  // digits
+  const int eq = unit_of(fmaxf(fmaxf(s.mx[0], s.mx[1]), s.mx[2]));
+  const int ek = unit_of(fmaxf(fmaxf(s.mx[3], s.mx[4]), s.mx[5]));
 
   // ---- the C x C tiles: lane (n, g) holds rows t = 16 tt + 4 g + i, column
   // j = 16 jt + n
@@ -559,26 +567,17 @@ __device__ __forceinline__ void grad16_chunk(const BArgs& p, GradMem<K>& s, cons
       for (int kb = 0; kb < K; kb += 32)
         kk = mma(w16::frag8_s<32>(&s.st[kb / 32][0][isq ? 0 : 1][0], 16 * tt + n, 8 * g),
                  w16::frag8_s<32>(&s.st[kb / 32][0][1][0], j, 8 * g), kk);
-      const f32x4 bt4 = *reinterpret_cast<const f32x4*>(&s.gt[0][tb]);
       const f32x4 be4 = *reinterpret_cast<const f32x4*>(&s.gt[3][tb]);
-      const float bj = s.gt[0][j];
       float x[4], col = 0.f;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const int t = tb + i;
-        const float e = aJ[job / NW][i];
-        float w;  // the tile's entry of db's row-minus-column sums
-        if (isq) {
-          const float m = j <= t ? expf(bt4[i] - bj) : 0.f;
-          x[i] = scale * m * e;
-          w = x[i] * kk[i];
-        } else {
-          const float dm = j < t ? -e * expf(bt4[i] - bj) : 0.f;  // dA o M
-          x[i] = be4[i] * dm;
-          w = x[i] * kk[i];
-          const float a = sum16(dm * kk[i]);
+        x[i] = aJ[job / NW][i];
+        if (!isq) {
+          const float a = sum16(x[i] * kk[i]);
           if (n == 0) s.am[job % 3][4 * g + i] = a;
+          x[i] *= be4[i];
         }
+        const float w = x[i] * kk[i];  // the tile's entry of db's row-minus-column sums
         col += w;
         const float r = sum16(w);
         if (n == 0) s.rs[job][4 * g + i] = r;
