@@ -107,3 +107,22 @@ def test_small_do_rows(pkg, cuda, K, V, p):
         err = ((a - b).norm(dim=-1) / b.norm(dim=-1)).max().item()
         print(f"  dq {err:.2e}", flush=True)
         assert err <= EPS[dtype] + 2.0 ** -10
+
+
+@pytest.mark.parametrize("which,p", [("q", 13), ("k", 20), ("k", 40)])
+@pytest.mark.parametrize("K", [128, 64, 32])
+def test_small_q_k(pkg, cuda, which, p, K):
+    """bf16 q or k near 2^-p in one chunk (what carries from chunk to chunk goes
+    through the walks, which take q and k as fp16 holds them, and P to 2^-25): dq
+    of small k, dk of small q keep the bound of their own magnitude."""
+    dtype = torch.bfloat16
+    x = _inputs(30, 2, K, 48, dtype, seed=K + p, gate=0.3)
+    x[which] *= 2.0 ** -p
+    x["h0"] *= 0.0
+    x["dfs"] *= 0.0
+    print(f"[small] {which} 2^-{p} K={K}", flush=True)
+    got, want = _grads(pkg, cuda, x, dtype, scale=0.3)
+    name = "dk" if which == "q" else "dq"
+    err = _err(got[name], want[name])
+    print(f"  {name} {err:.2e}", flush=True)
+    assert err <= EPS[dtype] + 2.0 ** -10

@@ -182,18 +182,6 @@ __global__ __launch_bounds__(NTP) void prep_kernel(const BArgs p) {
                         [&](int kk, int n) { return s.bt[kk] * s.gam[kk] * s.k[kk][n]; }));
 }
 
-// 16-bit q or k rows as MFMA operands: 8 elements (16 bytes) per lane, in
-// their own type (exact), on v_mfma_f32_16x16x32_f16 or _bf16.
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-template <typename TIn>
-__device__ __forceinline__ f32x4 mma16(const u32x4& a, const u32x4& b, const f32x4& acc) {
-  if constexpr (std::is_same<TIn, f16>::value)
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), acc, 0,
-                                                  0, 0);
-  else
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), acc,
-                                                   0, 0, 0);
-}
 // The prep of the 16-bit recurrences: one wave per two (chunk, head)
 // records, with no workgroup barrier.  Per record: the gates (a prefix sum
 // across lanes), K K^T and Q K^T on the 16-bit matrix cores (exact

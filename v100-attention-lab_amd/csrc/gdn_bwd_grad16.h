@@ -111,7 +111,7 @@ struct alignas(16) GradMem {
   static constexpr int LD = C + 8;
   // per wave: its 32 keys of S and dS' of a V step, as stored (32 state
   // columns x 32 keys); after the V walk, in [w][0], its keys of the q and k
-  // rows in fp16 (swz<32>)
+  // rows in their own type (swz<32>)
   f16 st[NW][RING][2][32 * 32];
   union {
     // a V step's operand rows (swz<32>), double-buffered
@@ -488,25 +488,33 @@ __device__ __forceinline__ void grad16_chunk(const BArgs& p, GradMem<K>& s, cons
   // ---- q and k rows -> this wave's own ring, row dots
   f16* const qs = &s.st[wave][0][0][0];
   f16* const ks = &s.st[wave][0][1][0];
+  int uq[2] = {0, 0};  // bf16: the units that take this wave's keys of q and k to fp16
+  if constexpr (SHIFT) {
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {
+      uint32_t a = 0;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) a = max(a, max(bf16x2_absmax_bits(qk[m][0][e]), bf16x2_absmax_bits(qk[m][1][e])));
+      uq[m] = __builtin_amdgcn_readfirstlane(unit_of(max_wave(__uint_as_float(a))));
+    }
+  }
 #pragma unroll
   for (int tt = 0; tt < 2; ++tt) {
     const int t = 16 * tt + n;
-    f16x8 x8[2];
+    float y[2][8];
 #pragma unroll
     for (int m = 0; m < 2; ++m) {
-      float y[8];
-      unpack16<TIn>(qk[m][tt], y);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) x8[m][e] = t < nval ? (f16)y[e] : (f16)0.f;
+      for (int e = 0; e < 4; ++e) qk[m][tt][e] = t < nval ? qk[m][tt][e] : 0u;
+      unpack16<TIn>(qk[m][tt], y[m]);
+      *reinterpret_cast<u32x4*>((m ? ks : qs) + w16::soff<32>(t, 8 * g)) = qk[m][tt];
     }
-    *reinterpret_cast<f16x8*>(qs + w16::soff<32>(t, 8 * g)) = x8[0];
-    *reinterpret_cast<f16x8*>(ks + w16::soff<32>(t, 8 * g)) = x8[1];
     float rq = 0.f, rk = 0.f, rw = 0.f;
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-      rq = __builtin_fmaf((float)x8[0][e], aQ[e >> 2][tt][e & 3], rq);
-      rk = __builtin_fmaf((float)x8[1][e], aK[e >> 2][tt][e & 3], rk);
-      rw = __builtin_fmaf((float)x8[1][e], -aW[e >> 2][tt][e & 3], rw);
+      rq = __builtin_fmaf(y[0][e], aQ[e >> 2][tt][e & 3], rq);
+      rk = __builtin_fmaf(y[1][e], aK[e >> 2][tt][e & 3], rk);
+      rw = __builtin_fmaf(y[1][e], -aW[e >> 2][tt][e & 3], rw);
     }
     rq = sum_groups(rq);
     rk = sum_groups(rk);
@@ -562,11 +570,12 @@ __device__ __forceinline__ void grad16_chunk(const BArgs& p, GradMem<K>& s, cons
     if (job % NW == wave) {
       const bool isq = job < 3;
       const int tt = tile_t(job), jt = tile_j(job), j = 16 * jt + n, tb = 16 * tt + 4 * g;
-      f32x4 kk = zero4;  // Q K^T or K K^T
+      f32x4 kk = zero4;  // Q K^T or K K^T, of the rows in their own type
 #pragma unroll
-      for (int kb = 0; kb < K; kb += 32)
-        kk = mma(w16::frag8_s<32>(&s.st[kb / 32][0][isq ? 0 : 1][0], 16 * tt + n, 8 * g),
-                 w16::frag8_s<32>(&s.st[kb / 32][0][1][0], j, 8 * g), kk);
+      for (int w = 0; w < NW; ++w)
+        kk = mma16<TIn>(
+            __builtin_bit_cast(u32x4, w16::frag8_s<32>(&s.st[w][0][isq ? 0 : 1][0], 16 * tt + n, 8 * g)),
+            __builtin_bit_cast(u32x4, w16::frag8_s<32>(&s.st[w][0][1][0], j, 8 * g)), kk);
       const f32x4 be4 = *reinterpret_cast<const f32x4*>(&s.gt[3][tb]);
       float x[4], col = 0.f;
 #pragma unroll
@@ -638,10 +647,19 @@ __device__ __forceinline__ void grad16_chunk(const BArgs& p, GradMem<K>& s, cons
   for (int kt = 0; kt < 2; ++kt) {
     const int at = 8 * g + (n >> 2), col = 8 * (n & 3) + 4 * kt;
     const int o0 = w16::soff<32>(at, col), o1 = w16::soff<32>(at + 4, col);
-    const f16x4 a0 = w16::read_tr4(ks + o0), a1 = w16::read_tr4(ks + o1);
-    const f16x4 b0 = w16::read_tr4(qs + o0), b1 = w16::read_tr4(qs + o1);
-    kT[kt] = f16x8{a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], a1[2], a1[3]};
-    qT[kt] = f16x8{b0[0], b0[1], b0[2], b0[3], b1[0], b1[1], b1[2], b1[3]};
+    auto frag = [&](const f16* x, int u) __attribute__((always_inline)) {
+      const f16x4 lo = w16::read_tr4(x + o0), hi = w16::read_tr4(x + o1);
+      f16x8 y = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+      if constexpr (SHIFT) {
+        float z[8];
+        unpack16<TIn>(__builtin_bit_cast(u32x4, y), z);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) y[e] = (f16)ldexpf(z[e], -u);
+      }
+      return y;
+    };
+    kT[kt] = frag(ks, uq[1]);
+    qT[kt] = frag(qs, uq[0]);
   }
 #pragma unroll
   for (int tt = 0; tt < 2; ++tt) {
@@ -661,8 +679,8 @@ __device__ __forceinline__ void grad16_chunk(const BArgs& p, GradMem<K>& s, cons
       e = mma(kT[kt], zcl, mma(kT[kt], zch, e));
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        dq[4 * kt + i] = ldexpf(a[i], eq) + scale * gam * aQ[kt][tt][i];
-        dk[4 * kt + i] = ldexpf(b[i], eq) + ldexpf(e[i], ek) + (D * aK[kt][tt][i] - bg * aW[kt][tt][i]);
+        dq[4 * kt + i] = ldexpf(a[i], eq + uq[1]) + scale * gam * aQ[kt][tt][i];
+        dk[4 * kt + i] = ldexpf(b[i], eq + uq[0]) + ldexpf(e[i], ek + uq[1]) + (D * aK[kt][tt][i] - bg * aW[kt][tt][i]);
       }
     }
     if (t < nval) {
