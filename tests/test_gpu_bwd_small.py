@@ -126,3 +126,22 @@ def test_small_q_k(pkg, cuda, which, p, K):
     err = _err(got[name], want[name])
     print(f"  {name} {err:.2e}", flush=True)
     assert err <= EPS[dtype] + 2.0 ** -10
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("K,V", [(128, 128), (64, 48), (32, 32)])
+def test_dbeta_precision(pkg, cuda, dtype, K, V):
+    """dbeta, an fp32 output, does not see the chunk states' fp16: 5e-6 (fp32 sums
+    of u and z, whose operands are fp16 pairs), with beta down to 2^-9, also
+    negative; where beta is zero the products with S take over (2^-10)."""
+    x = _inputs(200, 2, K, V, dtype, seed=K + V, gate=0.05)
+    x["beta"][:, ::3] *= 2.0 ** -7
+    x["beta"][:, 1::5] *= -1.0
+    x["beta"][:, 2::9] = 0.0
+    print(f"[small] dbeta {dtype} K={K} V={V}", flush=True)
+    got, want = _grads(pkg, cuda, x, dtype, scale=0.3)
+    zero = x["beta"] == 0
+    a, b = got["dbeta"], want["dbeta"]
+    err = [((a - b)[m].norm() / b[m].norm()).item() for m in (~zero, zero)]
+    print(f"  dbeta {err[0]:.2e} {err[1]:.2e}", flush=True)
+    assert err[0] <= 5e-6 and err[1] <= 2.0 ** -10

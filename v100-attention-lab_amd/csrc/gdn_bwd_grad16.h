@@ -11,7 +11,8 @@
 //   dQK = M o (scale dO u^T),  dKK = dA o beta_t M,
 //   dq  = dQK K + scale diag(gam) dO S^T,
 //   dk  = dQK^T Q + (dKK + dKK^T) K + diag(D) u dS'^T + diag(beta gam) dW~,
-//   dbeta_t = v_t.z_t + gam_t k_t.dW~_t + sum_j (dA M KK)_tj,
+//   dbeta_t = v_t.z_t + gam_t k_t.dW~_t + sum_j (dA M KK)_tj
+//           = z_t.u_t / beta_t,
 //   db through gam, gam_C, D, M and A; dg = reverse cumsum of db.
 #pragma once
 
@@ -125,7 +126,7 @@ struct alignas(16) GradMem {
   };
   float gt[4][C];           // b, gam, D, beta
   float row[3][NW][C];      // per wave: q.(dO S^T), k.(u dS'^T), k.dW~
-  float vz[C];              // v.z
+  float vz[C], zu[C];       // v.z, z.u
   float rs[6][16], cs[6][16];  // row and column sums of the C x C tiles
   float am[3][16];          // row sums of dA M KK
   float dgc[NW];
@@ -547,6 +548,7 @@ __device__ __forceinline__ void grad16_chunk(const BArgs& p, GradMem<K>& s, cons
       for (int i = 0; i < 4; ++i) {
         const int t = tb + i;
         const float e = aJ[job / NW][i], d = expf(bt4[i] - bj);
+        if ((job == 3 || job == 5) && t == j) s.zu[t] = e;
         const float x = job < 3 ? (j <= t ? scale * d * e : 0.f) : (j < t ? -e * d : 0.f);
         aJ[job / NW][i] = x;
         m = fmaxf(m, fabsf(job < 3 ? x : be4[i] * x));
@@ -624,7 +626,10 @@ __device__ __forceinline__ void grad16_chunk(const BArgs& p, GradMem<K>& s, cons
     const float csum = up ? s.cs[2][tl] + s.cs[5][tl] : (s.cs[0][tl] + s.cs[1][tl]) + (s.cs[3][tl] + s.cs[4][tl]);
     const float am = up ? s.am[1][tl] + s.am[2][tl] : s.am[0][tl];
     const float gam = s.gt[1][t], D = s.gt[2][t], be = s.gt[3][t];
-    const float dbeta = s.vz[t] + gam * rw + am;
+    // u = T diag(beta) Y with Y = V - diag(gam) K S makes z.u / beta the same as
+    // z.Y: no fp16 state in it, and the walks' u and z are fp32.  Where beta is
+    // too small for that, by the products with S.
+    const float dbeta = fabsf(be) > 0x1p-10f ? s.zu[t] / be : s.vz[t] + gam * rw + am;
     const float dD = rk * D;  // through D: u_t.(K dS')_t D_t
     float db = (rsum - csum) + (scale * rq + be * rw) * gam - dD;
     // ... and (last row) through gam_C and every D_j
