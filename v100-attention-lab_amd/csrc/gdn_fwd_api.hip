@@ -189,9 +189,22 @@ static int launch_impl(const GdnFwdParams& P, hipStream_t s, int64_t scratch_byt
   a.g_dtype = P.g_dtype; a.beta_dtype = P.beta_dtype; a.o_dtype = P.o_dtype;
   a.xcd_remap = (units % 8 == 0) ? 1 : 0;
   a.cu = P.cu_seqlens;
+  a.min_rows = 0;
+  a.max_rows = 0x7fffffff;
 
-  if (!(P.flags & GDN_FLAG_PHASED_KERNEL) && f32_batch_runs(P) && pipe_offsets_fit(P))
-    return launch_f32_batch(a, P.K, s);
+  if (!(P.flags & GDN_FLAG_PHASED_KERNEL) && f32_batch_supported(P) && pipe_offsets_fit(P)) {
+    // by a sequence's own length, whatever it is batched or packed with (packed
+    // runs give the bits of separate ones): a packed call of both kinds is two
+    // launches
+    const int rows = f32_batch_min_rows(P.V);
+    if (P.T >= rows) {
+      KArgs b = a;
+      b.min_rows = rows;
+      const int st = launch_f32_batch(b, P.K, s);
+      if (st != 0 || P.cu_seqlens == nullptr || rows == 0) return st;
+      a.max_rows = rows - 1;
+    }
+  }
   const int grid = (int)units;
   if (!(P.flags & GDN_FLAG_PHASED_KERNEL) && pipe_supported(P.qkv_dtype, P.K, P.chunk_size, bv) &&
       pipe_offsets_fit(P)) {

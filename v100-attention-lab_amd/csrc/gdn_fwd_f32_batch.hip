@@ -21,8 +21,8 @@
 //
 // Bound by the scan's chain (matrix instructions of 32 cycles: 64 of them and
 // one exchange a chunk at K = 128, 36 at K = 64) and, per batch, the
-// substitution.  1 x 256 rows, 2 heads, K = V = 64: 83 -> 28.7 us; 2 x 1024
-// rows, 16 heads, K = V = 128: 531 -> 164 us.
+// substitution.  1 x 256 rows, 2 heads, K = V = 64: 82.4 -> 27.7 us; 2 x 1024
+// rows, 16 heads, K = V = 128: 531 -> 162 us.
 
 #include "gdn_fwd_pipe.h"
 
@@ -165,7 +165,25 @@ __device__ __forceinline__ void produce(const KArgs& p, Slot& s, const float* kg
   }
 }
 
-template <int K, int NG>
+// The j-th sequence (in order) of at least min_rows rows, -1 if there are
+// fewer; by every wave for itself, all 64 lanes active.
+__device__ __forceinline__ int nth_long(const int64_t* cu, int T, int N, int j, int min_rows) {
+  const int lane = threadIdx.x & 63;
+  for (int i = 0; i < N; i += 64) {
+    uint64_t m = __ballot(i + lane < N && row_span(cu, T, min(i + lane, N - 1)).T >= min_rows);
+    const int n = __builtin_popcountll(m);
+    if (j < n) {
+      for (; j > 0; --j) m &= m - 1;
+      return i + __builtin_ctzll(m);
+    }
+    j -= n;
+  }
+  return -1;
+}
+
+// MANY: more than kMaxRanked packed sequences (an instance of its own: the search
+// costs the others registers, and K = 64 then spills)
+template <int K, int NG, bool MANY>
 __global__ __launch_bounds__(64 * NW) void f32_batch_kernel(const KArgs p) {
   constexpr int KT = K / 16, KO = KT / NS;  // key tiles, of them a wave's own
   __shared__ Smem<NG> s;
@@ -173,7 +191,17 @@ __global__ __launch_bounds__(64 * NW) void f32_batch_kernel(const KArgs p) {
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wave = wid % NS, grp = wid / NS;  // of the scan
   const int r = lane & 15, g = lane >> 4;
-  const ScanUnit su = scan_unit<1>(p.cu, p.T, p.B, p.H, p.nv, blockIdx.x);
+  ScanUnit su;
+  if constexpr (!MANY) {
+    // (before the ranking: a batch of short sequences ends here)
+    if (p.cu != nullptr && nth_long(p.cu, p.T, p.B, blockIdx.x / (p.H * p.nv), p.min_rows) < 0) return;
+    su = scan_unit<1>(p.cu, p.T, p.B, p.H, p.nv, blockIdx.x);
+  } else {
+    const int per = p.H * p.nv;
+    su = scan_unit<1>(nullptr, p.T, 1, p.H, p.nv, blockIdx.x % per);
+    su.bi = nth_long(p.cu, p.T, p.B, blockIdx.x / per, p.min_rows);
+    if (su.bi < 0) return;
+  }
   const int bi = su.bi, hi = su.hi, v0 = 16 * (NG * su.vs + (grp < NG ? grp : 0));
   const RowSpan rs = row_span(p.cu, p.T, bi);
   const int T = rs.T, nch = (T + C - 1) / C;
@@ -345,37 +373,49 @@ __global__ __launch_bounds__(64 * NW) void f32_batch_kernel(const KArgs p) {
 
 }  // namespace f32b
 
-// Where this kernel runs.  A workgroup takes a whole CU's LDS, so a dense batch
-// of several short sequences with more than a workgroup per CU keeps the
-// phase-by-phase kernel, several of whose workgroups share a CU: 8 x 64 rows,
-// 32 heads, K = V = 128 81 us against 96 here, 8 x 16 rows 44 against 62;
-// from 128 rows on this one is ahead (150 against 134, at 512 rows 588 against
-// 440), and below a workgroup per CU always (2 x 16 rows, 16 heads 21.7
-// against 16.9; 2 x 1024 rows 531 against 164).  One sequence and packed ones
-// always run here: packed runs give the bits of separate ones.
-bool f32_batch_runs(const GdnFwdParams& P) {
-  if (P.qkv_dtype != GDN_DTYPE_F32 || P.chunk_size != f32b::C || (P.K != 64 && P.K != 128)) return false;
-  const int64_t bh = (int64_t)P.B * P.H;
-  if (bh * (P.V / 16) > 0x7fffffffLL) return false;
-  return P.cu_seqlens != nullptr || P.B == 1 || P.T >= 128 || bh * (P.V / 32) <= 256;
+bool f32_batch_supported(const GdnFwdParams& P) {
+  return P.qkv_dtype == GDN_DTYPE_F32 && P.chunk_size == f32b::C && (P.K == 64 || P.K == 128) &&
+         (int64_t)P.B * P.H * (P.V / 16) <= 0x7fffffffLL;
 }
+
+// Sequences of fewer rows take the phase-by-phase kernel.  A workgroup here
+// takes a whole CU's LDS, and forms a chunk's half once per 16 or 32 columns:
+// where there are more than one to a CU, short sequences are faster on that
+// kernel's small ones of up to 64 columns (us, phased against here: K = V = 128,
+// 256 heads, 32 rows 45 against 71, 64 rows 80 against 100, 96 rows 114 against
+// 124, 128 rows 149 against 144; K = V = 64, 1024 heads, 96 rows 139 against
+// 152, 128 rows 179 against 176).  With few heads short ones would be faster
+// here (8 heads, 64 rows 38 against 20); but the line is drawn by a sequence's
+// own length, so that its bits do not depend on what it is batched or packed
+// with.  V an odd multiple of 16 above 16 leaves the phased kernel 16 columns,
+// and this one is ahead at every length (K = 128, V = 48, 256 heads, 1 row 57
+// against 44, 64 rows 109 against 63).
+int f32_batch_min_rows(int V) { return V > 16 && V % 32 != 0 ? 0 : 97; }
 
 // The launch (a.nv is set here): 16 columns a workgroup up to one per CU, 32
 // beyond (a batch's chunks are then formed once for both halves: 4 x 1024
 // rows, 16 heads, K = V = 128 217 us against 330).  A column's arithmetic is
-// the same in both.
+// the same in both.  With cu: workgroups for as many sequences as can have
+// min_rows rows (the longest ones first, or in order beyond kMaxRanked); the
+// others of these end at once (64 packed sequences of 64 rows, 16 heads, K = V =
+// 128: 337 us with this launch, 329 without).
 int launch_f32_batch(KArgs a, int K, hipStream_t s) {
-  const int64_t bh = (int64_t)a.B * a.H;
+  int64_t n = a.B;
+  if (a.cu != nullptr && a.min_rows > 0 && a.T / a.min_rows < n) n = a.T / a.min_rows;
+  const int64_t bh = n * a.H;
   const bool two = a.V % 32 == 0 && bh * (a.V / 16) > 256;
   a.nv = a.V / (two ? 32 : 16);
   const dim3 grid((unsigned)(bh * a.nv)), block(64 * f32b::NW);
-  if (K == 64) {
-    if (two) hipLaunchKernelGGL((f32b::f32_batch_kernel<64, 2>), grid, block, 0, s, a);
-    else hipLaunchKernelGGL((f32b::f32_batch_kernel<64, 1>), grid, block, 0, s, a);
-  } else {
-    if (two) hipLaunchKernelGGL((f32b::f32_batch_kernel<128, 2>), grid, block, 0, s, a);
-    else hipLaunchKernelGGL((f32b::f32_batch_kernel<128, 1>), grid, block, 0, s, a);
-  }
+  auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, block, 0, s, a); };
+  auto pick = [&](auto many) {
+    constexpr bool M = decltype(many)::value;
+    if (K == 64 && two) go(f32b::f32_batch_kernel<64, 2, M>);
+    else if (K == 64) go(f32b::f32_batch_kernel<64, 1, M>);
+    else if (two) go(f32b::f32_batch_kernel<128, 2, M>);
+    else go(f32b::f32_batch_kernel<128, 1, M>);
+  };
+  if (a.cu != nullptr && a.B > kMaxRanked) pick(std::true_type{});
+  else pick(std::false_type{});
   return (int)hipGetLastError();
 }
 

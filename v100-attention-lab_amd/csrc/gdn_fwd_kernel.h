@@ -422,6 +422,7 @@ struct KArgs {
   int g_dtype, beta_dtype, o_dtype;
   int xcd_remap;
   const int64_t* cu;  // nullable: B + 1 row offsets of packed sequences
+  int min_rows, max_rows;  // with cu: sequences of other lengths are another launch's
 };
 
 // Rows of work unit bi.  Without cu: rows [0, T) of batch bi.  With cu
@@ -561,6 +562,7 @@ __global__ __launch_bounds__(kThreads) void gdn_fwd_kernel(const KArgs p) {
   const int hi = bh % p.H;
   const int v0 = vs * BV;
   const RowSpan rs = row_span(p, bi);
+  if (p.cu != nullptr && rs.T > p.max_rows) return;
   const int T = rs.T;
 
   const TIn* qg = static_cast<const TIn*>(p.q) + head_base(rs, hi, p.sq);
@@ -979,9 +981,11 @@ inline bool pipe_supported(int dtype, int K, int C, int BV) {
 }
 int launch_pipe_f16(const KArgs& a, int K, int bv, int grid, hipStream_t s);
 int launch_pipe_bf16(const KArgs& a, int K, int bv, int grid, hipStream_t s);
-// fp32 inputs with 32-row chunks and K in {64, 128} run in one launch of
-// batched chunks (gdn_fwd_f32_batch.hip).
-bool f32_batch_runs(const GdnFwdParams& P);
+// fp32 inputs with 32-row chunks and K in {64, 128}: sequences of at least
+// f32_batch_min_rows rows run in one launch of batched chunks
+// (gdn_fwd_f32_batch.hip), shorter ones on the phased kernel.
+bool f32_batch_supported(const GdnFwdParams& P);
+int f32_batch_min_rows(int V);
 int launch_f32_batch(KArgs a, int K, hipStream_t s);
 // 64-row chunks with K in {32, 64, 128} run as two launches (gdn_fwd_c64.hip)
 // over a caller-owned workspace of per-chunk records.
