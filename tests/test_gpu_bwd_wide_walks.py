@@ -17,12 +17,23 @@ EPS = {torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}
 NAMES = ("dq", "dk", "dv", "dg", "dbeta", "dh0")
 
 
-# 2 B H V / 16 workgroups of 16 columns: over 512 at K = 128, over 768 below
+# workgroups of 16 and of 32 columns that run at once on 256 CUs
+ROUND = {128: (512, 512), 64: (768, 512), 32: (1024, 768)}
+
+
+def _wide(B, H, K, V):
+    """The launcher's rule: 32 columns where they take fewer rounds."""
+    units, (n16, n32) = B * H * (V // 16), ROUND[K]
+    return V % 32 == 0 and -(-units // n32) < -(-2 * units // n16)
+
+
+# 2 B H V / 16 workgroups of 16 columns: over 512 at K = 128, 768 at 64, 1024 at 32
 @pytest.mark.parametrize("B,T,H,K,V", [(3, 1, 45, 128, 32), (3, 33, 16, 128, 96), (3, 95, 12, 128, 128),
-                                       (3, 64, 17, 64, 128), (3, 70, 67, 32, 32)])
+                                       (3, 64, 17, 64, 128), (3, 70, 90, 32, 32)])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("spread", [0, 14])
 def test_wide_walks(pkg, cuda, dtype, B, T, H, K, V, spread):
+    assert _wide(B, H, K, V) and not _wide(1, H, K, V)
     gen = torch.Generator().manual_seed(T + K + V)
     n = lambda *s: torch.randn(*s, generator=gen)
     q, k = ref.l2norm(n(B, T, H, K)), ref.l2norm(n(B, T, H, K))
