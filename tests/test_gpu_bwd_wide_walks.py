@@ -58,3 +58,23 @@ def test_wide_walks(pkg, cuda, dtype, B, T, H, K, V, spread):
         a = got[i][:1, :2] if name == "dh0" else got[i][:1, :, :2]
         err = ref.rel_err(want, a.cpu().double())
         assert err <= 1e-3 + EPS[dtype], (name, err)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("B,T,H,K,V", [(3, 70, 12, 128, 128), (3, 40, 17, 64, 128)])
+def test_wide_walks_do_row_offset(pkg, cuda, dtype, B, T, H, K, V):
+    """dO rows that start 4-byte aligned only: the bits of a dense dO."""
+    assert _wide(B, H, K, V)
+    gen = torch.Generator().manual_seed(K)
+    n = lambda *s: torch.randn(*s, generator=gen)
+    q, k = ref.l2norm(n(B, T, H, K)).to(dtype), ref.l2norm(n(B, T, H, K)).to(dtype)
+    v, g, beta = n(B, T, H, V).to(dtype), 0.3 * torch.nn.functional.logsigmoid(n(B, T, H)), torch.sigmoid(n(B, T, H))
+    d = [x.to(cuda) for x in (q, k, v, g, beta, 0.1 * n(B, H, K, V))]
+    buf = 1e-3 * n(B, T, H, V + 8).to(dtype).to(cuda)
+    do, dfs = buf[..., 2:2 + V], 1e-3 * n(B, H, K, V).to(cuda)
+    assert do.data_ptr() % 16 == 4
+    print(f"[wide] {dtype} K={K} V={V} dO rows at 4 bytes", flush=True)
+    got = pkg.gdn_bwd(*d, do, dfs, scale=0.5)
+    want = pkg.gdn_bwd(*d, do.contiguous(), dfs, scale=0.5)
+    for name, a, b in zip(NAMES, got, want):
+        assert torch.equal(a, b), name

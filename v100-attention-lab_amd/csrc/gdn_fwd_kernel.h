@@ -199,23 +199,32 @@ __device__ __forceinline__ uint32_t block_max_bits(uint32_t m, uint32_t* red) {
   return m;
 }
 
-// Bits of the largest magnitude of a 16-byte piece of 8 bf16 columns at v
-// over rows r, r + rstep, ... (`rstride` bytes apart), eight loads in flight.
+// 16 bytes of global memory at a multiple of 4 (all that a four-word load asks
+// for): the backward's dO rows start at any pair of elements.
+__device__ __forceinline__ uint4 load_words4(const char* p) {
+  typedef uint32_t words __attribute__((ext_vector_type(4), aligned(4)));
+  const words w = *reinterpret_cast<const words*>(p);
+  return uint4{w[0], w[1], w[2], w[3]};
+}
+
+// Bits of the largest magnitude of a piece of 8 bf16 columns at v (a multiple
+// of 4 bytes) over rows r, r + rstep, ... (`rstride` bytes apart), eight loads
+// in flight.
 __device__ __forceinline__ uint32_t column_absmax_bits(const char* v, int64_t rstride, int rows, int r, int rstep) {
   uint32_t m = 0;
   for (; r + 7 * rstep < rows; r += 8 * rstep) {
     uint4 x[8];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) x[u] = *reinterpret_cast<const uint4*>(v + (int64_t)(r + u * rstep) * rstride);
+    for (int u = 0; u < 8; ++u) x[u] = load_words4(v + (int64_t)(r + u * rstep) * rstride);
 #pragma unroll
     for (int u = 0; u < 8; ++u) m = max(m, bf16x8_absmax_bits(x[u]));
   }
-  for (; r < rows; r += rstep) m = max(m, bf16x8_absmax_bits(*reinterpret_cast<const uint4*>(v + (int64_t)r * rstride)));
+  for (; r < rows; r += rstep) m = max(m, bf16x8_absmax_bits(load_words4(v + (int64_t)r * rstride)));
   return m;
 }
 
 // Largest magnitude of v[rows x cols] (bf16, rows `rstride` bytes apart,
-// cols a multiple of 8, 16-byte aligned rows) and of h0[K x cols] (fp32,
+// cols a multiple of 8, rows at multiples of 4 bytes) and of h0[K x cols] (fp32,
 // element strides sk and sc; nullable), over the whole workgroup: every
 // thread of the workgroup calls it (one barrier).  NaN if either holds one.
 __device__ __forceinline__ float slice_absmax_bf16(const char* v, int64_t rstride, int rows, int cols,
@@ -232,7 +241,7 @@ __device__ __forceinline__ float slice_absmax_bf16(const char* v, int64_t rstrid
     for (int64_t i = tid; i < nv; i += nthr) {
       const int64_t r = i / pieces;
       const int c = (int)(i - r * pieces);
-      m = max(m, bf16x8_absmax_bits(*reinterpret_cast<const uint4*>(v + r * rstride + c * 16)));
+      m = max(m, bf16x8_absmax_bits(load_words4(v + r * rstride + c * 16)));
     }
   }
   return __uint_as_float(block_max_bits(max(m, state_absmax_bits(h0, sk, sc, K, cols)), red));
