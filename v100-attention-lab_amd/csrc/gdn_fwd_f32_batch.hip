@@ -194,7 +194,10 @@ __global__ __launch_bounds__(64 * NW) void f32_batch_kernel(const KArgs p) {
   ScanUnit su;
   if constexpr (!MANY) {
     // (before the ranking: a batch of short sequences ends here)
-    if (p.cu != nullptr && nth_long(p.cu, p.T, p.B, blockIdx.x / (p.H * p.nv), p.min_rows) < 0) return;
+    if (p.cu != nullptr &&
+        __popcll(__ballot(lane < p.B && row_span(p.cu, p.T, lane).T >= p.min_rows)) <=
+            (int)(blockIdx.x / (p.H * p.nv)))
+      return;
     su = scan_unit<1>(p.cu, p.T, p.B, p.H, p.nv, blockIdx.x);
   } else {
     const int per = p.H * p.nv;

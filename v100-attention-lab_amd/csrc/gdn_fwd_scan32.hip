@@ -225,10 +225,6 @@ __device__ __forceinline__ unsigned long long ps_now() {
 #endif
 
 // ---------------------------------------------------------------------------
-// 1. records
-// ---------------------------------------------------------------------------
-
-// ---------------------------------------------------------------------------
 // short sequences: the step recurrence itself
 // ---------------------------------------------------------------------------
 
@@ -382,6 +378,10 @@ __device__ __forceinline__ void short_job(const SArgs& p, int blk) {
   if (rs.T > 0 && rs.T <= kShortRows) short_walk<TIn, K, NT>(p, rs, bh / p.H, bh % p.H, 16 * vs);
 }
 inline int short_blocks(const SArgs& a) { return (int)(((int64_t)a.B * a.H * (a.V / 16) + 3) / 4); }
+
+// ---------------------------------------------------------------------------
+// 1. records
+// ---------------------------------------------------------------------------
 
 // Record job r of a segment -> (sequence bi, head hi, its rows, chunk c0 + lc);
 // the record is number (bi H + hi) L + lc.  A dense batch has one job per
