@@ -145,3 +145,20 @@ def test_dbeta_precision(pkg, cuda, dtype, K, V):
     err = [((a - b)[m].norm() / b[m].norm()).item() for m in (~zero, zero)]
     print(f"  dbeta {err[0]:.2e} {err[1]:.2e}", flush=True)
     assert err[0] <= 5e-6 and err[1] <= 2.0 ** -10
+
+
+@pytest.mark.parametrize("T,K,V", [(32, 64, 48), (97, 64, 96), (97, 128, 80)])
+def test_small_v_and_gradients_f16(pkg, cuda, T, K, V):
+    """fp16 v near 2^-10 and gradients near 2^-16: u and z are far below 1, the
+    unit of fp16 inputs; dg and dbeta, fp32 outputs, keep 2^-9 (the carried
+    state gradient, an fp16 pair to 2^-25, gives half of that)."""
+    dtype = torch.float16
+    x = _inputs(T, 4, K, V, dtype, seed=T + V, gate=0.3)
+    for n, p in (("v", 10), ("do", 16), ("dfs", 16)):
+        x[n] *= 2.0 ** -p
+    print(f"[small] fp16 v and gradients T={T} K={K} V={V}", flush=True)
+    got, want = _grads(pkg, cuda, x, dtype, scale=0.3)
+    for n in ("dg", "dbeta"):
+        err = _err(got[n], want[n])
+        print(f"  {n} {err:.2e}", flush=True)
+        assert err <= 2.0 ** -9, n
