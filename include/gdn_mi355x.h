@@ -143,7 +143,8 @@ typedef struct GdnFwdParams {
  *     workspace (gdn_fwd_workspace_size is 0, params->workspace is not read).
  *   - C = 32 without a workspace (or GDN_FLAG_FUSED_KERNEL), fp32 inputs at
  *     C = 32, or K = 256 / GDN_FLAG_PHASED_KERNEL: one fused kernel, no
- *     workspace.
+ *     workspace (two for packed fp32 sequences at K in {64, 128}, by their
+ *     length).
  * The state stays on chip in every path: no chunk state is written. */
 int gdn_fwd_launch(const GdnFwdParams* params, void* stream);
 
@@ -317,7 +318,7 @@ int64_t gdn_bwd_workspace_size(int B, int T, int H, int K, int V, int n_seq);
  * sizes, dtypes, d_o alignment and cu_seqlens; pointers other than d_o and
  * cu_seqlens are not read); -1 if unsupported.  With 16-bit q, k, v and dO
  * of the same type, 4-byte aligned, the walks keep the chunk states in
- * fp16 and their records hold T and the gates only: about 55 % of
+ * fp16 and their records hold the gates, T and P only: about 55 % of
  * gdn_bwd_workspace_size at K = V = 128.  Without cu_seqlens, at most 256
  * chunks per sequence at a time. */
 int64_t gdn_bwd_workspace_size_params(const GdnBwdParams* params);

@@ -303,7 +303,11 @@ def gdn_fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Tensor,
       kernel: ``"auto"`` picks per shape: for fp16 or bf16 with chunk 32
         and K in {64, 128}, per-chunk records then the scan (two launches
         per segment, a workspace of records; bf16 records also carry the
-        chunk's k rows in fp16); the phase-by-phase kernel elsewhere.  ``"fused"``
+        chunk's k rows in fp16), where sequences of at most 4 rows are
+        walked step by step in fp32; for chunk 64 and K <= 128 two launches
+        likewise; for fp32 with chunk 32 and K in {64, 128}, sequences of
+        97 rows or more (any length where V is an odd multiple of 16 above
+        16) in batches of chunks; the phase-by-phase kernel elsewhere.  ``"fused"``
         forces the fused pipelined kernel (no workspace) where it applies,
         ``"phased"`` the phase-by-phase kernel.
       cu_seqlens: optional int64 ``[N + 1]`` row offsets: N sequences
@@ -559,7 +563,7 @@ def gdn_bwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Tensor,
     same strides, dtypes and ``cu_seqlens`` convention as the forward.  One
     call enqueues the backward's three kernels on the current stream; the
     workspace (per-chunk records, chunk-start states and their gradients,
-    u and du) is allocated here and released when the call returns.  It
+    u and, for 16-bit inputs, T^T du, else du) is allocated here and released when the call returns.  It
     holds at most ``max_segment_chunks`` chunks of 32 rows per sequence
     (default 256): a longer batch runs in segments, with one forward pass
     over all but the last segment for the states at their starts
