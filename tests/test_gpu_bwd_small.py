@@ -162,3 +162,19 @@ def test_small_v_and_gradients_f16(pkg, cuda, T, K, V):
         err = _err(got[n], want[n])
         print(f"  {n} {err:.2e}", flush=True)
         assert err <= 2.0 ** -9, n
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+def test_dbeta_before_a_bad_row(pkg, cuda, dtype, bad):
+    """v not finite in one row: dbeta of the chunk's first row, which does not
+    see it, is that of finite values."""
+    x = _inputs(8, 2, 64, 32, dtype, seed=8)
+    want, _ = _grads(pkg, cuda, x, dtype, scale=0.3)
+    x["v"][:, 5, :, 3] = bad
+    print(f"[small] {dtype} v {bad} in row 5", flush=True)
+    d = {n: t.to(dtype).to(cuda) if n in ("q", "k", "v", "do") else t.to(cuda) for n, t in x.items()}
+    got = pkg.gdn_bwd(d["q"], d["k"], d["v"], d["g"], d["beta"], d["h0"], d["do"], d["dfs"], scale=0.3)[4].cpu()
+    assert torch.isfinite(got[:, 0]).all()
+    # by the products with the fp16 chunk state: 2^-10
+    assert ((got[:, 0] - want["dbeta"][:, 0]).norm() / want["dbeta"][:, 0].norm()).item() <= 2.0 ** -10

@@ -630,8 +630,10 @@ __device__ __forceinline__ void grad16_chunk(const BArgs& p, GradMem<K>& s, cons
     const float gam = s.gt[1][t], D = s.gt[2][t], be = s.gt[3][t];
     // u = T diag(beta) Y with Y = V - diag(gam) K S makes z.u / beta the same as
     // z.Y: no fp16 state in it, and the walks' u and z are fp32.  Where beta is
-    // too small for that, by the products with S.
-    const float dbeta = fabsf(be) > 0x1p-10f ? s.zu[t] / be : s.vz[t] + gam * rw + am;
+    // too small for that, or a row of u is not finite (a zero of T times an inf
+    // or NaN of a later row), by the products with S.
+    const float zu = s.zu[t] / be;
+    const float dbeta = fabsf(be) > 0x1p-10f && fabsf(zu) < __builtin_inff() ? zu : s.vz[t] + gam * rw + am;
     const float dD = rk * D;  // through D: u_t.(K dS')_t D_t
     float db = (rsum - csum) + (scale * rq + be * rw) * gam - dD;
     // ... and (last row) through gam_C and every D_j
